@@ -1080,8 +1080,10 @@ static int contract_impl(const char *cptrn, talsh_tens_t *dtens, talsh_tens_t *l
       }
     }
     int e = plan_contraction(dig, dr, lr, rr, dd, ld, rd, es, acc, plan_variant, P, nullptr);
-    // the three-way BF16 split reads matricized operands: no fused gather
-    if (!e && P.fused && (kind == R4 || kind == C4) && d->r4mode == R4Mode::kBF16x3)
+    // the three-way BF16 split reads matricized operands, and a gather takes
+    // its index digits in 32 bits: no fused gather then
+    const bool wide = P.m > INT32_MAX || P.n > INT32_MAX || P.k > INT32_MAX;
+    if (!e && P.fused && (wide || ((kind == R4 || kind == C4) && d->r4mode == R4Mode::kBF16x3)))
       e = plan_contraction(dig, dr, lr, rr, dd, ld, rd, es, acc, -1, P, nullptr);
     if (e) return e;
   }
@@ -1141,17 +1143,27 @@ static int contract_impl(const char *cptrn, talsh_tens_t *dtens, talsh_tens_t *l
       }
       int e = 0;
       if (P.fused) {
-        wsb = gemm_gather_workspace_bytes(gemm_args(t.d->r4mode));
-        return wsb ? t.alloc(wsb, &ws) : 0;
+        const GemmArgs g = gemm_args(t.d->r4mode);
+        return workspace(t, gemm_gather_workspace_bytes(g), gemm_split_bytes(g));
       }
       if (!P.l_o2n.empty()) e = t.alloc(tensor_volume(L->t) * es, &lt);
       if (!e && !P.r_o2n.empty()) e = t.alloc(tensor_volume(R->t) * es, &rt);
       if (!e && !P.d_in_o2n.empty()) e = t.alloc(tensor_volume(D->t) * es, &dt);
       if (!e) {
-        wsb = gemm_workspace_bytes(gemm_args(t.d->r4mode));
-        if (wsb) e = t.alloc(wsb, &ws);
+        const GemmArgs g = gemm_args(t.d->r4mode);
+        e = workspace(t, gemm_workspace_bytes(g), gemm_split_bytes(g));
       }
       return e;
+    }
+    // The product's workspace: `need` bytes or the call is deferred (callers
+    // rely on a full arena giving TRY_LATER), `want` bytes if there is room,
+    // so that K can be split further.
+    int workspace(Temps &t, size_t need, size_t want)
+    {
+      wsb = want;
+      if (want > need && t.alloc(want, &ws) == 0) return 0;
+      wsb = need;
+      return need ? t.alloc(need, &ws) : 0;
     }
     int enqueue(Task *k, Device *dev)
     {
@@ -1863,7 +1875,7 @@ int talshAmdGemm(int data_kind, int fast_math, size_t m, size_t n, size_t k, con
   hipStream_t s = d->streams[0];
   hipEvent_t pr[2];
   prof_begin(s, kKGemm, pr);
-  const int e = need <= workspace_bytes ? launch_gemm_ws(g, workspace, workspace_bytes, s)
+  const int e = need <= workspace_bytes ? launch_gemm_ws(g, workspace, need, s)
                                         : launch_gemm_ws(g, nullptr, 0, s);
   prof_end(s, kKGemm, pr);
   if (e) return e;
@@ -1890,7 +1902,7 @@ int talshAmdGemmNoAlloc(int data_kind, int fast_math, size_t m, size_t n, size_t
   }
   (void)hipSetDevice(d->ordinal);
   hipStream_t s = d->streams[0];
-  const int e = launch_gemm_ws(g, d->noalloc_scratch, kGemmNoAllocScratchBytes, s);
+  const int e = launch_gemm_ws(g, d->noalloc_scratch, need, s);
   if (e) return e;
   return XT_HIP_OK(hipStreamSynchronize(s)) ? 0 : TALSH_FAILURE;
 }

@@ -16,514 +16,10 @@
 #include <algorithm>
 #include <type_traits>
 
-#include "bf16x3.hpp"
-#include "kernels.hpp"
+#include "gemm_native.hpp"
 
 namespace xt {
 namespace {
-
-typedef double d4 __attribute__((ext_vector_type(4)));
-typedef float f4 __attribute__((ext_vector_type(4)));
-
-template <typename T>
-struct Acc;
-template <>
-struct Acc<double> { typedef d4 type; };
-template <>
-struct Acc<float> { typedef f4 type; };
-
-__device__ __forceinline__ d4 mfma(double a, double b, d4 c)
-{
-  return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-}
-__device__ __forceinline__ f4 mfma(float a, float b, f4 c)
-{
-  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-}
-
-struct GemmParams {
-  const void *a;
-  const void *b;
-  void *c;
-  int64_t m, n, k;
-  int64_t lda, ldb, ldc;     // leading dims in elements (complex: in complex elements)
-  double alpha_re, alpha_im;
-  int beta_zero;
-  int conj_a, conj_b;
-  int tiles_m, tiles_n;
-  int xcd_remap;             // 1: blockIdx -> tile remap that keeps neighbours on one XCD
-  int vec_a, vec_b;          // 16-byte aligned rows of k-fast operands (vector loads allowed)
-  // split K (real kinds): workgroup row blockIdx.y takes k in [y * kchunk,
-  // (y + 1) * kchunk) and writes its raw m x n partial to part + y * m * n;
-  // part == nullptr: one pass over all of K, epilogue into C
-  void *part;
-  int64_t kchunk;
-  // fused index gather (GATHER kernels): A element (r, kk) at a_row[r] +
-  // a_kof[kk], B element (c, kk) at b_row[c] + b_kof[kk], C element (r, c) at
-  // c_row[r] + c_col[c] (element offsets into the tensor bodies); vec_a /
-  // vec_b: aligned groups of 16 bytes along the staging direction are
-  // contiguous
-  const int64_t *a_row, *a_kof, *b_row, *b_kof, *c_row, *c_col;
-  int64_t a_ks0, b_ks0;      // stride of the first contracted dimension in A / B (gather)
-  int64_t a_rs0, b_rs0;      // stride of the first row dimension of A / B (gather)
-  const void *zpad;          // 64 zero bytes, 16-byte aligned (gather)
-  int part_rowmajor;         // split-K partials m x n row-major (else column-major)
-};
-
-// Maps a workgroup to an output tile: first gather the workgroups that the
-// dispatcher places on one XCD (round-robin over 8) into a contiguous range,
-// then walk that range in column groups of G M-tiles so neighbouring
-// workgroups share B panels (and A panels within a group) in their XCD's L2.
-template <int G = 8>
-__device__ __forceinline__ void tile_of(const GemmParams &p, int &tm, int &tn)
-{
-  const int nb = gridDim.x;
-  int t = blockIdx.x;
-  if (p.xcd_remap && (nb % 8) == 0) t = (t % 8) * (nb / 8) + t / 8;
-  const int per_group = G * p.tiles_n;
-  const int group = t / per_group;
-  const int first_m = group * G;
-  const int gm = min(p.tiles_m - first_m, G);
-  const int r = t - group * per_group;
-  tm = first_m + r % gm;
-  tn = r / gm;
-}
-
-// ---------------------------------------------------------------------------
-// FP64 / FP32 16x16x4 family. Workgroup: 256 threads = 2x2 waves; each wave
-// owns a (BM/2) x (BN/2) sub-tile of 16x16 MFMA blocks.
-//
-// Operand tiles sit in LDS with k fastest ([row][k], padded rows). Inside a
-// 16-deep k slice, lane group g = lane/16 feeds k = 4g+s at MFMA step s, so a
-// lane's four steps use four consecutive k and its fragment for the whole
-// slice is one contiguous LDS read (summation order over k is immaterial).
-template <typename T>
-struct Frag4;
-template <>
-struct Frag4<float> { typedef float4 type; };
-template <>
-struct Frag4<double> { typedef double4 type; };
-
-// GATHER: 0 matricized operands; 1 fused gather where every thread's staged
-// elements stay inside one run of the staging direction's first dimension
-// (offsets by stride arithmetic from one table entry) and real operands load
-// in vectors; 2 fused gather with a table lookup per staged element or
-// vector.
-template <typename T, bool CPLX, bool AK, bool BKF, int BM, int BN, int BK, int OCC, int GATHER = 0>
-__global__ __launch_bounds__(256, OCC) void k_gemm_mfma(const GemmParams p)
-{
-  constexpr int NP = CPLX ? 2 : 1;                 // LDS planes (re, im)
-  constexpr int KP = BK + (sizeof(T) == 4 ? 4 : 2); // padded k extent of an LDS row
-  constexpr int FM = BM / 32, FN = BN / 32;        // MFMA blocks per wave along m / n
-  constexpr int LA = BM * BK / 256;                // A elements staged per thread
-  constexpr int LB = BN * BK / 256;
-  typedef typename Acc<T>::type AccT;
-  typedef typename Frag4<T>::type F4;
-  __shared__ __align__(16) T As[2][NP][BM][KP];
-  __shared__ __align__(16) T Bs[2][NP][BN][KP];
-
-  int tm, tn;
-  tile_of(p, tm, tn);
-  const int64_t m0 = (int64_t)tm * BM, n0 = (int64_t)tn * BN;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wm = (wave & 1) * (BM / 2), wn = (wave >> 1) * (BN / 2);
-  const T *A = static_cast<const T *>(p.a);
-  const T *B = static_cast<const T *>(p.b);
-  const bool interior_mn = (m0 + BM <= p.m) && (n0 + BN <= p.n);
-  const bool split = !CPLX && p.part != nullptr;
-  const int64_t kbeg = split ? (int64_t)blockIdx.y * p.kchunk : 0;
-  const int64_t kend = split ? min(p.k, kbeg + p.kchunk) : p.k;
-
-  // staging coordinates. k-fast operands: a thread covers LA consecutive k of
-  // one row. Row-fast operands: RV consecutive rows (one vector of two real
-  // elements; one complex element) at each of KV = L / RV consecutive k, so a
-  // wave's loads of one k are contiguous along rows and each row's KV values
-  // go to LDS in one store. Registers: element (row + e, k + j) of a row-fast
-  // operand is r[.][j * RV + e].
-  constexpr int RV = CPLX ? 1 : 2;
-  constexpr int KVA = LA / RV, KVB = LB / RV;
-  int a_r, a_k, b_r, b_k;
-  if (AK) { a_r = tid / (BK / LA); a_k = (tid % (BK / LA)) * LA; }
-  else { a_r = (tid % (BM / RV)) * RV; a_k = (tid / (BM / RV)) * KVA; }
-  if (BKF) { b_r = tid / (BK / LB); b_k = (tid % (BK / LB)) * LB; }
-  else { b_r = (tid % (BN / RV)) * RV; b_k = (tid / (BN / RV)) * KVB; }
-
-  // fused gather: offset of the thread's first staged row (loop invariant)
-  int64_t ga_row = 0, gb_row = 0;
-  if (GATHER) {
-    ga_row = p.a_row[m0 + a_r < p.m ? m0 + a_r : 0];
-    gb_row = p.b_row[n0 + b_r < p.n ? n0 + b_r : 0];
-  }
-  // One operand element (or vector of N elements) of a gather load; lanes out
-  // of range (ok == false) read a zero block instead. The load itself is
-  // unconditional and its value is used as loaded: a lane-masked load, or a
-  // select on the loaded value, makes the compiler wait for the loads in
-  // flight right there instead of at the LDS store.
-  constexpr int VW = 16 / (int)sizeof(T);
-  const T *zpad = static_cast<const T *>(p.zpad);
-  auto gather_vec = [&](const T *X, int64_t off, bool ok, T *dst, auto n) {
-    constexpr int N = decltype(n)::value;
-    typedef T TN __attribute__((ext_vector_type(N)));
-    const TN v = *reinterpret_cast<const TN *>(ok ? X + off : zpad);
-#pragma unroll
-    for (int e = 0; e < N; ++e) dst[e] = v[e];
-  };
-  auto gather_one = [&](const T *X, int64_t off, bool ok, int conj, T &re, T &im) {
-    if (CPLX) {
-      const T *q = ok ? X + 2 * off : zpad;
-      re = q[0];
-      const T b = q[1];
-      im = conj ? -b : b;
-    } else {
-      re = *(ok ? X + off : zpad);
-    }
-  };
-  // Gather staging of one operand tile, kf: along k (row offset fixed), else
-  // along rows. kbase is the table entry of the thread's first k (loaded one
-  // tile ahead), row_base the offset of its first row. GATHER == 1: a
-  // thread's consecutive k (rows) stay inside one run of the first contracted
-  // (row) dimension, stride ks0 (rs0) (the launcher checks the extents);
-  // GATHER == 2: each k (row) looks up its own table entry. vec: 16-byte (k
-  // direction) or RV-element (row direction) groups are contiguous.
-  auto gather_load = [&](const T *X, const int64_t *rowtab, int64_t row_base, int64_t rs0, const int64_t *kof,
-                         int64_t kbase, int64_t ks0, int64_t rows, int64_t row0,
-                         int k_off, int64_t k0, bool vec, int conj, auto kf, auto dst) {
-    constexpr int L = (int)(sizeof(dst[0]) / sizeof(T));
-    constexpr bool RUNS = GATHER == 1;
-    // GATHER == 1 kernels of real kinds always take the vector path (the
-    // launcher checks it applies): a run-time choice between vector and
-    // scalar loads made the compiler wait for one operand's loads before
-    // issuing the other's
-    if (RUNS && !CPLX) vec = true;
-    const int64_t kk0 = k0 + k_off;
-    if (decltype(kf)::value) {
-      const bool rok = row0 < rows;
-      if (RUNS) {
-        if (!CPLX && vec) {
-#pragma unroll
-          for (int i = 0; i < L; i += VW)
-            gather_vec(X, row_base + kbase + i, rok && kk0 + i < kend, &dst[0][i], std::integral_constant<int, VW>());
-        } else {
-#pragma unroll
-          for (int i = 0; i < L; ++i)
-            gather_one(X, row_base + kbase + i * ks0, rok && kk0 + i < kend, conj, dst[0][i], dst[1 % NP][i]);
-        }
-      } else if (!CPLX && vec) {
-#pragma unroll
-        for (int i = 0; i < L; i += VW) {
-          const bool ok = rok && kk0 + i < kend;
-          gather_vec(X, row_base + kof[ok ? kk0 + i : 0], ok, &dst[0][i], std::integral_constant<int, VW>());
-        }
-      } else {
-#pragma unroll
-        for (int i = 0; i < L; ++i) {
-          const bool ok = rok && kk0 + i < kend;
-          gather_one(X, row_base + kof[ok ? kk0 + i : 0], ok, conj, dst[0][i], dst[1 % NP][i]);
-        }
-      }
-    } else {
-      constexpr int KV = L / RV;
-#pragma unroll
-      for (int j = 0; j < KV; ++j) {
-        const bool kok = kk0 + j < kend;
-        const int64_t ko = RUNS ? kbase + j * ks0 : (j == 0 ? kbase : kof[kok ? kk0 + j : 0]);
-        if (!CPLX && vec) {
-          // rows come in contiguous groups of RV (the row extent is a multiple)
-          const int64_t ro = RUNS ? row_base : rowtab[row0 < rows ? row0 : 0];
-          gather_vec(X, ro + ko, kok && row0 < rows, &dst[0][j * RV], std::integral_constant<int, RV>());
-        } else {
-#pragma unroll
-          for (int e = 0; e < RV; ++e) {
-            const bool ok = kok && row0 + e < rows;
-            const int64_t ro = RUNS ? row_base + e * rs0 : rowtab[ok ? row0 + e : 0];
-            gather_one(X, ro + ko, ok, conj, dst[0][j * RV + e], dst[1 % NP][j * RV + e]);
-          }
-        }
-      }
-    }
-  };
-  // table entry of a thread's first k in the tile at k0 (clamped into range)
-  auto kof_at = [&](const int64_t *kof, int64_t k0, int k_off) -> int64_t {
-    const int64_t kk = k0 + k_off;
-    return kof[kk < kend ? kk : kbeg];
-  };
-  int64_t ka_next = 0, kb_next = 0;  // gather: entries of the next tile to load
-
-  // Matricized staging of one operand tile: X stored rows x k with leading
-  // dimension ld (k fastest when kf, rows fastest otherwise); vec: 16-byte
-  // aligned rows (kf) or columns.
-  // force: the caller has checked that the vector form applies.
-  auto mat_load = [&](const T *X, int64_t ld, int64_t rows, int64_t row0, int k_off, int64_t k0, bool vec,
-                      bool interior, int conj, auto kf, auto dst, auto force) {
-    constexpr int L = (int)(sizeof(dst[0]) / sizeof(T));
-    constexpr bool F = decltype(force)::value;
-    const int64_t kk0 = k0 + k_off;
-    if (decltype(kf)::value) {
-      if (F || (!CPLX && vec && interior && k0 + BK <= kend)) {
-        const T *src = X + row0 * ld + kk0;
-#pragma unroll
-        for (int i = 0; i < L; i += VW) {
-          typedef T TV __attribute__((ext_vector_type(16 / sizeof(T))));
-          const TV v = *reinterpret_cast<const TV *>(src + i);
-#pragma unroll
-          for (int e = 0; e < VW; ++e) dst[0][i + e] = v[e];
-        }
-        return;
-      }
-#pragma unroll
-      for (int i = 0; i < L; ++i) {
-        const int64_t kk = kk0 + i;
-        const bool ok = row0 < rows && kk < kend;
-        const int64_t off = row0 * ld + kk;
-        if (CPLX) {
-          dst[0][i] = ok ? X[2 * off] : T(0);
-          const T im = ok ? X[2 * off + 1] : T(0);
-          dst[1 % NP][i] = conj ? -im : im;
-        } else {
-          dst[0][i] = ok ? X[off] : T(0);
-        }
-      }
-    } else {
-      constexpr int KV = L / RV;
-      if (F || (!CPLX && vec && interior && k0 + BK <= kend)) {
-        typedef T TR __attribute__((ext_vector_type(RV)));
-#pragma unroll
-        for (int j = 0; j < KV; ++j) {
-          const TR v = *reinterpret_cast<const TR *>(X + (kk0 + j) * ld + row0);
-#pragma unroll
-          for (int e = 0; e < RV; ++e) dst[0][j * RV + e] = v[e];
-        }
-        return;
-      }
-#pragma unroll
-      for (int j = 0; j < KV; ++j)
-#pragma unroll
-        for (int e = 0; e < RV; ++e) {
-          const int64_t kk = kk0 + j, r = row0 + e;
-          const bool ok = r < rows && kk < kend;
-          const int64_t off = kk * ld + r;
-          if (CPLX) {
-            dst[0][j * RV + e] = ok ? X[2 * off] : T(0);
-            const T im = ok ? X[2 * off + 1] : T(0);
-            dst[1 % NP][j * RV + e] = conj ? -im : im;
-          } else {
-            dst[0][j * RV + e] = ok ? X[off] : T(0);
-          }
-        }
-    }
-  };
-
-  T ra[NP][LA], rb[NP][LB];
-  auto load_a = [&](int64_t k0) {
-    if (GATHER)
-      gather_load(A, p.a_row, ga_row, p.a_rs0, p.a_kof, ka_next, p.a_ks0, p.m, m0 + a_r, a_k, k0,
-                  p.vec_a != 0, p.conj_a, std::integral_constant<bool, AK>(), ra);
-    else
-      mat_load(A, p.lda, p.m, m0 + a_r, a_k, k0, p.vec_a != 0, interior_mn, p.conj_a,
-               std::integral_constant<bool, AK>(), ra, std::false_type());
-  };
-  auto load_b = [&](int64_t k0) {
-    if (GATHER)
-      gather_load(B, p.b_row, gb_row, p.b_rs0, p.b_kof, kb_next, p.b_ks0, p.n, n0 + b_r, b_k, k0,
-                  p.vec_b != 0, p.conj_b, std::integral_constant<bool, BKF>(), rb);
-    else
-      mat_load(B, p.ldb, p.n, n0 + b_r, b_k, k0, p.vec_b != 0, interior_mn, p.conj_b,
-               std::integral_constant<bool, BKF>(), rb, std::false_type());
-  };
-  // Both operands of a tile: when both take the vector form, their loads are
-  // issued back to back in one branch (separate per-operand choices made the
-  // compiler wait for A's loads at the join before issuing B's).
-  auto load_ab = [&](int64_t k0) {
-    if (!GATHER && !CPLX && p.vec_a && p.vec_b && interior_mn && k0 + BK <= kend) {
-      mat_load(A, p.lda, p.m, m0 + a_r, a_k, k0, true, true, 0, std::integral_constant<bool, AK>(), ra,
-               std::true_type());
-      mat_load(B, p.ldb, p.n, n0 + b_r, b_k, k0, true, true, 0, std::integral_constant<bool, BKF>(), rb,
-               std::true_type());
-      return;
-    }
-    load_a(k0);
-    load_b(k0);
-  };
-  // LDS store of one operand's staged tile: k-fast rows in 16-byte pieces;
-  // row-fast: each of the RV rows gets its KV consecutive k in one store.
-  auto lds_store = [&](auto S, const auto &r, int row, int k, auto kf) {
-    constexpr int L = (int)(sizeof(r[0]) / sizeof(T));
-#pragma unroll
-    for (int q = 0; q < NP; ++q) {
-      if (decltype(kf)::value) {
-#pragma unroll
-        for (int i = 0; i < L; i += VW) {
-          typedef T TV __attribute__((ext_vector_type(16 / sizeof(T))));
-          TV v;
-#pragma unroll
-          for (int e = 0; e < VW; ++e) v[e] = r[q][i + e];
-          *reinterpret_cast<TV *>(&S[q][row][k + i]) = v;
-        }
-      } else {
-        constexpr int KV = L / RV;
-#pragma unroll
-        for (int e = 0; e < RV; ++e) {
-          if constexpr (KV == 1) {
-            S[q][row + e][k] = r[q][e];
-          } else {
-            typedef T TK __attribute__((ext_vector_type(KV)));
-            TK v;
-#pragma unroll
-            for (int j = 0; j < KV; ++j) v[j] = r[q][j * RV + e];
-            *reinterpret_cast<TK *>(&S[q][row + e][k]) = v;
-          }
-        }
-      }
-    }
-  };
-  auto store = [&](int buf) {
-    lds_store(As[buf], ra, a_r, a_k, std::integral_constant<bool, AK>());
-    lds_store(Bs[buf], rb, b_r, b_k, std::integral_constant<bool, BKF>());
-  };
-
-  AccT acc[NP][FM][FN];
-#pragma unroll
-  for (int q = 0; q < NP; ++q)
-#pragma unroll
-    for (int i = 0; i < FM; ++i)
-#pragma unroll
-      for (int j = 0; j < FN; ++j) acc[q][i][j] = AccT{0, 0, 0, 0};
-
-  const int64_t nk = (kend - kbeg + BK - 1) / BK;
-  if (GATHER) {
-    ka_next = kof_at(p.a_kof, kbeg, a_k);
-    kb_next = kof_at(p.b_kof, kbeg, b_k);
-  }
-  load_ab(kbeg);
-  if (GATHER) {  // table entries one tile ahead of the operand loads
-    ka_next = kof_at(p.a_kof, kbeg + BK, a_k);
-    kb_next = kof_at(p.b_kof, kbeg + BK, b_k);
-  }
-  store(0);
-  __syncthreads();
-  const int fr = lane & 15, fg = (lane >> 4) * 4;
-  for (int64_t kt = 0; kt < nk; ++kt) {
-    const int cur = kt & 1;
-    if (kt + 1 < nk) {
-      load_ab(kbeg + (kt + 1) * BK);
-      if (GATHER) {
-        ka_next = kof_at(p.a_kof, kbeg + (kt + 2) * BK, a_k);
-        kb_next = kof_at(p.b_kof, kbeg + (kt + 2) * BK, b_k);
-      }
-    }
-#pragma unroll
-    for (int ks = 0; ks < BK; ks += 16) {
-      F4 fa[NP][FM], fb[NP][FN];
-#pragma unroll
-      for (int q = 0; q < NP; ++q) {
-#pragma unroll
-        for (int i = 0; i < FM; ++i) fa[q][i] = *reinterpret_cast<const F4 *>(&As[cur][q][wm + i * 16 + fr][ks + fg]);
-#pragma unroll
-        for (int j = 0; j < FN; ++j) fb[q][j] = *reinterpret_cast<const F4 *>(&Bs[cur][q][wn + j * 16 + fr][ks + fg]);
-      }
-#pragma unroll
-      for (int st = 0; st < 4; ++st) {
-#pragma unroll
-        for (int i = 0; i < FM; ++i) {
-#pragma unroll
-          for (int j = 0; j < FN; ++j) {
-            const T a0 = st == 0 ? fa[0][i].x : st == 1 ? fa[0][i].y : st == 2 ? fa[0][i].z : fa[0][i].w;
-            const T b0 = st == 0 ? fb[0][j].x : st == 1 ? fb[0][j].y : st == 2 ? fb[0][j].z : fb[0][j].w;
-            if (CPLX) {
-              const F4 &ai4 = fa[1 % NP][i], &bi4 = fb[1 % NP][j];
-              const T a1 = st == 0 ? ai4.x : st == 1 ? ai4.y : st == 2 ? ai4.z : ai4.w;
-              const T b1 = st == 0 ? bi4.x : st == 1 ? bi4.y : st == 2 ? bi4.z : bi4.w;
-              // (ar + i ai)(br + i bi) = (ar br - ai bi) + i (ar bi + ai br)
-              acc[0][i][j] = mfma(a0, b0, acc[0][i][j]);
-              acc[0][i][j] = mfma(-a1, b1, acc[0][i][j]);
-              acc[1 % NP][i][j] = mfma(a0, b1, acc[1 % NP][i][j]);
-              acc[1 % NP][i][j] = mfma(a1, b0, acc[1 % NP][i][j]);
-            } else {
-              acc[0][i][j] = mfma(a0, b0, acc[0][i][j]);
-            }
-          }
-        }
-      }
-    }
-    if (kt + 1 < nk) store(cur ^ 1);
-    __syncthreads();
-  }
-  // epilogue: C = alpha * acc + beta * C (beta 0 or 1), or the raw partial
-  T *C = static_cast<T *>(p.c);
-  T *Pz = split ? static_cast<T *>(p.part) + (int64_t)blockIdx.y * p.m * p.n : nullptr;
-  const T ar = (T)p.alpha_re, ai = (T)p.alpha_im;
-  const int fk = (lane >> 4) & 3;
-  int64_t gcol[FN];
-  if (GATHER && !split) {
-#pragma unroll
-    for (int j = 0; j < FN; ++j) {
-      const int64_t col = n0 + wn + j * 16 + fr;
-      gcol[j] = p.c_col[col < p.n ? col : 0];
-    }
-  }
-  // Per 16-row block of the wave: the offsets (-1: outside C), then every C
-  // load of the block at once (clamped addresses, no lane-masked branches),
-  // one wait, then the stores; a load-add-store per element would wait for
-  // each load in turn behind the stores already issued.
-#pragma unroll
-  for (int i = 0; i < FM; ++i) {
-    int64_t off[FN][4];
-    T cv[FN][4][NP];
-    // accumulator layout: FP32 16x16x4 keeps rows 4*(lane/16)+r in a lane,
-    // FP64 16x16x4 keeps rows lane/16 + 4*r
-    int64_t grow[4];
-    if (GATHER && !split) {
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int64_t row = m0 + wm + i * 16 + (sizeof(T) == 8 ? fk + 4 * r : fk * 4 + r);
-        grow[r] = p.c_row[row < p.m ? row : 0];
-      }
-    }
-#pragma unroll
-    for (int j = 0; j < FN; ++j) {
-      const int64_t col = n0 + wn + j * 16 + fr;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int64_t row = m0 + wm + i * 16 + (sizeof(T) == 8 ? fk + 4 * r : fk * 4 + r);
-        off[j][r] = (row < p.m && col < p.n)
-                        ? (split ? (p.part_rowmajor ? row * p.n + col : row + col * p.m)
-                                 : GATHER ? grow[r] + gcol[j] : row + col * p.ldc)
-                        : -1;
-      }
-    }
-    if (!split && !p.beta_zero) {
-#pragma unroll
-      for (int j = 0; j < FN; ++j)
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-#pragma unroll
-          for (int q = 0; q < NP; ++q) cv[j][r][q] = C[NP * (off[j][r] < 0 ? 0 : off[j][r]) + q];
-      wait_all_vmem();  // on every lane, before the lane-masked stores
-    } else {
-#pragma unroll
-      for (int j = 0; j < FN; ++j)
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-#pragma unroll
-          for (int q = 0; q < NP; ++q) cv[j][r][q] = T(0);
-    }
-#pragma unroll
-    for (int j = 0; j < FN; ++j)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        if (off[j][r] < 0) continue;
-        if (CPLX) {
-          const T xr = acc[0][i][j][r], xi = acc[1 % NP][i][j][r];
-          C[2 * off[j][r]] = ar * xr - ai * xi + cv[j][r][0];
-          C[2 * off[j][r] + 1] = ar * xi + ai * xr + cv[j][r][1 % NP];
-        } else if (split) {
-          Pz[off[j][r]] = acc[0][i][j][r];
-        } else {
-          C[off[j][r]] = ar * acc[0][i][j][r] + cv[j][r][0];
-        }
-      }
-  }
-}
 
 // ---------------------------------------------------------------------------
 // Three-way BF16 split (helpers in bf16x3.hpp): six bf16 products per k-step
@@ -708,11 +204,7 @@ struct B3Params {
 // rows per k-step for 32 tiles.
 __device__ __forceinline__ void tile_of_b3(const B3Params &p, int &tm, int &tn)
 {
-  GemmParams q{};
-  q.tiles_m = p.tiles_m;
-  q.tiles_n = p.tiles_n;
-  q.xcd_remap = 1;
-  tile_of<4>(q, tm, tn);
+  tile_walk<4>(xcd_order(blockIdx.x, gridDim.x), p.tiles_m, p.tiles_n, tm, tn);
 }
 
 // Issue the DMA of one k-stage: NL 1 KB blocks (A planes x row bands, then B),
@@ -955,99 +447,6 @@ __global__ __launch_bounds__(256) void k_realify(const T *__restrict__ x, int64_
   }
 }
 
-template <typename K>
-int launch_grid(K kern, const GemmParams &p, hipStream_t s)
-{
-  const int nb = p.tiles_m * p.tiles_n;
-  const int nz = p.part ? (int)((p.k + p.kchunk - 1) / p.kchunk) : 1;
-  hipLaunchKernelGGL(kern, dim3(nb, nz), dim3(256), 0, s, p);
-  return XT_HIP_OK(hipGetLastError()) ? 0 : TALSH_FAILURE;
-}
-
-// C = alpha * sum_z part[z] (+ C) for split-K partials of a real GEMM, summed
-// in FP64; C and the partials are m x n column-major with leading dimension m.
-template <typename T>
-__global__ __launch_bounds__(256) void k_splitk_sum(const T *__restrict__ part, int nz, int64_t mn,
-                                                    T *__restrict__ c, double alpha, int beta_zero)
-{
-  const int64_t st = (int64_t)gridDim.x * 256;
-  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < mn; i += st) {
-    double v = 0.0;
-    for (int z = 0; z < nz; ++z) v += (double)part[(int64_t)z * mn + i];
-    v *= alpha;
-    if (!beta_zero) v += (double)c[i];
-    c[i] = (T)v;
-  }
-}
-
-// Split-K sum of a gathered product: the partials are m x n, column-major or
-// (rowmajor) row-major; C element (r, c) sits at c_row[r] + c_col[c]. The
-// launcher makes the partials row-major when D's stride-1 index leads the
-// columns, so both the product's epilogue (16 consecutive columns per row)
-// and this sum write along it.
-template <typename T>
-__global__ __launch_bounds__(256) void k_splitk_sum_gather(const T *__restrict__ part, int nz, int64_t m, int64_t n,
-                                                           int rowmajor, const int64_t *__restrict__ c_row,
-                                                           const int64_t *__restrict__ c_col, T *__restrict__ c,
-                                                           double alpha, int beta_zero)
-{
-  const int64_t st = (int64_t)gridDim.x * 256, mn = m * n;
-  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < mn; i += st) {
-    int64_t row, col;
-    if (rowmajor) { row = i / n; col = i - row * n; }
-    else { col = i / m; row = i - col * m; }
-    const int64_t off = c_row[row] + c_col[col];
-    double v = 0.0;
-    for (int z = 0; z < nz; ++z) v += (double)part[(int64_t)z * mn + i];
-    v *= alpha;
-    if (!beta_zero) v += (double)c[off];
-    c[off] = (T)v;
-  }
-}
-
-// Offset tables of a gathered product, back to back: table t holds
-// count[t] = prod(ext[t][.]) entries, entry i = sum_j digit_j(i) * str[t][j].
-// After the tables, from entry zero0 on, kGatherZeroWords zero entries (the
-// zero block of out-of-range gather loads).
-constexpr int kGatherZeroWords = 8;
-struct GatherTables {
-  int64_t *out;
-  int64_t start[7];  // first entry of table t; start[6] = total
-  int64_t zero0;     // first zero entry (even, so the block is 16-byte aligned)
-  int nd[6];
-  int ext[6][kGatherMaxDims];
-  int64_t str[6][kGatherMaxDims];
-};
-
-__global__ __launch_bounds__(256) void k_gather_tables(const GatherTables g)
-{
-  const int64_t st = (int64_t)gridDim.x * 256;
-  if (blockIdx.x == 0 && threadIdx.x < kGatherZeroWords) g.out[g.zero0 + threadIdx.x] = 0;
-  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < g.start[6]; i += st) {
-    int t = 0;
-    while (t < 5 && i >= g.start[t + 1]) ++t;
-    int64_t x = i - g.start[t], off = 0;
-    for (int j = 0; j < g.nd[t]; ++j) {
-      const int64_t e = g.ext[t][j];
-      const int64_t q = x / e;
-      off += (x - q * e) * g.str[t][j];
-      x = q;
-    }
-    g.out[i] = off;
-  }
-}
-
-template <typename T, bool CPLX, int BM, int BN, int BK, int OCC, int GATHER = 0>
-int launch_family(GemmParams p, bool ak, bool bk, hipStream_t s)
-{
-  p.tiles_m = (int)((p.m + BM - 1) / BM);
-  p.tiles_n = (int)((p.n + BN - 1) / BN);
-  if (ak && bk) return launch_grid(k_gemm_mfma<T, CPLX, true, true, BM, BN, BK, OCC, GATHER>, p, s);
-  if (ak) return launch_grid(k_gemm_mfma<T, CPLX, true, false, BM, BN, BK, OCC, GATHER>, p, s);
-  if (bk) return launch_grid(k_gemm_mfma<T, CPLX, false, true, BM, BN, BK, OCC, GATHER>, p, s);
-  return launch_grid(k_gemm_mfma<T, CPLX, false, false, BM, BN, BK, OCC, GATHER>, p, s);
-}
-
 constexpr int kB3Form = 16;               // kernel form of the three-way split
 
 int64_t round_up(int64_t x, int64_t q) { return (x + q - 1) / q * q; }
@@ -1150,27 +549,73 @@ int current_cus()
   return cus;
 }
 
-// Split-K of a real FP64/FP32 GEMM on 64x64 tiles: when the output has fewer
-// tiles than two resident workgroups per CU, K is cut into parts of >= 256
-// k-values (multiples of the 16-deep k-step) so that the grid fills the chip;
-// the partials are summed in FP64 by k_splitk_sum. Returns the number of
-// parts (1: no split) and the chunk length.
-int splitk_parts_cus(const GemmArgs &g, int tile, int cus, int64_t *kchunk)
+// Output tiles of the native-precision kernels: rows x columns and the k-depth
+// of one LDS stage (128 bytes of a row; complex kinds hold two planes).
+struct TileShape { int bm, bn, bk, groups; };
+TileShape tile_shape(int kind, int tile)
 {
-  *kchunk = (int64_t)g.k;
-  const bool real = g.kind == R8 || (g.kind == R4 && g.r4mode == R4Mode::kNativeF32);
-  if (!real || tile != 2 || g.k < 512) return 1;
-  const int64_t tiles = (int64_t)((g.m + 63) / 64) * (int64_t)((g.n + 63) / 64);
-  const int64_t want = 2 * (int64_t)cus;
-  if (tiles >= want) return 1;
-  int64_t nz = std::min<int64_t>({8, want / tiles, (int64_t)g.k / 256});
-  if (nz < 2) return 1;
-  const int64_t chunk = ((int64_t)g.k + nz - 1) / nz;
-  *kchunk = (chunk + 15) / 16 * 16;
-  return (int)(((int64_t)g.k + *kchunk - 1) / *kchunk);
+  const int bk = kind == R4 ? 32 : 16;
+  if (kind == C8 || kind == C4) return {64, 64, bk, tile == 1 ? 2 : 1};
+  return tile == 2 ? TileShape{64, 64, bk, 1} : tile == 1 ? TileShape{64, 64, bk, 4} : TileShape{128, 128, bk, 1};
 }
 
-int splitk_parts(const GemmArgs &g, int tile, int64_t *kchunk) { return splitk_parts_cus(g, tile, current_cus(), kchunk); }
+bool native_real(const GemmArgs &g) { return g.kind == R8 || (g.kind == R4 && g.r4mode == R4Mode::kNativeF32); }
+
+// How a product's tiles are cut along K: tiles [0, full) run whole, the later
+// ones in `parts` pieces of kchunk k-values.
+struct SplitGeom {
+  int64_t tiles = 0, full = 0, kchunk = 0, zstride = 0;
+  int parts = 1;
+  size_t bytes = 0;  // workspace of the partials
+};
+
+// Cost model of the cut. Workgroups of several k-groups fill a CU alone; of
+// the others a CU holds two, and one alone hides its latencies worse (a 64x64
+// FP64 tile per CU runs at 41 TFLOP/s, two at 51, a 128x128 one at 58 and 63).
+// Whole rounds of tiles need no cut; what is left over is cut into the number
+// of parts that ends soonest, the sum of the pieces (a launch and a pass over
+// the partials) included. Pieces are at least 128 k-values deep. budget:
+// bytes available for the partials.
+SplitGeom split_geom(const GemmArgs &g, const TileShape &ts, int cus, size_t budget)
+{
+  SplitGeom G;
+  const int64_t m = (int64_t)g.m, n = (int64_t)g.n, k = (int64_t)g.k;
+  const int64_t tm = (m + ts.bm - 1) / ts.bm, tn = (n + ts.bn - 1) / ts.bn;
+  G.tiles = G.full = tm * tn;
+  G.kchunk = k;
+  const int es = kind_size(g.kind);
+  const bool cplx = g.kind == C8 || g.kind == C4, dp = g.kind == R8 || g.kind == C8;
+  const int64_t round = (ts.groups > 1 ? 1 : 2) * (int64_t)cus;
+  const int64_t full = G.tiles / round * round, rem = G.tiles - full;
+  if (rem == 0 || k < 256 || k > kMaxDepth) return G;
+  // microseconds of one tile on a CU of its own at 80% of its matrix rate
+  const double tau = (cplx ? 8.0 : 2.0) * ts.bm * ts.bn * (double)k / (0.8 * (dp ? 78.6e6 : 157.3e6) / 256.0);
+  auto cost = [&](int64_t parts) {
+    const int64_t q = (rem * parts + cus - 1) / cus;  // pieces per CU
+    const double eff = q > 1 || ts.groups > 1 ? 1.0 : 0.8;
+    double c = tau * (double)q / (double)parts / eff;
+    if (parts > 1) c += 8.0 + 2.0 * (double)rem * ts.bm * ts.bn * es * (double)parts / 4.0e6;
+    return c;
+  };
+  double best = 0.95 * cost(1);
+  for (int64_t parts = 2; parts <= 64 && k / parts >= 128; ++parts) {
+    const int64_t chunk = ((k + parts - 1) / parts + ts.bk - 1) / ts.bk * ts.bk;
+    if ((k + chunk - 1) / chunk != parts) continue;
+    const int64_t zs = full > 0 ? rem * ts.bm * ts.bn : m * n;
+    const size_t bytes = (size_t)parts * (size_t)zs * es;
+    if (bytes > budget) break;
+    const double c = cost(parts);
+    if (c < best) {
+      best = c;
+      G.full = full;
+      G.parts = (int)parts;
+      G.kchunk = chunk;
+      G.zstride = zs;
+      G.bytes = bytes;
+    }
+  }
+  return G;
+}
 
 // Large complex products in native precision run realified through the real
 // 128x128 kernels (which re-read operands from L2 half as often as the 64x64
@@ -1189,13 +634,28 @@ size_t realified_bytes(const GemmArgs &g)
   return ((2 * g.m * k2 * es + 255) / 256 * 256) + g.n * k2 * es + 16;
 }
 
+// Tile choice of the kernels: a caller's, or the default; complex kinds have
+// one choice, their two forms are told apart here (two k-groups per workgroup
+// when the tiles do not give every CU two workgroups).
+int resolved_tile(const GemmArgs &g)
+{
+  if (g.kind == C8 || g.kind == C4) {
+    const int64_t tiles = (int64_t)((g.m + 63) / 64) * (int64_t)((g.n + 63) / 64);
+    return tiles < 2 * (int64_t)current_cus() ? 1 : 0;
+  }
+  return g.tile < 0 ? gemm_default_tile(g.kind, g.r4mode, g.m, g.n, g.k) : g.tile;
+}
+
+// Partials of the published workspace query (talshAmdGemmWorkspace): up to
+// eight pieces of a real product with few 64x64 output tiles.
 size_t gemm_workspace_bytes(const GemmArgs &g)
 {
   if (!gemm_uses_split3(g)) {
     if (g.kind == C8 || g.kind == C4) return complex_realified(g) ? realified_bytes(g) : 0;
-    const int tile = g.tile < 0 ? gemm_default_tile(g.kind, g.r4mode, g.m, g.n, g.k) : g.tile;
-    int64_t kc;
-    const int nz = splitk_parts(g, tile, &kc);
+    if (resolved_tile(g) == 0 || g.k < 512) return 0;
+    const int64_t tiles = (int64_t)((g.m + 63) / 64) * (int64_t)((g.n + 63) / 64);
+    const int64_t want = 2 * (int64_t)current_cus();
+    const int64_t nz = tiles >= want ? 1 : std::min<int64_t>({8, want / tiles, (int64_t)g.k / 256});
     return nz > 1 ? (size_t)nz * g.m * g.n * (size_t)kind_size(g.kind) + 16 : 0;
   }
   const B3Geom G = b3_geom(g);
@@ -1203,6 +663,24 @@ size_t gemm_workspace_bytes(const GemmArgs &g)
   const int64_t cx = g.kind == C4 ? 2 : 1;
   return (size_t)(3 * (G.plane_a + G.plane_b)) * sizeof(unsigned short) +
          (size_t)(G.nz * cx * (int64_t)g.m * (int64_t)g.n) * 4 + 16;
+}
+
+// Bytes of partials worth having for a product whose workspace is free to
+// choose (a contraction's temporaries); a product runs with less, or none.
+size_t gemm_split_bytes(const GemmArgs &g)
+{
+  if (gemm_uses_split3(g) || complex_realified(g) || g.m == 0 || g.n == 0 || g.k == 0) return 0;
+  return split_geom(g, tile_shape(g.kind, resolved_tile(g)), current_cus(), kSplitBytesMax).bytes;
+}
+
+// The partials, and room that keeps a gathered contraction subject to the
+// arena's back-pressure like one with transposes (the kernels need none of
+// it: they compute their offsets).
+size_t gemm_gather_workspace_bytes(const GemmArgs &g)
+{
+  if (gemm_uses_split3(g)) return 0;
+  const size_t room = ((2 * (g.m + g.n + g.k) + 10) * sizeof(int64_t) + 255) / 256 * 256;
+  return room + (g.kind == C8 || g.kind == C4 ? 0 : gemm_workspace_bytes(g));
 }
 
 int launch_gemm(const GemmArgs &g, hipStream_t s) { return launch_gemm_ws(g, nullptr, 0, s); }
@@ -1240,9 +718,9 @@ int gemm_default_tile(int kind, R4Mode r4mode, size_t m, size_t n, size_t k)
 int gemm_splitk_count(int kind, R4Mode r4mode, size_t m, size_t n, size_t k, int tile, int cus)
 {
   GemmArgs g{};
-  g.kind = kind; g.r4mode = r4mode; g.m = m; g.n = n; g.k = k;
-  int64_t kc;
-  return splitk_parts_cus(g, tile, cus, &kc);
+  g.kind = kind; g.r4mode = r4mode; g.m = m; g.n = n; g.k = k; g.tile = tile;
+  if (gemm_uses_split3(g) || complex_realified(g) || k == 0) return 1;
+  return split_geom(g, tile_shape(kind, tile), cus, kSplitBytesMax).parts;
 }
 
 int gemm_tile_choices(int kind, R4Mode r4mode)
@@ -1255,271 +733,228 @@ void gemm_tile_shape(int kind, R4Mode r4mode, int tile, int *bm, int *bn, int *o
 {
   *bm = *bn = 128;
   *occupancy = 2;
-  if (kind == C8 || kind == C4) { *bm = *bn = 64; return; }
   if (kind == R4 && r4mode == R4Mode::kBF16x3) { *occupancy = 1; return; }
-  if (tile == 1) *occupancy = 1;
-  if (tile == 2) *bm = *bn = 64;
+  const TileShape ts = tile_shape(kind, tile);
+  *bm = ts.bm;
+  *bn = ts.bn;
 }
+
+namespace {
+
+typedef DevGroup<kGatherMaxDims> FullGroup;
+
+FullGroup dev_group(const GatherGroup &g)
+{
+  FullGroup d{};
+  d.nd = g.nd;
+  for (int j = 0; j < g.nd; ++j) {
+    d.str[j] = g.str[j];
+    if (j + 1 < g.nd) {
+      const FastDiv f((uint32_t)g.ext[j]);
+      d.div[j] = DevDivisor{f.d, f.m, f.s};
+    }
+  }
+  return d;
+}
+
+FullGroup line_group(int64_t stride)
+{
+  FullGroup d{};
+  d.nd = 1;
+  d.str[0] = stride;
+  return d;
+}
+
+// Launches product q of g's shape (g.m, g.n after any exchange of A and B) on
+// tile choice `tile`, cutting K as the workspace allows.
+int launch_product(Product &q, const GemmArgs &g, int tile, void *ws, size_t ws_bytes, hipStream_t s)
+{
+  if (q.mode == kWide) tile = 0;  // 64-bit offsets: one tile shape
+  const TileShape ts = tile_shape(g.kind, tile);
+  const int64_t tm = ((int64_t)g.m + ts.bm - 1) / ts.bm, tn = ((int64_t)g.n + ts.bn - 1) / ts.bn;
+  if (tm >= (1ll << 31) || tn >= (1ll << 31) || tm * tn >= (1ll << 31) - 65536) return TALSH_LIMIT_EXCEEDED;
+  auto &p = q.p;
+  p.tiles_m = (int)tm;
+  p.tiles_n = (int)tn;
+  const SplitGeom G = split_geom(g, ts, current_cus(), ws ? ws_bytes : 0);
+  p.part = ws;
+  p.full = (int)G.full;
+  p.parts = G.parts;
+  p.kchunk = G.kchunk;
+  p.zstride = G.zstride;
+  // K beyond kMaxDepth runs in stretches that accumulate in C, one after the
+  // other
+  for (int64_t k0 = 0; k0 < (int64_t)g.k || k0 == 0; k0 += kMaxDepth) {
+    p.k0 = k0;
+    p.k = std::min((int64_t)g.k, k0 + kMaxDepth);
+    if (k0 > 0) p.beta_zero = 0;
+    int e;
+    switch (g.kind) {
+    case R8: e = launch_native_r8(q, tile, s); break;
+    case R4: e = launch_native_r4(q, tile, s); break;
+    case C8:
+    case C4: e = launch_native_cx(q, g.kind, tile, s); break;
+    default: return TALSH_INVALID_ARGS;
+    }
+    if (e) return e;
+  }
+  return 0;
+}
+
+// Exchanges A and B (the product of the transposes, C^T = B^T A^T).
+void exchange(Product &q, GemmArgs &g)
+{
+  auto &p = q.p;
+  std::swap(p.a, p.b);
+  std::swap(p.m, p.n);
+  std::swap(p.conj_a, p.conj_b);
+  std::swap(p.a_row, p.b_row);
+  std::swap(p.a_k, p.b_k);
+  std::swap(p.c_row, p.c_col);
+  std::swap(q.a_kfast, q.b_kfast);
+  std::swap(g.m, g.n);
+}
+
+Product product_of(const GemmArgs &g)
+{
+  Product q;
+  auto &p = q.p;
+  p.a = g.a; p.b = g.b; p.c = g.c;
+  p.m = (int64_t)g.m; p.n = (int64_t)g.n; p.k = (int64_t)g.k;
+  p.alpha_re = g.alpha_re; p.alpha_im = g.alpha_im;
+  p.beta_zero = g.beta_zero ? 1 : 0;
+  p.conj_a = g.conj_a; p.conj_b = g.conj_b;
+  q.a_kfast = g.a_kfast;
+  q.b_kfast = g.b_kfast;
+  return q;
+}
+
+// A matricized product. C is column-major, so A and B change places: the
+// kernels write along the result's columns (16 lanes of a wave on consecutive
+// columns), which then are C's contiguous index.
+int launch_matrix(GemmArgs g, int tile, void *ws, size_t ws_bytes, hipStream_t s)
+{
+  Product q = product_of(g);
+  auto &p = q.p;
+  p.a_row = line_group(g.a_kfast ? p.k : 1);
+  p.a_k = line_group(g.a_kfast ? 1 : p.m);
+  p.b_row = line_group(g.b_kfast ? p.k : 1);
+  p.b_k = line_group(g.b_kfast ? 1 : p.n);
+  p.c_row = line_group(1);
+  p.c_col = line_group(p.m);
+  const int es = kind_size(g.kind);
+  const int64_t lim = (1ll << 31) - 1, bytes = std::max(p.m, p.n) * p.k * es;
+  const bool off32 = p.m <= lim && p.n <= lim && p.k <= lim && bytes < (1ll << 32);
+  const int64_t vw = 16 / es;
+  auto vec = [&](bool kfast, int64_t rows) { return kfast ? p.k % vw == 0 : p.k % 8 == 0 && rows % 2 == 0; };
+  q.mode = !off32 ? kWide : vec(g.a_kfast, p.m) && vec(g.b_kfast, p.n) ? kVec : kUni;
+  exchange(q, g);
+  return launch_product(q, g, tile, ws, ws_bytes, s);
+}
+
+}  // namespace
 
 int launch_gemm_ws(const GemmArgs &g, void *ws, size_t ws_bytes, hipStream_t s)
 {
   if (g.m == 0 || g.n == 0) return 0;
   if (g.k == 0 && !g.beta_zero) return 0;  // empty contraction leaves C unchanged
-  if (ws && ws_bytes < gemm_workspace_bytes(g)) {
-    if (gemm_uses_split3(g)) return TALSH_INVALID_ARGS;
-    ws = nullptr;  // too small for split-K partials: unsplit
+  if (gemm_uses_split3(g)) {
+    if (!ws || ws_bytes < gemm_workspace_bytes(g)) return TALSH_INVALID_ARGS;
+    return launch_bf16x3(g, ws, s);
   }
-  GemmParams p{};
-  p.a = g.a; p.b = g.b; p.c = g.c;
-  p.m = (int64_t)g.m; p.n = (int64_t)g.n; p.k = (int64_t)g.k;
-  p.lda = g.a_kfast ? p.k : p.m;
-  p.ldb = g.b_kfast ? p.k : p.n;
-  p.ldc = p.m;
-  p.alpha_re = g.alpha_re; p.alpha_im = g.alpha_im;
-  p.beta_zero = g.beta_zero ? 1 : 0;
-  p.conj_a = g.conj_a; p.conj_b = g.conj_b;
-  p.xcd_remap = 1;
-  {
-    const int es = kind_size(g.kind);
-    p.vec_a = (((uintptr_t)g.a % 16) == 0) && ((p.lda * es) % 16 == 0);
-    p.vec_b = (((uintptr_t)g.b % 16) == 0) && ((p.ldb * es) % 16 == 0);
-  }
-  if ((p.m + 63) / 64 * ((p.n + 63) / 64) >= (1ll << 31)) return TALSH_LIMIT_EXCEEDED;
-  const int tile = g.tile < 0 ? gemm_default_tile(g.kind, g.r4mode, g.m, g.n, g.k) : g.tile;
-  {
-    int64_t kc;
-    const int nz = ws ? splitk_parts(g, tile, &kc) : 1;
-    if (nz > 1) {
-      p.part = ws;
-      p.kchunk = kc;
-      const int64_t mn = (int64_t)g.m * (int64_t)g.n;
-      const unsigned rb = (unsigned)std::min<int64_t>((mn + 255) / 256, 4096);
-      int e;
-      if (g.kind == R8) {
-        e = launch_family<double, false, 64, 64, 16, 2>(p, g.a_kfast, g.b_kfast, s);
-        if (!e) hipLaunchKernelGGL(k_splitk_sum<double>, dim3(rb), dim3(256), 0, s, static_cast<const double *>(ws), nz,
-                                   mn, static_cast<double *>(g.c), g.alpha_re, p.beta_zero);
-      } else {
-        e = launch_family<float, false, 64, 64, 16, 2>(p, g.a_kfast, g.b_kfast, s);
-        if (!e) hipLaunchKernelGGL(k_splitk_sum<float>, dim3(rb), dim3(256), 0, s, static_cast<const float *>(ws), nz,
-                                   mn, static_cast<float *>(g.c), g.alpha_re, p.beta_zero);
-      }
-      if (e) return e;
-      return XT_HIP_OK(hipGetLastError()) ? 0 : TALSH_FAILURE;
-    }
-  }
-  if (ws && complex_realified(g)) {
-    const bool dp = g.kind == C8;
-    const size_t es = dp ? 8 : 4;
-    const int64_t k2 = 2 * (int64_t)g.k;
-    char *a2 = static_cast<char *>(ws);
-    char *b2 = a2 + (2 * g.m * (size_t)k2 * es + 255) / 256 * 256;
-    const bool real_alpha = g.alpha_im == 0.0;
-    const double are = real_alpha ? 1.0 : g.alpha_re, aim = real_alpha ? 0.0 : g.alpha_im;
-    const int64_t lda = g.a_kfast ? (int64_t)g.k : (int64_t)g.m, ldb = g.b_kfast ? (int64_t)g.k : (int64_t)g.n;
-    const int ga = (int)std::min<int64_t>(((int64_t)g.m * (int64_t)g.k + 255) / 256, 65536);
-    const int gb = (int)std::min<int64_t>(((int64_t)g.n * (int64_t)g.k + 255) / 256, 65536);
-    GemmParams q = p;
-    q.m = 2 * (int64_t)g.m;
-    q.n = (int64_t)g.n;
-    q.k = k2;
-    q.lda = q.ldb = k2;
-    q.ldc = q.m;
-    q.a = a2;
-    q.b = b2;
-    q.conj_a = q.conj_b = 0;
-    q.alpha_re = real_alpha ? g.alpha_re : 1.0;
-    q.alpha_im = 0.0;
-    q.vec_a = q.vec_b = ((k2 * (int64_t)es) % 16) == 0;
-    if (dp) {
-      hipLaunchKernelGGL((k_realify<double, true>), dim3(ga), dim3(256), 0, s, static_cast<const double *>(g.a),
-                         (int64_t)g.m, (int64_t)g.k, lda, g.a_kfast ? 1 : 0, g.conj_a ? 1 : 0, are, aim,
-                         reinterpret_cast<double *>(a2));
-      hipLaunchKernelGGL((k_realify<double, false>), dim3(gb), dim3(256), 0, s, static_cast<const double *>(g.b),
-                         (int64_t)g.n, (int64_t)g.k, ldb, g.b_kfast ? 1 : 0, g.conj_b ? 1 : 0, 1.0, 0.0,
-                         reinterpret_cast<double *>(b2));
-      return launch_family<double, false, 128, 128, 16, 2>(q, true, true, s);
-    }
+  if (!ws) ws_bytes = 0;
+  const int tile = resolved_tile(g);
+  if (!complex_realified(g) || ws_bytes < realified_bytes(g)) return launch_matrix(g, tile, ws, ws_bytes, s);
+  const bool dp = g.kind == C8;
+  const size_t es = dp ? 8 : 4;
+  const int64_t k2 = 2 * (int64_t)g.k;
+  char *a2 = static_cast<char *>(ws);
+  char *b2 = a2 + (2 * g.m * (size_t)k2 * es + 255) / 256 * 256;
+  const bool real_alpha = g.alpha_im == 0.0;
+  const double are = real_alpha ? 1.0 : g.alpha_re, aim = real_alpha ? 0.0 : g.alpha_im;
+  const int64_t lda = g.a_kfast ? (int64_t)g.k : (int64_t)g.m, ldb = g.b_kfast ? (int64_t)g.k : (int64_t)g.n;
+  const int ga = (int)std::min<int64_t>(((int64_t)g.m * (int64_t)g.k + 255) / 256, 65536);
+  const int gb = (int)std::min<int64_t>(((int64_t)g.n * (int64_t)g.k + 255) / 256, 65536);
+  GemmArgs r = g;
+  r.kind = dp ? R8 : R4;
+  r.m = 2 * g.m;
+  r.k = (size_t)k2;
+  r.a = a2;
+  r.b = b2;
+  r.a_kfast = r.b_kfast = true;
+  r.conj_a = r.conj_b = false;
+  r.alpha_re = real_alpha ? g.alpha_re : 1.0;
+  r.alpha_im = 0.0;
+  if (dp) {
+    hipLaunchKernelGGL((k_realify<double, true>), dim3(ga), dim3(256), 0, s, static_cast<const double *>(g.a),
+                       (int64_t)g.m, (int64_t)g.k, lda, g.a_kfast ? 1 : 0, g.conj_a ? 1 : 0, are, aim,
+                       reinterpret_cast<double *>(a2));
+    hipLaunchKernelGGL((k_realify<double, false>), dim3(gb), dim3(256), 0, s, static_cast<const double *>(g.b),
+                       (int64_t)g.n, (int64_t)g.k, ldb, g.b_kfast ? 1 : 0, g.conj_b ? 1 : 0, 1.0, 0.0,
+                       reinterpret_cast<double *>(b2));
+  } else {
     hipLaunchKernelGGL((k_realify<float, true>), dim3(ga), dim3(256), 0, s, static_cast<const float *>(g.a),
                        (int64_t)g.m, (int64_t)g.k, lda, g.a_kfast ? 1 : 0, g.conj_a ? 1 : 0, are, aim,
                        reinterpret_cast<float *>(a2));
     hipLaunchKernelGGL((k_realify<float, false>), dim3(gb), dim3(256), 0, s, static_cast<const float *>(g.b),
                        (int64_t)g.n, (int64_t)g.k, ldb, g.b_kfast ? 1 : 0, g.conj_b ? 1 : 0, 1.0, 0.0,
                        reinterpret_cast<float *>(b2));
-    return launch_family<float, false, 128, 128, 16, 2>(q, true, true, s);
   }
-  switch (g.kind) {
-  case R8:
-    switch (tile) {
-    case 1: return launch_family<double, false, 128, 128, 16, 1>(p, g.a_kfast, g.b_kfast, s);
-    case 2: return launch_family<double, false, 64, 64, 16, 2>(p, g.a_kfast, g.b_kfast, s);
-    default: return launch_family<double, false, 128, 128, 16, 2>(p, g.a_kfast, g.b_kfast, s);
-    }
-  case C8: return launch_family<double, true, 64, 64, 16, 2>(p, g.a_kfast, g.b_kfast, s);
-  case R4:
-    if (g.r4mode == R4Mode::kBF16x3) return launch_bf16x3(g, ws, s);
-    switch (tile) {
-    case 1: return launch_family<float, false, 128, 128, 16, 1>(p, g.a_kfast, g.b_kfast, s);
-    case 2: return launch_family<float, false, 64, 64, 16, 2>(p, g.a_kfast, g.b_kfast, s);
-    default: return launch_family<float, false, 128, 128, 16, 2>(p, g.a_kfast, g.b_kfast, s);
-    }
-  case C4:
-    if (g.r4mode == R4Mode::kBF16x3) return launch_bf16x3(g, ws, s);
-    return launch_family<float, true, 64, 64, 16, 2>(p, g.a_kfast, g.b_kfast, s);
-  default: return TALSH_INVALID_ARGS;
-  }
+  return launch_matrix(r, 0, nullptr, 0, s);
 }
 
-namespace {
-
-int64_t group_count(const GatherGroup &g)
+int launch_gemm_gather(const GemmArgs &args, const GatherMaps &mp, void *ws, size_t ws_bytes, hipStream_t s)
 {
-  int64_t v = 1;
-  for (int j = 0; j < g.nd; ++j) v *= g.ext[j];
-  return v;
-}
-
-// 16-byte groups along a staging direction are contiguous and aligned when the
-// group's first dimension is the tensor's stride-1 dimension with an extent
-// that is a multiple of the vector width (every other stride of the tensor is
-// then a multiple of that extent) and the body is 16-byte aligned.
-bool gather_vec_ok(const GatherGroup &g, int es, const void *base)
-{
-  return g.nd > 0 && g.str[0] == 1 && (g.ext[0] * es) % 16 == 0 && ((uintptr_t)base % 16) == 0;
-}
-
-size_t gather_tables_bytes(const GemmArgs &g)
-{
-  return ((2 * (g.m + g.n + g.k) + 2 + kGatherZeroWords) * sizeof(int64_t) + 255) / 256 * 256;
-}
-
-}  // namespace
-
-size_t gemm_gather_workspace_bytes(const GemmArgs &g)
-{
-  if (gemm_uses_split3(g)) return 0;
-  const size_t tb = gather_tables_bytes(g);
-  if (g.kind == C8 || g.kind == C4) return tb;
-  const int tile = g.tile < 0 ? gemm_default_tile(g.kind, g.r4mode, g.m, g.n, g.k) : g.tile;
-  int64_t kc;
-  const int nz = splitk_parts(g, tile, &kc);
-  return tb + (nz > 1 ? (size_t)nz * g.m * g.n * (size_t)kind_size(g.kind) + 16 : 0);
-}
-
-int launch_gemm_gather(const GemmArgs &g, const GatherMaps &mp, void *ws, size_t ws_bytes, hipStream_t s)
-{
+  GemmArgs g = args;
   if (gemm_uses_split3(g)) return TALSH_NOT_IMPLEMENTED;
   if (g.m == 0 || g.n == 0) return 0;
   if (g.k == 0 && !g.beta_zero) return 0;  // empty contraction leaves C unchanged
   const GatherGroup *grp[6] = {&mp.a_row, &mp.a_k, &mp.b_row, &mp.b_k, &mp.c_row, &mp.c_col};
-  const int64_t want[6] = {(int64_t)g.m, (int64_t)g.k, (int64_t)g.n, (int64_t)g.k, (int64_t)g.m, (int64_t)g.n};
-  GatherTables T{};
-  T.start[0] = 0;
+  const size_t want[6] = {g.m, g.k, g.n, g.k, g.m, g.n};
+  int64_t last[6];  // offset of a group's last index
   for (int t = 0; t < 6; ++t) {
-    if (grp[t]->nd < 0 || grp[t]->nd > kGatherMaxDims || group_count(*grp[t]) != want[t]) return TALSH_INVALID_ARGS;
-    T.nd[t] = grp[t]->nd;
+    if (grp[t]->nd < 0 || grp[t]->nd > kGatherMaxDims) return TALSH_INVALID_ARGS;
+    size_t count = 1;
+    last[t] = 0;
     for (int j = 0; j < grp[t]->nd; ++j) {
       if (grp[t]->ext[j] < 1 || grp[t]->str[j] < 0) return TALSH_INVALID_ARGS;
-      T.ext[t][j] = grp[t]->ext[j];
-      T.str[t][j] = grp[t]->str[j];
+      count *= (size_t)grp[t]->ext[j];
+      last[t] += (int64_t)(grp[t]->ext[j] - 1) * grp[t]->str[j];
     }
-    T.start[t + 1] = T.start[t] + want[t];
+    if (count != want[t]) return TALSH_INVALID_ARGS;
+    if (count > INT32_MAX && grp[t]->nd > 1) return TALSH_LIMIT_EXCEEDED;  // digits are taken in 32 bits
   }
-  const size_t tb = gather_tables_bytes(g);
-  if (!ws || ws_bytes < tb) return TALSH_INVALID_ARGS;
-  if ((int64_t)((g.m + 63) / 64) * (int64_t)((g.n + 63) / 64) >= (1ll << 31)) return TALSH_LIMIT_EXCEEDED;
-  int64_t *tab = static_cast<int64_t *>(ws);
-  T.out = tab;
-  T.zero0 = (T.start[6] + 1) / 2 * 2;
-  hipLaunchKernelGGL(k_gather_tables, dim3((unsigned)std::min<int64_t>((T.start[6] + 255) / 256, 1024)), dim3(256), 0,
-                     s, T);
-  if (!XT_HIP_OK(hipGetLastError())) return TALSH_FAILURE;
-
   const int es = kind_size(g.kind);
-  const bool cplx = g.kind == C8 || g.kind == C4;
-  GemmParams p{};
-  p.a = g.a; p.b = g.b; p.c = g.c;
-  p.m = (int64_t)g.m; p.n = (int64_t)g.n; p.k = (int64_t)g.k;
-  p.alpha_re = g.alpha_re; p.alpha_im = g.alpha_im;
-  p.beta_zero = g.beta_zero ? 1 : 0;
-  p.conj_a = g.conj_a; p.conj_b = g.conj_b;
-  p.xcd_remap = 1;
-  p.vec_a = !cplx && gather_vec_ok(g.a_kfast ? mp.a_k : mp.a_row, es, g.a);
-  p.vec_b = !cplx && gather_vec_ok(g.b_kfast ? mp.b_k : mp.b_row, es, g.b);
-  p.a_row = tab + T.start[0];
-  p.a_kof = tab + T.start[1];
-  p.b_row = tab + T.start[2];
-  p.b_kof = tab + T.start[3];
-  p.c_row = tab + T.start[4];
-  p.c_col = tab + T.start[5];
-  p.zpad = tab + T.zero0;
-  p.a_ks0 = mp.a_k.nd ? mp.a_k.str[0] : 0;
-  p.b_ks0 = mp.b_k.nd ? mp.b_k.str[0] : 0;
-  p.a_rs0 = mp.a_row.nd ? mp.a_row.str[0] : 0;
-  p.b_rs0 = mp.b_row.nd ? mp.b_row.str[0] : 0;
-  // every thread's staged elements (L = 8 on 128x128 tiles, 4 on 64x64) stay
-  // inside runs of the first dimensions: L consecutive k of a k-fast operand;
-  // RV consecutive rows (2 real, 1 complex) at L / RV consecutive k of a
-  // row-fast one
-  auto runs = [&](int L) {
-    const int rv = cplx ? 1 : 2;
-    auto e0 = [](const GatherGroup &q) { return q.nd ? q.ext[0] : 1; };
-    auto ok = [&](bool kf, const GatherGroup &row, const GatherGroup &k) {
-      return kf ? e0(k) % L == 0 : (e0(row) % rv == 0 && e0(k) % (L / rv) == 0);
-    };
-    return ok(g.a_kfast, mp.a_row, mp.a_k) && ok(g.b_kfast, mp.b_row, mp.b_k) && (cplx || (p.vec_a && p.vec_b));
+  Product q = product_of(g);
+  auto &p = q.p;
+  p.a_row = dev_group(mp.a_row);
+  p.a_k = dev_group(mp.a_k);
+  p.b_row = dev_group(mp.b_row);
+  p.b_k = dev_group(mp.b_k);
+  p.c_row = dev_group(mp.c_row);
+  p.c_col = dev_group(mp.c_col);
+  // a k-tile starts at one offset for all lanes when it cannot cross a digit
+  // of the first contracted dimension; operands of real kinds then load
+  // vectors if their runs hold whole ones
+  const int bk = tile_shape(g.kind, 0).bk, vw = 16 / es;
+  auto uniform = [&](const GatherGroup &x) { return x.nd <= 1 || x.ext[0] % bk == 0; };
+  auto vec = [&](bool kfast, const GatherGroup &row, const GatherGroup &k) {
+    const GatherGroup &x = kfast ? k : row;
+    return x.nd > 0 && x.str[0] == 1 && x.ext[0] % (kfast ? vw : 2) == 0 && (kfast || g.k % 8 == 0);
   };
-  const int tile = g.tile < 0 ? gemm_default_tile(g.kind, g.r4mode, g.m, g.n, g.k) : g.tile;
-  if (!cplx) {
-    int64_t kc;
-    const int nz = splitk_parts(g, tile, &kc);
-    const int64_t mn = (int64_t)g.m * (int64_t)g.n;
-    if (nz > 1 && ws_bytes >= tb + (size_t)nz * (size_t)mn * es) {
-      p.part = static_cast<char *>(ws) + tb;
-      p.kchunk = kc;
-      p.part_rowmajor = mp.c_col.nd > 0 && mp.c_col.str[0] == 1;
-      const unsigned rb = (unsigned)std::min<int64_t>((mn + 255) / 256, 4096);
-      int e;
-      if (g.kind == R8) {
-        e = runs(4) ? launch_family<double, false, 64, 64, 16, 2, 1>(p, g.a_kfast, g.b_kfast, s)
-                    : launch_family<double, false, 64, 64, 16, 2, 2>(p, g.a_kfast, g.b_kfast, s);
-        if (!e)
-          hipLaunchKernelGGL(k_splitk_sum_gather<double>, dim3(rb), dim3(256), 0, s,
-                             static_cast<const double *>(p.part), nz, p.m, p.n, p.part_rowmajor, p.c_row, p.c_col,
-                             static_cast<double *>(g.c), g.alpha_re, p.beta_zero);
-      } else {
-        e = runs(4) ? launch_family<float, false, 64, 64, 16, 2, 1>(p, g.a_kfast, g.b_kfast, s)
-                    : launch_family<float, false, 64, 64, 16, 2, 2>(p, g.a_kfast, g.b_kfast, s);
-        if (!e)
-          hipLaunchKernelGGL(k_splitk_sum_gather<float>, dim3(rb), dim3(256), 0, s,
-                             static_cast<const float *>(p.part), nz, p.m, p.n, p.part_rowmajor, p.c_row, p.c_col,
-                             static_cast<float *>(g.c), g.alpha_re, p.beta_zero);
-      }
-      if (e) return e;
-      return XT_HIP_OK(hipGetLastError()) ? 0 : TALSH_FAILURE;
-    }
-  }
-#define XT_GATHER(T_, CPLX_, BM_, OCC_)                                                          \
-  (runs(BM_ / 16) ? launch_family<T_, CPLX_, BM_, BM_, 16, OCC_, 1>(p, g.a_kfast, g.b_kfast, s) \
-                  : launch_family<T_, CPLX_, BM_, BM_, 16, OCC_, 2>(p, g.a_kfast, g.b_kfast, s))
-  switch (g.kind) {
-  case R8:
-    switch (tile) {
-    case 1: return XT_GATHER(double, false, 128, 1);
-    case 2: return XT_GATHER(double, false, 64, 2);
-    default: return XT_GATHER(double, false, 128, 2);
-    }
-  case C8: return XT_GATHER(double, true, 64, 2);
-  case R4:
-    switch (tile) {
-    case 1: return XT_GATHER(float, false, 128, 1);
-    case 2: return XT_GATHER(float, false, 64, 2);
-    default: return XT_GATHER(float, false, 128, 2);
-    }
-  case C4: return XT_GATHER(float, true, 64, 2);
-  default: return TALSH_INVALID_ARGS;
-  }
-#undef XT_GATHER
+  const size_t lim = INT32_MAX;
+  const bool off32 = g.m <= lim && g.n <= lim && g.k <= lim && (last[0] + last[1] + 1) * es < (1ll << 32) &&
+                     (last[2] + last[3] + 1) * es < (1ll << 32);
+  bool small = true;
+  for (int t = 0; t < 6; ++t) small = small && grp[t]->nd <= kSmallDims;
+  q.mode = kGen;
+  if (!off32 || !small) q.mode = kWide;
+  else if (uniform(mp.a_k) && uniform(mp.b_k))
+    q.mode = vec(g.a_kfast, mp.a_row, mp.a_k) && vec(g.b_kfast, mp.b_row, mp.b_k) ? kVec : kUni;
+  const int tile = resolved_tile(g);
+  // write along the columns: they should hold C's stride-1 index
+  if (mp.c_row.nd > 0 && mp.c_row.str[0] == 1 && !(mp.c_col.nd > 0 && mp.c_col.str[0] == 1)) exchange(q, g);
+  return launch_product(q, g, tile, ws, ws_bytes, s);
 }
 
 }  // namespace xt

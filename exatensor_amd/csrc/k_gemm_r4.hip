@@ -1,0 +1,16 @@
+// R4 (FP32) products: tile choices 0 (128x128), 1 (64x64, four k-groups per
+// workgroup) and 2 (64x64).
+#define XT_GEMM_KERNELS
+#include "gemm_native.hpp"
+
+namespace xt {
+
+int launch_native_r4(const Product &q, int tile, hipStream_t s)
+{
+  if (q.mode == kWide) return launch_orient<float, false, 128, 128, 32, 1, 1, 2, kWide>(q, s);
+  if (tile == 2) return launch_modes<float, false, 64, 64, 32, 1, 1, 4>(q, s);
+  if (tile == 1) return launch_modes<float, false, 64, 64, 32, 4, 1, 4>(q, s);
+  return launch_modes<float, false, 128, 128, 32, 1, 1, 2>(q, s);
+}
+
+}  // namespace xt

@@ -63,12 +63,18 @@ int launch_gemm(const GemmArgs &g, hipStream_t s);
 // R4 and C4 products under fast math run as the three-way BF16 split (C4
 // realified: one real product over 2m x 2k and n x 2k operands).
 bool gemm_uses_split3(const GemmArgs &g);
-// Bytes of scratch needed by launch_gemm_ws: BF16x3 split planes and K-chunk
-// partials, or the partials of a split-K real product; 0 otherwise.
+// Bytes of scratch of launch_gemm_ws: BF16x3 split planes and K-chunk partials
+// or realified complex operands, or the partials of a split-K real product;
+// 0 otherwise.
 size_t gemm_workspace_bytes(const GemmArgs &g);
 // ws holds ws_bytes; a workspace smaller than gemm_workspace_bytes(g) is an
-// error for the three-way split and runs a real product unsplit.
+// error for the three-way split; a product in native precision splits K as
+// far as the workspace allows.
 int launch_gemm_ws(const GemmArgs &g, void *ws, size_t ws_bytes, hipStream_t s);
+// Partials that a native-precision product (matricized or gathered) would
+// split K into, at most kSplitBytesMax: optional, it runs with less or none.
+constexpr size_t kSplitBytesMax = size_t(48) << 20;
+size_t gemm_split_bytes(const GemmArgs &g);
 // Fused index gather: a contraction's product read straight from the
 // tensors, no transposes. Each matrix index (rows and k of A and of B, rows
 // and columns of C) is a group of tensor dimensions; element i of a group
@@ -86,9 +92,11 @@ struct GatherGroup {
 struct GatherMaps {
   GatherGroup a_row, a_k, b_row, b_k, c_row, c_col;
 };
-// Workspace of launch_gemm_gather: the six offset tables (8 bytes per index)
-// and, for split K, the partial products.
+// Reservation of a gathered contraction in the arena: 16 bytes per matrix index
+// and the partials of gemm_workspace_bytes.
 size_t gemm_gather_workspace_bytes(const GemmArgs &g);
+// ws: partials of split K (gemm_split_bytes; may be null). Groups of more than
+// one dimension need fewer than 2^31 indices (TALSH_LIMIT_EXCEEDED otherwise).
 int launch_gemm_gather(const GemmArgs &g, const GatherMaps &maps, void *ws, size_t ws_bytes, hipStream_t s);
 // Fixed per-GPU scratch of the allocation-free product entry point: a
 // file-scope device array in k_gemm.hip (64 MiB, held by every GPU the
@@ -101,8 +109,8 @@ int gemm_noalloc_scratch(void **ptr);
 // (bm x bn) and occupancy target of a choice.
 int gemm_tile_choices(int kind, R4Mode r4mode);
 void gemm_tile_shape(int kind, R4Mode r4mode, int tile, int *bm, int *bn, int *occupancy);
-// Number of K parts of a real product in native precision on tile choice
-// `tile` on a GPU with cus compute units (1: no split K).
+// Number of K parts of a product in native precision on tile choice `tile` on
+// a GPU with cus compute units (1: no split K).
 int gemm_splitk_count(int kind, R4Mode r4mode, size_t m, size_t n, size_t k, int tile, int cus);
 // Tile choice of launch_gemm when GemmArgs::tile < 0.
 int gemm_default_tile(int kind, R4Mode r4mode, size_t m, size_t n, size_t k);
