@@ -975,15 +975,24 @@ int talshTensorAdd(const char *cptrn, talsh_tens_t *dtens, talsh_tens_t *ltens, 
   args[0].t = dtens; args[0].output = true;
   args[1].t = ltens;
   struct Body {
-    Arg *D, *L; std::vector<int> ld, o2n; bool conj; double sr, si; void *tmp = nullptr;
+    Arg *D, *L; std::vector<int> ld, o2n; bool conj; double sr, si; void *tmp = nullptr; bool one_pass = false;
     int allocate(Temps &t)
     {
       if (is_identity(o2n)) return 0;
+      // the permutation and the sum in one pass, unless the bodies overlap
+      const size_t bytes = tensor_volume(D->t) * (size_t)kind_size(D->kind);
+      const uintptr_t d0 = (uintptr_t)D->exec, l0 = (uintptr_t)L->exec;
+      one_pass = (d0 + bytes <= l0 || l0 + bytes <= d0) &&
+                 permute_add_planned(D->kind, (int)ld.size(), ld.data(), o2n.data());
+      if (one_pass) return 0;
       return t.alloc(tensor_volume(L->t) * (size_t)kind_size(tensor_kind(L->t)), &tmp);
     }
     int enqueue(Task *k, Device *)
     {
       const void *src = L->exec;
+      if (one_pass)
+        return launch_permute_add(L->exec, D->exec, D->kind, (int)ld.size(), ld.data(), o2n.data(),
+                                  conj && kind_complex(D->kind), sr, si, k->stream);
       if (tmp) {
         int e = launch_permute(L->exec, tmp, L->kind, (int)ld.size(), ld.data(), o2n.data(), false, k->stream);
         if (e) return e;

@@ -195,15 +195,6 @@ int grid_for(uint64_t n)
   return (int)(b < cap ? (b ? b : 1) : cap);
 }
 
-// Real approximant of a complex factor for real data kinds: modulus with the
-// sign of the real part, or the imaginary part when the real part is zero
-// (the CPU path's rule, TALSH/tensor_algebra_cpu.F90:430-445).
-double real_factor(double re, double im)
-{
-  if (re != 0.0) return std::sqrt(re * re + im * im) * (re > 0 ? 1.0 : -1.0);
-  return im;
-}
-
 // ---- box copy: tensor slice and insert ----------------------------------------
 // out[dbase + sum_i x_i ds_i] (+)= in[sbase + sum_i x_i ss_i] over the box
 // x < ext (dimension 0 fastest, its strides 1 on both sides after fusion).
@@ -356,6 +347,12 @@ int launch_box(const void *in, void *out, int kind, int rank, const int *box, co
   }
   if ((int)e.size() - 1 > kBoxDimsWide) return TALSH_LIMIT_EXCEEDED;
   return launch_box_cut(in, out, kind, e, a, b, sbase, dbase, acc, s);
+}
+
+double real_factor(double re, double im)
+{
+  if (re != 0.0) return std::sqrt(re * re + im * im) * (re > 0 ? 1.0 : -1.0);
+  return im;
 }
 
 int launch_fill(void *d, int kind, size_t vol, double re, double im, hipStream_t s)

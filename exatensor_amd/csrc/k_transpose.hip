@@ -8,17 +8,22 @@
 // Design:
 //  * host planner: drop unit extents, fuse input dimensions that stay adjacent
 //    and in order in the output, then pick an LDS tile = the union of an
-//    input-minor dimension group and an output-minor dimension group, grown
-//    until both contiguous runs reach >= 256 bytes (the last dimension of each
-//    group may be split, preferably so that the run is a whole number of
-//    128-byte lines; ragged splits are masked), then grown to >= 8192 elements;
+//    input-minor dimension group and an output-minor dimension group, walked
+//    until both contiguous runs are long enough;
+//  * two forms. Tiles that divide the tensor and whose runs are whole cache
+//    lines of 16-byte vectors: k_permute_tiled, streaming accesses. Everything
+//    else: k_permute_runs, vectors along the runs whatever their alignment;
 //  * LDS padding is chosen on the host by simulating the bank conflicts of the
 //    store phase for each candidate padding period;
-//  * persistent kernel (two resident 512-thread workgroups per CU): each thread decodes
-//    the intra-tile offsets of its vectors once (input offset, output offset,
-//    LDS read base) and keeps them in registers, so the per-tile work is one
-//    base-offset decode per workgroup plus one coalesced load and one
-//    coalesced store per vector.
+//  * persistent kernels (two resident 512-thread workgroups per CU): each thread decodes
+//    the intra-tile offsets of its vectors once and keeps them in registers, so
+//    the per-tile work is one base-offset decode per workgroup plus one
+//    coalesced load and one coalesced store per vector.
+// The run form against the lane-masked single-element tiles it replaces, kernel
+// time: R4 37,29,41,23,31 -> 2,4,1,0,3 132 to 89 us; R8 119,70,65,34 reversed
+// 113 to 71; C8 14,23,104,3,35 43 to 32; 26 instead of 34 us in the geometric
+// mean of 34 random shapes. A permuted addition in one pass: rank-6 extent-24
+// R8 1567 to 890 us.
 #include <algorithm>
 #include <mutex>
 #include <string>
@@ -59,18 +64,11 @@ struct TileParams {
   DevDiv t_out[kMaxTileDims];      // tile extents, store order
   uint64_t os_out[kMaxTileDims];   // output strides, store order
   uint32_t ls_out[kMaxTileDims];   // LDS (load-order linear) strides, store order
-  // ragged (partially tiled) dimensions: position in load / store order
-  int nrag;
-  int rag_in[2], rag_out[2];
-  uint32_t rag_t[2];
   // grid over all fused dims
   int ng;
   DevDiv gdiv[kMaxGridDims];       // number of tiles along each dim
   uint64_t g_is[kMaxGridDims];     // input stride * tile extent
   uint64_t g_os[kMaxGridDims];     // output stride * tile extent
-  uint32_t g_t[kMaxGridDims];      // tile extent along the dim
-  uint32_t g_ext[kMaxGridDims];    // full extent
-  int g_rag[kMaxGridDims];         // ragged slot (0/1) or -1
   uint32_t vol_tile;               // elements per tile
   uint32_t ntiles;
   DevDiv pad;                      // LDS slot = e + e / pad.d (pad.d = 0: no padding)
@@ -97,6 +95,9 @@ __device__ __forceinline__ void opaque(uint32_t &x) { asm volatile("" : "+v"(x))
 
 // Streaming (nontemporal) global accesses: every element is read once and
 // written once, so the data should not displace useful lines from L2/MALL.
+// For tiles whose runs are whole cache lines only (rank-6 extent-24 R8: 595 us
+// against 620 without the hint); a line shared with a neighbouring tile has to
+// wait for the rest of it.
 typedef unsigned int nt1 __attribute__((ext_vector_type(1)));
 typedef unsigned int nt2 __attribute__((ext_vector_type(2)));
 typedef unsigned int nt4 __attribute__((ext_vector_type(4)));
@@ -123,17 +124,42 @@ __device__ __forceinline__ void st_stream(P *p, const P &v)
   __builtin_nontemporal_store(__builtin_bit_cast(U, v), reinterpret_cast<U *>(p));
 }
 
+// Accesses of runs that begin and end inside cache lines, aligned to a 4-byte
+// word only. They are left to the caches (no streaming hint): the rest of a
+// line is the neighbouring tile's, and with the hint the R4 body of extents
+// 37,29,41,23,31 took 124 us instead of 90.
+typedef unsigned int un2 __attribute__((ext_vector_type(2), aligned(4)));
+typedef unsigned int un4 __attribute__((ext_vector_type(4), aligned(4)));
+template <int BYTES>
+struct RunWord;
+template <>
+struct RunWord<4> { typedef unsigned int type; };
+template <>
+struct RunWord<8> { typedef un2 type; };
+template <>
+struct RunWord<16> { typedef un4 type; };
+template <typename P>
+__device__ __forceinline__ P ld_run(const void *p)
+{
+  return __builtin_bit_cast(P, *static_cast<const typename RunWord<sizeof(P)>::type *>(p));
+}
+template <typename P>
+__device__ __forceinline__ void st_run(void *p, const P &v)
+{
+  *static_cast<typename RunWord<sizeof(P)>::type *>(p) = __builtin_bit_cast(typename RunWord<sizeof(P)>::type, v);
+}
+
 // One workgroup walks tiles (persistent grid). Each thread owns EPT vectors of
 // VEC consecutive elements along the input-minor dimension for the load and
 // along the output-minor dimension for the store, so global accesses are
 // 16-byte wide whenever both minor extents allow it.
 //
 // Register budget: a thread keeps per vector only its input offset, output
-// offset and LDS read base (plus the ragged-edge coordinates); the LDS slots
+// offset and LDS read base; the LDS slots
 // are recomputed per tile from those (a few integer operations) instead of
 // being held for every element, which keeps the common instantiations at
 // 30-60 VGPRs, i.e. at full occupancy.
-template <typename W, int VEC, int EPT, bool CONJ, typename OffT, bool RAG>
+template <typename W, int VEC, int EPT, bool CONJ, typename OffT>
 __global__ __launch_bounds__(kTNT) void k_permute_tiled(const W *__restrict__ in, W *__restrict__ out,
                                                         const TileParams p)
 {
@@ -144,12 +170,11 @@ __global__ __launch_bounds__(kTNT) void k_permute_tiled(const W *__restrict__ in
   const uint32_t nvec = p.vol_tile / VEC;
   OffT in_off[EPT], out_off[EPT];
   uint32_t st_ls[EPT];
-  uint32_t rin[RAG ? EPT : 1], rout[RAG ? EPT : 1];
   // one-time decode of this thread's tile vectors (kept in registers)
 #pragma unroll
   for (int k = 0; k < EPT; ++k) {
     const uint32_t v = tid + (uint32_t)k * kTNT;
-    uint32_t r = v, cin[2] = {0, 0}, cout[2] = {0, 0};
+    uint32_t r = v;
     OffT io = 0, oo = 0;
     uint32_t ls = 0;
     for (int j = 0; j < p.nt; ++j) {
@@ -159,10 +184,6 @@ __global__ __launch_bounds__(kTNT) void k_permute_tiled(const W *__restrict__ in
       if (j == 0) c *= VEC;
       r = q;
       io += (OffT)c * (OffT)p.is_in[j];
-      if (RAG) {
-        if (p.rag_in[0] == j) cin[0] = c;
-        if (p.nrag > 1 && p.rag_in[1] == j) cin[1] = c;
-      }
     }
     r = v;
     for (int j = 0; j < p.nt; ++j) {
@@ -173,62 +194,37 @@ __global__ __launch_bounds__(kTNT) void k_permute_tiled(const W *__restrict__ in
       r = q;
       oo += (OffT)c * (OffT)p.os_out[j];
       ls += c * p.ls_out[j];
-      if (RAG) {
-        if (p.rag_out[0] == j) cout[0] = c;
-        if (p.nrag > 1 && p.rag_out[1] == j) cout[1] = c;
-      }
     }
     in_off[k] = io;
     out_off[k] = oo;
     st_ls[k] = ls;
-    if (RAG) {
-      const bool valid = v < nvec;
-      rin[k] = valid ? (cin[0] | (cin[1] << 16)) : 0xFFFFFFFFu;
-      rout[k] = valid ? (cout[0] | (cout[1] << 16)) : 0xFFFFFFFFu;
-    }
   }
   const uint32_t step = p.ls_out[0];
-  struct TileBase { OffT bin, bout; uint32_t rem0, rem1; bool full; };
   // tile base decode (uniform across the workgroup)
-  auto decode = [&](uint32_t tile, TileBase &s) {
-    s.bin = 0;
-    s.bout = 0;
-    uint32_t rem[2] = {0xFFFFu, 0xFFFFu};
+  auto decode = [&](uint32_t tile, OffT &bin, OffT &bout) {
+    bin = bout = 0;
     uint32_t r = tile;
     for (int g = 0; g < p.ng; ++g) {
       const uint32_t q = fdiv(r, p.gdiv[g]);
       const uint32_t c = r - q * p.gdiv[g].d;
       r = q;
-      s.bin += (OffT)c * (OffT)p.g_is[g];
-      s.bout += (OffT)c * (OffT)p.g_os[g];
-      if (RAG && p.g_rag[g] >= 0) {
-        const uint32_t left = p.g_ext[g] - c * p.g_t[g];
-        rem[p.g_rag[g]] = left < p.g_t[g] ? left : p.g_t[g];
-      }
+      bin += (OffT)c * (OffT)p.g_is[g];
+      bout += (OffT)c * (OffT)p.g_os[g];
     }
-    s.rem0 = rem[0];
-    s.rem1 = rem[1];
-    s.full = !RAG || ((rem[0] == p.rag_t[0]) && (p.nrag < 2 || rem[1] == p.rag_t[1]));
   };
   P val[EPT];
-  auto load = [&](const TileBase &s) {
+  auto load = [&](OffT bin) {
 #pragma unroll
-    for (int k = 0; k < EPT; ++k) {
-      const uint32_t v = tid + (uint32_t)k * kTNT;
-      bool ok = v < nvec;
-      if (RAG && !s.full) ok = ok && (rin[k] & 0xFFFFu) < s.rem0 && (rin[k] >> 16) < s.rem1;
-      if (ok) val[k] = ld_stream(reinterpret_cast<const P *>(in + (s.bin + in_off[k])));
-    }
+    for (int k = 0; k < EPT; ++k)
+      if (tid + (uint32_t)k * kTNT < nvec) val[k] = ld_stream(reinterpret_cast<const P *>(in + (bin + in_off[k])));
   };
   // the padding period is a multiple of VEC (checked by the planner), so the
   // VEC slots of one loaded vector are consecutive: base slot + j
-  auto to_lds = [&](const TileBase &s) {
+  auto to_lds = [&]() {
 #pragma unroll
     for (int k = 0; k < EPT; ++k) {
       uint32_t v = tid + (uint32_t)k * kTNT;
-      bool ok = v < nvec;
-      if (RAG && !s.full) ok = ok && (rin[k] & 0xFFFFu) < s.rem0 && (rin[k] >> 16) < s.rem1;
-      if (ok) {
+      if (v < nvec) {
         opaque(v);
         const uint32_t e0 = v * VEC;
         const uint32_t b = e0 + fdiv(e0, p.pad);
@@ -237,13 +233,10 @@ __global__ __launch_bounds__(kTNT) void k_permute_tiled(const W *__restrict__ in
       }
     }
   };
-  auto from_lds = [&](const TileBase &s) {
+  auto from_lds = [&](OffT bout) {
 #pragma unroll
     for (int k = 0; k < EPT; ++k) {
-      const uint32_t f = tid + (uint32_t)k * kTNT;
-      bool ok = f < nvec;
-      if (RAG && !s.full) ok = ok && (rout[k] & 0xFFFFu) < s.rem0 && (rout[k] >> 16) < s.rem1;
-      if (ok) {
+      if (tid + (uint32_t)k * kTNT < nvec) {
         uint32_t base = st_ls[k];
         opaque(base);
         P o;
@@ -252,31 +245,274 @@ __global__ __launch_bounds__(kTNT) void k_permute_tiled(const W *__restrict__ in
           const uint32_t e = base + j * step;
           o.w[j] = conj_if<W, CONJ>(lds[e + fdiv(e, p.pad)]);
         }
-        st_stream(reinterpret_cast<P *>(out + (s.bout + out_off[k])), o);
+        st_stream(reinterpret_cast<P *>(out + (bout + out_off[k])), o);
       }
     }
   };
   uint32_t tile = blockIdx.x;
   if (tile >= p.ntiles) return;
-  TileBase cur;
-  decode(tile, cur);
-  load(cur);
+  OffT bin, bout;
+  decode(tile, bin, bout);
+  load(bin);
   // software pipeline: the next tile's loads are in flight while the current
   // tile drains from LDS to memory
   while (true) {
-    to_lds(cur);
+    to_lds();
     __syncthreads();
     const uint32_t next = tile + gridDim.x;
-    TileBase nxt;
+    const OffT cur = bout;
     if (next < p.ntiles) {
-      decode(next, nxt);
-      load(nxt);
+      decode(next, bin, bout);
+      load(bin);
     }
     from_lds(cur);
     if (next >= p.ntiles) break;
     __syncthreads();
     tile = next;
-    cur = nxt;
+  }
+}
+
+// ---------------------------------------------------------------------------
+// Permutation by runs: the form for tiles whose minor extents hold no whole
+// vectors (odd extents), for bodies aligned to an element only, and for D +=
+// f * L.
+//
+// A tile's contiguous run on each side may span several dimensions. A thread
+// takes vectors of VEC consecutive elements of a run, whatever the alignment
+// (global accesses need an element's only); a run's last vector starts early
+// enough to be whole, so it repeats elements of the one before. A dimension
+// that its tile extent does not divide is covered by tiles that overlap in
+// the same way. Copies write repeated elements twice, with the same value; in
+// the accumulating form the repeats are skipped. No access is masked, so a
+// thread's loads fly together: with one masked 4-byte access at a time, a
+// 31 M element R4 body of extents 37,29,41,23,31 took 130 us (1.9 TB/s).
+struct RunParams {
+  int nri, nro;                     // tile dimensions after the run, load / store order
+  uint32_t ri, ro;                  // run lengths (elements)
+  DevDiv nvi, nvo;                  // vectors per run
+  uint32_t vecs_i, vecs_o;          // vectors per tile
+  DevDiv t_in[kMaxTileDims];        // extents after the run, load order
+  uint64_t is_in[kMaxTileDims];
+  DevDiv t_run[kMaxTileDims];       // extents inside the output run
+  uint32_t ls_run[kMaxTileDims];    // their LDS strides
+  int nrun;
+  DevDiv t_out[kMaxTileDims];       // extents after the run, store order
+  uint64_t os_out[kMaxTileDims];
+  uint32_t ls_out[kMaxTileDims];
+  int g_out[kMaxTileDims];          // grid dimension of t_out[j]
+  int g_run;                        // grid dimension of the run's last dimension
+  uint32_t unit;                    // run elements per step of that dimension
+  int ng;
+  DevDiv gdiv[kMaxGridDims];        // tiles along each dimension, output order
+  uint64_t g_is[kMaxGridDims], g_os[kMaxGridDims];
+  uint32_t g_t[kMaxGridDims], g_last[kMaxGridDims];  // tile extent, start of the last tile
+  uint32_t ntiles;
+  DevDiv pad;                       // LDS slot = e + e / pad.d (pad.d = 0: no padding)
+};
+
+// Arithmetic view of a word for D += f * L (products and sums rounded
+// separately, as the element-wise kernels do).
+#pragma clang fp contract(off)
+template <int KIND>
+struct Acc1;
+template <>
+struct Acc1<R4> {
+  typedef uint32_t W;
+  __device__ __forceinline__ static W run(W d, W l, double fr, double)
+  {
+    const float t = __uint_as_float(l) * (float)fr;
+    return __float_as_uint(__uint_as_float(d) + t);
+  }
+};
+template <>
+struct Acc1<R8> {
+  typedef uint2 W;
+  __device__ __forceinline__ static W run(W d, W l, double fr, double)
+  {
+    const double t = __builtin_bit_cast(double, l) * fr;
+    return __builtin_bit_cast(uint2, __builtin_bit_cast(double, d) + t);
+  }
+};
+template <>
+struct Acc1<C4> {
+  typedef uint2 W;
+  __device__ __forceinline__ static W run(W d, W l, double fr, double fi)
+  {
+    const float re = __uint_as_float(l.x), im = __uint_as_float(l.y), f0 = (float)fr, f1 = (float)fi;
+    const float a = re * f0, b = im * f1, c = re * f1, e = im * f0;
+    const float tr = a - b, ti = c + e;
+    return make_uint2(__float_as_uint(__uint_as_float(d.x) + tr), __float_as_uint(__uint_as_float(d.y) + ti));
+  }
+};
+template <>
+struct Acc1<C8> {
+  typedef uint4 W;
+  struct D2 { double re, im; };
+  __device__ __forceinline__ static W run(W d, W l, double fr, double fi)
+  {
+    const D2 x = __builtin_bit_cast(D2, l), y = __builtin_bit_cast(D2, d);
+    const double a = x.re * fr, b = x.im * fi, c = x.re * fi, e = x.im * fr;
+    const double tr = a - b, ti = c + e;
+    return __builtin_bit_cast(uint4, D2{y.re + tr, y.im + ti});
+  }
+};
+// KIND 0: out[..] = conj?(in[..]); a data kind: out[..] += f * conj?(in[..]).
+template <typename W, int VEC, int EPT, bool CONJ, typename OffT, int KIND>
+__global__ __launch_bounds__(kTNT) void k_permute_runs(const W *__restrict__ in, W *__restrict__ out,
+                                                       const RunParams p, double fr, double fi)
+{
+  typedef Pack<W, VEC> P;
+  constexpr int NS = (VEC + 1) / 2;       // LDS slots of a vector, two to a register
+  extern __shared__ __align__(16) unsigned char lds_raw[];
+  W *lds = reinterpret_cast<W *>(lds_raw);
+  const uint32_t tid = threadIdx.x;
+  OffT in_off[EPT], out_off[EPT];
+  uint32_t lslot[EPT][NS], sslot[EPT][NS];
+  uint32_t skip[KIND ? EPT : 1];          // leading elements that repeat the vector before
+  uint32_t ocrd[KIND ? EPT : 1];          // position inside the run, for overlapping tiles
+#pragma unroll
+  for (int k = 0; k < EPT; ++k) {
+    {
+      const uint32_t v = min(tid + (uint32_t)k * kTNT, p.vecs_i - 1);
+      uint32_t q = fdiv(v, p.nvi);
+      const uint32_t s = min((v - q * p.nvi.d) * VEC, p.ri - VEC);
+#pragma unroll
+      for (int e = 0; e < VEC; ++e) {
+        const uint32_t sl = s + p.ri * q + e, slot = sl + fdiv(sl, p.pad);
+        if (e & 1) lslot[k][e / 2] |= slot << 16;
+        else lslot[k][e / 2] = slot;
+      }
+      OffT io = s;
+      for (int j = 0; j < p.nri; ++j) {
+        const uint32_t n = fdiv(q, p.t_in[j]);
+        io += (OffT)(q - n * p.t_in[j].d) * (OffT)p.is_in[j];
+        q = n;
+      }
+      in_off[k] = io;
+    }
+    const uint32_t v = min(tid + (uint32_t)k * kTNT, p.vecs_o - 1);
+    uint32_t q = fdiv(v, p.nvo);
+    const uint32_t s0 = (v - q * p.nvo.d) * VEC, s = min(s0, p.ro - VEC);
+    if (KIND) {
+      skip[k] = tid + (uint32_t)k * kTNT < p.vecs_o ? s0 - s : VEC;
+      ocrd[k] = v;
+    }
+    OffT oo = s;
+    uint32_t base = 0;
+    for (int j = 0; j < p.nro; ++j) {
+      const uint32_t n = fdiv(q, p.t_out[j]), c = q - n * p.t_out[j].d;
+      oo += (OffT)c * (OffT)p.os_out[j];
+      base += c * p.ls_out[j];
+      q = n;
+    }
+    out_off[k] = oo;
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) {
+      uint32_t r = s + e, sl = base;
+      for (int j = 0; j < p.nrun; ++j) {
+        const uint32_t n = fdiv(r, p.t_run[j]);
+        sl += (r - n * p.t_run[j].d) * p.ls_run[j];
+        r = n;
+      }
+      sl += fdiv(sl, p.pad);
+      if (e & 1) sslot[k][e / 2] |= sl << 16;
+      else sslot[k][e / 2] = sl;
+    }
+  }
+  // Place `at` of the grid-stride order -> tile: each XCD (workgroups go round
+  // robin over eight) takes a contiguous range, so that the tiles sharing a
+  // line meet in one L2 (1-3% over the plain order).
+  const uint32_t per_xcd = p.ntiles / 8;
+  auto tile_at = [&](uint32_t at) { return at < per_xcd * 8 ? at % 8 * per_xcd + at / 8 : at; };
+  // tile index -> start along each dimension (the last tile of a dimension
+  // ends at its end); lap: whether it repeats elements of the tile before
+  auto decode = [&](uint32_t place, OffT &bi, OffT &bo, bool &lap) {
+    bi = bo = 0;
+    lap = false;
+    uint32_t r = tile_at(place);
+    for (int g = 0; g < p.ng; ++g) {
+      const uint32_t q = fdiv(r, p.gdiv[g]), c = r - q * p.gdiv[g].d;
+      r = q;
+      const uint32_t at = min(c * p.g_t[g], p.g_last[g]);
+      lap = lap || at != c * p.g_t[g];
+      bi += (OffT)at * (OffT)p.g_is[g];
+      bo += (OffT)at * (OffT)p.g_os[g];
+    }
+  };
+  // elements of tile `tile` along grid dimension g that the tile before holds
+  auto lap_of = [&](uint32_t place, int g) {
+    uint32_t r = tile_at(place), c = 0;
+    for (int i = 0; i <= g; ++i) {
+      const uint32_t q = fdiv(r, p.gdiv[i]);
+      c = r - q * p.gdiv[i].d;
+      r = q;
+    }
+    return c * p.g_t[g] - min(c * p.g_t[g], p.g_last[g]);
+  };
+  uint32_t tile = blockIdx.x;
+  if (tile >= p.ntiles) return;
+  auto slot = [](const uint32_t (&x)[NS], int e) { return (e & 1) ? x[e / 2] >> 16 : x[e / 2] & 0xFFFFu; };
+  P val[EPT], d[KIND ? EPT : 1];
+  OffT bi, bo;
+  bool lap;
+  decode(tile, bi, bo, lap);
+  auto load = [&]() {
+#pragma unroll
+    for (int k = 0; k < EPT; ++k) val[k] = ld_run<P>(in + (bi + in_off[k]));
+  };
+  load();
+  while (true) {
+    // D before the next tile's loads: both are waited for in issue order
+    if constexpr (KIND != 0) {
+#pragma unroll
+      for (int k = 0; k < EPT; ++k) d[k] = ld_run<P>(out + (bo + out_off[k]));
+    }
+#pragma unroll
+    for (int k = 0; k < EPT; ++k)
+#pragma unroll
+      for (int e = 0; e < VEC; ++e) lds[slot(lslot[k], e)] = val[k].w[e];
+    __syncthreads();
+    const uint32_t next = tile + gridDim.x;
+    const OffT bo_cur = bo;
+    const bool lap_cur = lap;
+    if (next < p.ntiles) {
+      decode(next, bi, bo, lap);
+      load();
+    }
+#pragma unroll
+    for (int k = 0; k < EPT; ++k) {
+      P o;
+#pragma unroll
+      for (int e = 0; e < VEC; ++e) o.w[e] = conj_if<W, CONJ>(lds[slot(sslot[k], e)]);
+      W *dst = out + (bo_cur + out_off[k]);
+      if constexpr (KIND == 0) {
+        st_run<P>(dst, o);
+      } else {
+        uint32_t first = skip[k];
+        if (lap_cur && first < VEC) {  // elements that the tile before holds
+          uint32_t q = fdiv(ocrd[k], p.nvo);
+          const uint32_t s = min((ocrd[k] - q * p.nvo.d) * VEC, p.ro - VEC), run = lap_of(tile, p.g_run) * p.unit;
+          if (run > s) first = max(first, min(run - s, (uint32_t)VEC));
+          for (int j = 0; j < p.nro; ++j) {
+            const uint32_t n = fdiv(q, p.t_out[j]);
+            if (q - n * p.t_out[j].d < lap_of(tile, p.g_out[j])) first = VEC;
+            q = n;
+          }
+        }
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) o.w[e] = Acc1<KIND>::run(d[k].w[e], o.w[e], fr, fi);
+        if (first == 0) {
+          st_run<P>(dst, o);
+        } else {
+#pragma unroll
+          for (int e = 0; e < VEC; ++e)
+            if ((uint32_t)e >= first) dst[e] = o.w[e];
+        }
+      }
+    }
+    if (next >= p.ntiles) break;
+    __syncthreads();
+    tile = next;
   }
 }
 
@@ -521,15 +757,15 @@ DevDiv to_dev(uint32_t d)
 }
 
 struct Planned {
-  int path = 0;  // 0 copy, 1 tiled, 2 scatter
+  int path = 0;  // 0 copy, 1 tiled, 2 scatter, 3 tiled by runs
   Fused f;
   TileParams tp{};
+  RunParams rp{};
   int ept = 0;
   size_t lds_bytes = 0;
   int grid = 0;
   int vec = 1;        // elements per global access
   bool wide = false;  // 64-bit element offsets
-  bool rag = false;   // masked edge tiles
   int cus = 0;        // compute units the grid was sized for
   TilePlan tile;
 };
@@ -562,7 +798,163 @@ int tile_vec(const Fused &f, const TilePlan &tp, int es)
   return 1;
 }
 
-int plan(int es, int rank, const int *dims, const int *o2n, Planned &pl, int cus, bool choose_pad = true)
+// Tile of the run form: an input-minor and an output-minor group of
+// dimensions, each walked until it covers `target` elements; a dimension that
+// is cut gets tiles of nearly equal extent (the last one overlaps its
+// neighbour by less than the number of tiles).
+int balanced(int ext, long need)
+{
+  if (need >= ext) return ext;
+  const int n = std::max<int>(1, (int)(ext / need));  // tiles of at least `need`
+  return (ext + n - 1) / n;
+}
+
+bool plan_runs(int es, const Fused &f, int cus, int vec, int max_ept, Planned &pl)
+{
+  const int r = f.rank;
+  std::vector<int> n2o(r);
+  for (int i = 0; i < r; ++i) n2o[f.o2n[i]] = i;
+  uint64_t vol = 1;
+  for (int e : f.ext) vol *= (uint64_t)e;
+  const long max_vol = std::min<long>((long)kTNT * max_ept * vec, kTileMaxBytes / es);
+  const long min_vol =
+      std::min<long>({max_vol, kTileMinVol, std::max<long>(1024, (long)(vol / (4 * (uint64_t)std::max(cus, 1))))});
+  std::vector<int> t(r);
+  auto volume = [&] {
+    long v = 1;
+    for (int x : t) v *= std::max(x, 1);
+    return v;
+  };
+  auto walk = [&](long target, bool in) {
+    long run = 1;
+    for (int q = 0; q < r; ++q) {
+      const int i = in ? q : n2o[q];
+      const int want = balanced(f.ext[i], (target + run - 1) / run);
+      t[i] = std::max(t[i], want);
+      run *= t[i];
+      if (t[i] < f.ext[i] || run >= target) break;
+    }
+  };
+  auto try_target = [&](long target) {
+    std::fill(t.begin(), t.end(), 0);
+    walk(target, true);
+    walk(target, false);
+    return volume() <= max_vol && std::count_if(t.begin(), t.end(), [](int x) { return x > 0; }) <= kMaxTileDims;
+  };
+  // (tiles of at most a sixth of a CU's share: a 31 MB body in 1.5 tiles per
+  // resident workgroup took 48 us, in 6 smaller ones 30)
+  const long share = std::max<long>(2048, (long)(vol / (6 * (uint64_t)std::max(cus, 1))));
+  long target = std::max(8, 512 / es);
+  while (target > 1 && (!try_target(target) || (volume() > share && target * es > kLine))) target /= 2;
+  if (!try_target(target)) return false;
+  // grow towards min_vol, alternating sides
+  for (int side = 0, stuck = 0; volume() < min_vol && stuck < 2; side ^= 1) {
+    int dim = -1;
+    for (int q = 0; q < r && dim < 0; ++q) {
+      const int i = side == 0 ? q : n2o[q];
+      if (t[i] < f.ext[i]) dim = i;
+    }
+    if (dim < 0) { ++stuck; continue; }
+    const int old = t[dim], want = balanced(f.ext[dim], std::max(2l, 2l * old));
+    if (volume() / std::max(old, 1) * want > std::min(max_vol, share)) { ++stuck; continue; }
+    if (old == 0 && std::count_if(t.begin(), t.end(), [](int x) { return x > 0; }) == kMaxTileDims) { ++stuck; continue; }
+    stuck = 0;
+    t[dim] = want;
+  }
+  RunParams &P = pl.rp;
+  std::memset(&P, 0, sizeof(P));
+  std::vector<uint64_t> istr(r), ostr(r);
+  uint64_t st = 1;
+  for (int i = 0; i < r; ++i) { istr[i] = st; st *= (uint64_t)f.ext[i]; }
+  st = 1;
+  for (int q = 0; q < r; ++q) { ostr[n2o[q]] = st; st *= (uint64_t)f.ext[n2o[q]]; }
+  std::vector<uint32_t> ls(r, 0);
+  uint32_t lv = 1;
+  for (int i = 0; i < r; ++i)
+    if (t[i] > 0) { ls[i] = lv; lv *= (uint32_t)t[i]; }
+  // run prefixes
+  P.ri = P.ro = 1;
+  bool run = true;
+  for (int i = 0; i < r; ++i) {
+    if (run && t[i] > 0) P.ri *= (uint32_t)t[i];
+    else if (t[i] > 0) {
+      P.t_in[P.nri] = to_dev((uint32_t)t[i]);
+      P.is_in[P.nri++] = istr[i];
+    }
+    if (t[i] < f.ext[i]) run = false;
+  }
+  run = true;
+  P.unit = 1;
+  for (int q = 0; q < r; ++q) {
+    const int i = n2o[q];
+    if (run && t[i] > 0) {
+      P.unit = P.ro;
+      P.ro *= (uint32_t)t[i];
+      P.t_run[P.nrun] = to_dev((uint32_t)t[i]);
+      P.ls_run[P.nrun++] = ls[i];
+      P.g_run = q;
+    } else if (t[i] > 0) {
+      P.t_out[P.nro] = to_dev((uint32_t)t[i]);
+      P.os_out[P.nro] = ostr[i];
+      P.ls_out[P.nro] = ls[i];
+      P.g_out[P.nro++] = q;
+    }
+    if (t[i] < f.ext[i]) run = false;
+  }
+  if (P.ri < (uint32_t)vec || P.ro < (uint32_t)vec) return false;
+  const uint32_t tv = lv;
+  P.nvi = to_dev((P.ri + vec - 1) / vec);
+  P.nvo = to_dev((P.ro + vec - 1) / vec);
+  P.vecs_i = P.nvi.d * (tv / P.ri);
+  P.vecs_o = P.nvo.d * (tv / P.ro);
+  uint64_t ntiles = 1;
+  P.ng = r;
+  for (int q = 0; q < r; ++q) {  // output order (see plan)
+    const int i = n2o[q], ti = std::max(t[i], 1), n = (f.ext[i] + ti - 1) / ti;
+    P.gdiv[q] = to_dev((uint32_t)n);
+    P.g_is[q] = istr[i];
+    P.g_os[q] = ostr[i];
+    P.g_t[q] = (uint32_t)ti;
+    P.g_last[q] = (uint32_t)(f.ext[i] - ti);
+    ntiles *= (uint64_t)n;
+  }
+  if (ntiles >= (1ull << 31)) return false;
+  P.ntiles = (uint32_t)ntiles;
+  // LDS padding: simulated bank conflicts of the first vectors' store-phase reads
+  std::vector<uint32_t> slots;
+  for (uint32_t v = 0; v < std::min<uint32_t>(P.vecs_o, kTNT); ++v) {
+    uint32_t q = v / P.nvo.d, s = std::min((v % P.nvo.d) * (uint32_t)vec, P.ro - (uint32_t)vec), l = 0;
+    for (int j = 0; j < P.nro; ++j) { l += q % P.t_out[j].d * P.ls_out[j]; q /= P.t_out[j].d; }
+    for (int j = 0; j < P.nrun; ++j) { l += s % P.t_run[j].d * P.ls_run[j]; s /= P.t_run[j].d; }
+    slots.push_back(l);
+  }
+  const int words = std::max(1, es / 4);
+  std::vector<uint32_t> cands = {4, 8, 16, 32, 64, 128, 256, P.ri};
+  uint32_t best = 0;
+  int bestc = conflict_cost(slots, words, 0);
+  for (uint32_t c : cands) {
+    if (c < 4 || c >= tv) continue;
+    const int cc = conflict_cost(slots, words, c);
+    if (cc < bestc) { bestc = cc; best = c; }
+  }
+  P.pad = to_dev(best);
+  const uint32_t nv = std::max(P.vecs_i, P.vecs_o);
+  int ept = 1;
+  while ((uint32_t)ept * kTNT < nv) ept *= 2;
+  if (ept > max_ept) return false;
+  pl.ept = ept;
+  pl.vec = vec;
+  pl.wide = vol >= (1ull << 32);
+  pl.lds_bytes = (tv + (best ? tv / best + 1 : 0)) * (size_t)es;
+  pl.cus = cus;
+  const int per_cu = std::max(1, std::min(kTiledPerCU, (int)(160 * 1024 / std::max<size_t>(pl.lds_bytes, 1))));
+  pl.grid = (int)std::min<uint64_t>(ntiles, (uint64_t)cus * per_cu);
+  pl.path = 3;
+  return true;
+}
+
+// align: bytes that both bodies are aligned to (at most 16).
+int plan(int es, int rank, const int *dims, const int *o2n, Planned &pl, int cus, int align, bool choose_pad = true)
 {
   pl.f = fuse_dims(rank, dims, o2n);
   const Fused &f = pl.f;
@@ -607,8 +999,15 @@ int plan(int es, int rank, const int *dims, const int *o2n, Planned &pl, int cus
   }
   uint64_t ntiles = 1;
   for (int i = 0; i < f.rank; ++i) ntiles *= (uint64_t)((f.ext[i] + std::max(tp.t[i], 1) - 1) / std::max(tp.t[i], 1));
-  if (!ok || ntd > kMaxTileDims || nrag > 2 || ntiles >= (1ull << 31)) {
-    pl.path = 2;
+  // The vector form takes tiles that divide the tensor, with 16-byte vectors
+  // along both minor dimensions and runs of whole cache lines on both sides;
+  // everything else goes by runs (shapes of either kind that could go both
+  // ways: within 1% on 60 random ones)
+  const bool tiled = ok && ntd <= kMaxTileDims && nrag == 0 && ntiles < (1ull << 31) && align >= 16 &&
+                     tile_vec(f, tp, es) * es == 16 && (long)tp.in_run * es % kLine == 0 &&
+                     (long)tp.out_run * es % kLine == 0;
+  if (!tiled) {
+    pl.path = plan_runs(es, f, cus, 16 / es, kMaxEPT, pl) ? 3 : 2;
     return 0;
   }
   pl.path = 1;
@@ -644,17 +1043,6 @@ int plan(int es, int rank, const int *dims, const int *o2n, Planned &pl, int cus
     P.os_out[j] = ostr[tout[j]];
     P.ls_out[j] = lstride[tout[j]];
   }
-  P.nrag = 0;
-  for (int j = 0; j < P.nt; ++j) {
-    const int i = tin[j];
-    if (f.ext[i] % tp.t[i] != 0) {
-      const int slot = P.nrag++;
-      P.rag_in[slot] = j;
-      P.rag_t[slot] = (uint32_t)tp.t[i];
-      for (int jj = 0; jj < P.nt; ++jj)
-        if (tout[jj] == i) P.rag_out[slot] = jj;
-    }
-  }
   // grid: tile index decoded fastest along the output's minor dimension, then
   // in output order, so that the tiles in flight at once (consecutive indices
   // across the persistent grid) write neighbouring regions of the output.
@@ -668,11 +1056,6 @@ int plan(int es, int rank, const int *dims, const int *o2n, Planned &pl, int cus
     P.gdiv[q] = to_dev(n);
     P.g_is[q] = istr[i] * t;
     P.g_os[q] = ostr[i] * t;
-    P.g_t[q] = t;
-    P.g_ext[q] = (uint32_t)f.ext[i];
-    P.g_rag[q] = -1;
-    for (int k = 0; k < P.nrag; ++k)
-      if (tin[P.rag_in[k]] == i) P.g_rag[q] = k;
   }
   P.vol_tile = (uint32_t)tp.vol;
   P.ntiles = (uint32_t)ntiles;
@@ -699,13 +1082,11 @@ int plan(int es, int rank, const int *dims, const int *o2n, Planned &pl, int cus
     if (cc < bestc) { bestc = cc; best = c; }
   }
   P.pad = to_dev(best);
-  // vector width: both minor dimensions (input dim 0, output dim 0) and their
-  // tile extents must be multiples of it so every vector is aligned and whole
-  int vec = tile_vec(f, tp, es);
+  const int vec = 16 / es;
   // the kernel writes one vector to consecutive LDS slots, so a vector must
-  // not straddle a padding period (every candidate period above is a
-  // multiple of the width already; this keeps that invariant explicit)
-  while (vec > 1 && best % (uint32_t)vec != 0) vec /= 2;
+  // not straddle a padding period
+  if (best % (uint32_t)vec != 0) best = 0;
+  P.pad = to_dev(best);
   pl.vec = vec;
   P.tv_in0 = to_dev((uint32_t)(tp.t[tin[0]] / vec));
   P.tv_out0 = to_dev((uint32_t)(tp.t[tout[0]] / vec));
@@ -713,7 +1094,6 @@ int plan(int es, int rank, const int *dims, const int *o2n, Planned &pl, int cus
   while ((long)ept * kTNT * vec < tp.vol) ept *= 2;
   pl.ept = ept;
   pl.wide = vol >= (1ull << 32);
-  pl.rag = P.nrag > 0;
   const size_t slots = P.vol_tile + (best ? P.vol_tile / best + 1 : 0);
   pl.lds_bytes = slots * (size_t)es;
   // resident workgroups per CU: measured on the transpose workload, 16 waves
@@ -728,12 +1108,12 @@ int plan(int es, int rank, const int *dims, const int *o2n, Planned &pl, int cus
 // Workgroups of one kernel instantiation that a CU holds at once as far as its
 // registers allow (LDS is accounted for by the planner); the persistent grid
 // is capped at this so that every workgroup is resident from the start.
-template <typename W, int VEC, int EPT, bool CONJ, typename OffT, bool RAG>
+template <typename W, int VEC, int EPT, bool CONJ, typename OffT>
 int resident_per_cu()
 {
   static const int n = [] {
     int b = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, k_permute_tiled<W, VEC, EPT, CONJ, OffT, RAG>, kTNT, 0) !=
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, k_permute_tiled<W, VEC, EPT, CONJ, OffT>, kTNT, 0) !=
             hipSuccess || b <= 0)
       b = 1;
     return b;
@@ -741,18 +1121,18 @@ int resident_per_cu()
   return n;
 }
 
-template <typename W, int VEC, bool CONJ, typename OffT, bool RAG>
-int launch_tiled_v(const Planned &pl, const void *in, void *out, hipStream_t s)
+template <typename W, bool CONJ, typename OffT>
+int launch_tiled_o(const Planned &pl, const void *in, void *out, hipStream_t s)
 {
+  constexpr int VEC = 16 / (int)sizeof(W);
   const W *a = static_cast<const W *>(in);
   W *b = static_cast<W *>(out);
-  const dim3 blk(kTNT);
   switch (pl.ept) {
 #define XT_CASE(E)                                                                                             \
   case E: {                                                                                                    \
-    const int cap = pl.cus * resident_per_cu<W, VEC, E, CONJ, OffT, RAG>();                                    \
+    const int cap = pl.cus * resident_per_cu<W, VEC, E, CONJ, OffT>();                                         \
     const dim3 g(std::min(pl.grid, cap));                                                                      \
-    hipLaunchKernelGGL((k_permute_tiled<W, VEC, E, CONJ, OffT, RAG>), g, blk, pl.lds_bytes, s, a, b, pl.tp);   \
+    hipLaunchKernelGGL((k_permute_tiled<W, VEC, E, CONJ, OffT>), g, dim3(kTNT), pl.lds_bytes, s, a, b, pl.tp); \
     break;                                                                                                     \
   }
     XT_CASE(1) XT_CASE(2) XT_CASE(4) XT_CASE(8)
@@ -762,26 +1142,44 @@ int launch_tiled_v(const Planned &pl, const void *in, void *out, hipStream_t s)
   return XT_HIP_OK(hipGetLastError()) ? 0 : TALSH_FAILURE;
 }
 
-template <typename W, int VEC, bool CONJ>
-int launch_tiled_w(const Planned &pl, const void *in, void *out, hipStream_t s)
-{
-  if (pl.wide) return pl.rag ? launch_tiled_v<W, VEC, CONJ, uint64_t, true>(pl, in, out, s)
-                             : launch_tiled_v<W, VEC, CONJ, uint64_t, false>(pl, in, out, s);
-  return pl.rag ? launch_tiled_v<W, VEC, CONJ, uint32_t, true>(pl, in, out, s)
-                : launch_tiled_v<W, VEC, CONJ, uint32_t, false>(pl, in, out, s);
-}
-
 template <typename W, bool CONJ>
 int launch_tiled_t(const Planned &pl, const void *in, void *out, hipStream_t s)
 {
-  // only vector widths that keep one access <= 16 bytes are instantiated
-  if constexpr (sizeof(W) == 4) {
-    if (pl.vec == 4) return launch_tiled_w<W, 4, CONJ>(pl, in, out, s);
-    if (pl.vec == 2) return launch_tiled_w<W, 2, CONJ>(pl, in, out, s);
-  } else if constexpr (sizeof(W) == 8) {
-    if (pl.vec == 2) return launch_tiled_w<W, 2, CONJ>(pl, in, out, s);
+  return pl.wide ? launch_tiled_o<W, CONJ, uint64_t>(pl, in, out, s) : launch_tiled_o<W, CONJ, uint32_t>(pl, in, out, s);
+}
+
+// Launches the run form (KIND 0: copy; a data kind: accumulate f times the
+// permuted input).
+template <typename W, bool CONJ, int KIND, typename OffT>
+int launch_runs_o(const Planned &pl, const void *in, void *out, double fr, double fi, hipStream_t s)
+{
+  constexpr int VEC = 16 / (int)sizeof(W);
+  const W *a = static_cast<const W *>(in);
+  W *b = static_cast<W *>(out);
+  switch (pl.ept) {
+#define XT_CASE(E)                                                                                              \
+  case E:                                                                                                       \
+    hipLaunchKernelGGL((k_permute_runs<W, VEC, E, CONJ, OffT, KIND>), dim3(pl.grid), dim3(kTNT), pl.lds_bytes, s, \
+                       a, b, pl.rp, fr, fi);                                                                    \
+    break;
+    XT_CASE(1) XT_CASE(2) XT_CASE(4)
+  case 8:
+    if constexpr (KIND == 0) {
+      hipLaunchKernelGGL((k_permute_runs<W, VEC, 8, CONJ, OffT, 0>), dim3(pl.grid), dim3(kTNT), pl.lds_bytes, s, a, b,
+                         pl.rp, fr, fi);
+      break;
+    }
+    return TALSH_FAILURE;
+#undef XT_CASE
+  default: return TALSH_FAILURE;
   }
-  return launch_tiled_w<W, 1, CONJ>(pl, in, out, s);
+  return XT_HIP_OK(hipGetLastError()) ? 0 : TALSH_FAILURE;
+}
+template <typename W, bool CONJ, int KIND>
+int launch_runs(const Planned &pl, const void *in, void *out, double fr, double fi, hipStream_t s)
+{
+  return pl.wide ? launch_runs_o<W, CONJ, KIND, uint64_t>(pl, in, out, fr, fi, s)
+                 : launch_runs_o<W, CONJ, KIND, uint32_t>(pl, in, out, fr, fi, s);
 }
 
 template <typename W, bool CONJ>
@@ -833,7 +1231,56 @@ int dispatch(const Planned &pl, const void *in, void *out, uint64_t vol, hipStre
 {
   if (pl.path == 0) return launch_copy_t<W, CONJ>(in, out, vol, s, cus);
   if (pl.path == 1) return launch_tiled_t<W, CONJ>(pl, in, out, s);
+  if (pl.path == 3) return launch_runs<W, CONJ, 0>(pl, in, out, 0.0, 0.0, s);
   return launch_scatter_t<W, CONJ>(pl.f, in, out, s, cus);
+}
+
+int compute_units()
+{
+  static const int cus = num_cus_current();
+  return cus;
+}
+
+// The plan of a permutation (add: of its accumulating form, path 3 or none).
+// Plans are memoized per (form, element size, alignment, extents,
+// permutation): planning (fusion, tile choice, bank-conflict simulation) costs
+// far more host time than a launch.
+Planned planned(int es, int rank, const int *dims, const int *o2n, const void *in, const void *out, bool add)
+{
+  static std::mutex mu;
+  static std::unordered_map<std::string, Planned> cache;
+  const uintptr_t addr = (uintptr_t)in | (uintptr_t)out;
+  const int align = add || addr % 16 == 0 ? 16 : addr % 8 == 0 ? 8 : 4;
+  std::string key;
+  key.reserve(8 * rank + 8);
+  key.append(std::to_string(add ? -es : es)).push_back('@');
+  key.append(std::to_string(align)).push_back(':');
+  for (int i = 0; i < rank; ++i) key.append(std::to_string(dims[i])).append(",").append(std::to_string(o2n[i])).push_back(';');
+  std::lock_guard<std::mutex> g(mu);
+  auto it = cache.find(key);
+  if (it != cache.end()) return it->second;
+  Planned pl;
+  if (add) {
+    pl.f = fuse_dims(rank, dims, o2n);
+    // (half the vectors per thread: the accumulating form holds D's as well)
+    if (pl.f.rank < 2 || pl.f.rank > kMaxGridDims || !plan_runs(es, pl.f, compute_units(), 16 / es, kMaxEPT / 2, pl))
+      pl.path = 2;
+  } else {
+    plan(es, rank, dims, o2n, pl, compute_units(), align);
+  }
+  if (cache.size() >= 4096) cache.clear();
+  cache.emplace(key, pl);
+  return pl;
+}
+
+bool valid_permutation(int rank, const int *dims, const int *o2n)
+{
+  std::vector<int> seen(std::max(rank, 1), 0);
+  for (int i = 0; i < rank; ++i) {
+    if (dims[i] <= 0 || o2n[i] < 0 || o2n[i] >= rank || seen[o2n[i]]) return false;
+    seen[o2n[i]] = 1;
+  }
+  return true;
 }
 
 }  // namespace
@@ -843,8 +1290,17 @@ int plan_permute_info(int kind, int rank, const int *dims_in, const int *o2n, Pe
   const int es = kind_size(kind);
   if (es == 0 || rank < 0 || rank > kMaxRank) return TALSH_INVALID_ARGS;
   Planned pl;
-  plan(es, rank, dims_in, o2n, pl, 256, with_padding);
+  plan(es, rank, dims_in, o2n, pl, 256, 16, with_padding);
   info->fused_rank = pl.f.rank;
+  if (pl.path == 3) {
+    info->path = 1;
+    info->tile_volume = (int)(pl.rp.ri * (pl.rp.vecs_i / pl.rp.nvi.d));
+    info->in_run = (int)pl.rp.ri;
+    info->out_run = (int)pl.rp.ro;
+    info->grid = pl.grid;
+    info->vec = pl.vec;
+    return 0;
+  }
   info->path = pl.path;
   info->tile_volume = pl.path == 1 ? (int)pl.tile.vol : 0;
   info->in_run = pl.path == 1 ? pl.tile.in_run : 0;
@@ -859,51 +1315,16 @@ int launch_permute(const void *in, void *out, int kind, int rank, const int *dim
 {
   const int es = kind_size(kind);
   if (es == 0 || rank < 0 || rank > kMaxRank) return TALSH_INVALID_ARGS;
-  std::vector<int> seen(rank, 0);
+  if (!valid_permutation(rank, dims_in, o2n)) return TALSH_INVALID_ARGS;
   uint64_t vol = 1;
-  for (int i = 0; i < rank; ++i) {
-    if (dims_in[i] <= 0 || o2n[i] < 0 || o2n[i] >= rank || seen[o2n[i]]) return TALSH_INVALID_ARGS;
-    seen[o2n[i]] = 1;
-    vol *= (uint64_t)dims_in[i];
-  }
+  for (int i = 0; i < rank; ++i) vol *= (uint64_t)dims_in[i];
   if (vol == 0) return 0;
   if (in == out) return TALSH_INVALID_ARGS;  // out-of-place only
-  static int cus = num_cus_current();
-  Planned pl;
-  {
-    // plans are memoized per (element size, extents, permutation): planning
-    // (fusion, tile choice, bank-conflict simulation) costs far more host time
-    // than a launch
-    static std::mutex mu;
-    static std::unordered_map<std::string, Planned> cache;
-    std::string key;
-    key.reserve(8 * rank + 8);
-    key.append(std::to_string(es)).push_back(':');
-    for (int i = 0; i < rank; ++i) key.append(std::to_string(dims_in[i])).append(",").append(std::to_string(o2n[i])).push_back(';');
-    std::lock_guard<std::mutex> g(mu);
-    auto it = cache.find(key);
-    if (it != cache.end()) {
-      pl = it->second;
-    } else {
-      plan(es, rank, dims_in, o2n, pl, cus);
-      if (cache.size() >= 4096) cache.clear();
-      cache.emplace(key, pl);
-    }
-  }
-  if (pl.path == 1) {
-    // vector accesses need both bodies aligned to the vector size
-    if (pl.vec > 1 && (((uintptr_t)in | (uintptr_t)out) % (uintptr_t)(pl.vec * es)) != 0) {
-      pl.tp.tv_in0 = to_dev(pl.tp.t_in[0].d);
-      pl.tp.tv_out0 = to_dev(pl.tp.t_out[0].d);
-      pl.vec = 1;
-      pl.ept = 1;
-      while ((long)pl.ept * kTNT < (long)pl.tp.vol_tile) pl.ept *= 2;
-      if (pl.ept > kMaxEPT) pl.path = 2;  // one element per access: too many per thread for the tiled kernel
-    }
-    // the persistent grid and per-thread vector slots must cover the tile
-    if (pl.path == 1 && ((long)pl.ept * kTNT * pl.vec < (long)pl.tp.vol_tile || pl.grid <= 0 || pl.ept > kMaxEPT))
-      return TALSH_FAILURE;
-  }
+  const Planned pl = planned(es, rank, dims_in, o2n, in, out, false);
+  // the persistent grid and the per-thread vector slots must cover the tile
+  if (pl.path == 1 && ((long)pl.ept * kTNT * pl.vec < (long)pl.tp.vol_tile || pl.grid <= 0 || pl.ept > kMaxEPT))
+    return TALSH_FAILURE;
+  const int cus = compute_units();
   const bool cj = conj && kind_complex(kind);
   hipEvent_t pr[2];
   prof_begin(s, kKTranspose, pr);  // timing brackets the launch only
@@ -917,6 +1338,28 @@ int launch_permute(const void *in, void *out, int kind, int rank, const int *dim
   }
   prof_end(s, kKTranspose, pr);
   return e;
+}
+
+bool permute_add_planned(int kind, int rank, const int *dims_in, const int *o2n)
+{
+  const int es = kind_size(kind);
+  if (es == 0 || rank < 0 || rank > kMaxRank || !valid_permutation(rank, dims_in, o2n)) return false;
+  return planned(es, rank, dims_in, o2n, nullptr, nullptr, true).path == 3;
+}
+
+int launch_permute_add(const void *in, void *out, int kind, int rank, const int *dims_in, const int *o2n, bool conj,
+                       double re, double im, hipStream_t s)
+{
+  if (in == out || !permute_add_planned(kind, rank, dims_in, o2n)) return TALSH_INVALID_ARGS;
+  const Planned pl = planned(kind_size(kind), rank, dims_in, o2n, in, out, true);
+  const double f = real_factor(re, im);
+  switch (kind) {
+  case R4: return launch_runs<uint32_t, false, R4>(pl, in, out, f, 0.0, s);
+  case R8: return launch_runs<uint2, false, R8>(pl, in, out, f, 0.0, s);
+  case C4: return conj ? launch_runs<uint2, true, C4>(pl, in, out, re, im, s) : launch_runs<uint2, false, C4>(pl, in, out, re, im, s);
+  case C8: return conj ? launch_runs<uint4, true, C8>(pl, in, out, re, im, s) : launch_runs<uint4, false, C8>(pl, in, out, re, im, s);
+  default: return TALSH_INVALID_ARGS;
+  }
 }
 
 }  // namespace xt

@@ -14,6 +14,18 @@ namespace xt {
 int launch_permute(const void *in, void *out, int kind, int rank, const int *dims_in, const int *o2n, bool conj,
                    hipStream_t s);
 
+// out[idx'] += f * (conj?) in[idx] under the same index map, f = re + i im (real
+// kinds: real_factor(re, im)); products and sums rounded separately, as
+// launch_axpy does. permute_add_planned: whether this form exists for the
+// shape (else permute into a temporary and add).
+bool permute_add_planned(int kind, int rank, const int *dims_in, const int *o2n);
+int launch_permute_add(const void *in, void *out, int kind, int rank, const int *dims_in, const int *o2n, bool conj,
+                       double re, double im, hipStream_t s);
+// Real approximant of a complex factor for real data kinds: modulus with the
+// sign of the real part, or the imaginary part when the real part is zero
+// (the CPU path's rule, TALSH/tensor_algebra_cpu.F90:430-445).
+double real_factor(double re, double im);
+
 // Transpose plan summary for diagnostics and the plan selector.
 struct PermuteInfo {
   int fused_rank;       // rank after dropping unit extents and fusing runs
