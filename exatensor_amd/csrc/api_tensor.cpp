@@ -258,13 +258,17 @@ hipStream_t image_last_stream(void *img)
   return it == g_last_use.end() ? nullptr : it->second.s;
 }
 
-void images_touch(hipStream_t s, void *const *imgs, int n)
+void images_touch(hipStream_t s, void *const *imgs, int n, hipEvent_t own)
 {
-  if (n <= 0) return;
-  hipEvent_t ev = event_get(false);
-  if (!ev) return;
-  (void)hipEventRecord(ev, s);
+  hipEvent_t ev = own;
+  if (!ev) {
+    if (n <= 0) return;
+    ev = event_get(false);
+    if (!ev) return;
+    (void)hipEventRecord(ev, s);
+  }
   std::lock_guard<std::mutex> g(g_sync_mu);
+  if (own) ++g_ev_refs[own];  // the caller's, until event_unshare
   for (int i = 0; i < n; ++i) {
     auto it = g_last_use.find(imgs[i]);
     if (it != g_last_use.end()) {
@@ -280,6 +284,12 @@ void images_touch(hipStream_t s, void *const *imgs, int n)
 }
 
 void image_touch(hipStream_t s, void *img) { images_touch(s, &img, 1); }
+
+void event_unshare(hipEvent_t ev)
+{
+  std::lock_guard<std::mutex> g(g_sync_mu);
+  ev_unref(ev);
+}
 
 void image_forget_all()
 {

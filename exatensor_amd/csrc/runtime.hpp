@@ -72,6 +72,7 @@ struct Task {
   bool timed = true;  // start/input/output/GEMM events recorded (a blocking call's task records only its finish)
   int status = TALSH_TASK_EMPTY;
   bool finalized = false;
+  bool shared_finish = false;          // ev_finish also stands for the last use of the task's images
   std::vector<PendingFree> frees;      // temporaries released at completion
   // coherence actions applied at completion, one entry per argument; images
   // are identified by their body pointers (indices shift as images come and go)

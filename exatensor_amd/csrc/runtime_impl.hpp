@@ -19,8 +19,11 @@ size_t tensor_volume(const talsh_tens_t *t);
 void image_wait(hipStream_t s, void *img);
 void image_touch(hipStream_t s, void *img);
 // One event recorded on s after the current work, as the last use of every
-// listed image.
-void images_touch(hipStream_t s, void *const *imgs, int n);
+// listed image: own (a non-timing event that the caller has just recorded
+// there and gives back with event_unshare), else one of the pool's. Every
+// recorded event costs the call and the stream a few microseconds.
+void images_touch(hipStream_t s, void *const *imgs, int n, hipEvent_t own = nullptr);
+void event_unshare(hipEvent_t ev);
 // Stream of the last recorded use of an image (nullptr if none).
 hipStream_t image_last_stream(void *img);
 int prof_collect(int id, double *total_ms, long long *count);
