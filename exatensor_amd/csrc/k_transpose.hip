@@ -809,7 +809,7 @@ int balanced(int ext, long need)
   return (ext + n - 1) / n;
 }
 
-bool plan_runs(int es, const Fused &f, int cus, int vec, int max_ept, Planned &pl)
+bool plan_runs(int es, const Fused &f, int cus, int vec, int max_ept, Planned &pl, bool choose_pad)
 {
   const int r = f.rank;
   std::vector<int> n2o(r);
@@ -920,9 +920,10 @@ bool plan_runs(int es, const Fused &f, int cus, int vec, int max_ept, Planned &p
   }
   if (ntiles >= (1ull << 31)) return false;
   P.ntiles = (uint32_t)ntiles;
-  // LDS padding: simulated bank conflicts of the first vectors' store-phase reads
+  // LDS padding: simulated bank conflicts of the first vectors' store-phase
+  // reads (a millisecond or so per plan: not for a plan that is only described)
   std::vector<uint32_t> slots;
-  for (uint32_t v = 0; v < std::min<uint32_t>(P.vecs_o, kTNT); ++v) {
+  for (uint32_t v = 0; choose_pad && v < std::min<uint32_t>(P.vecs_o, kTNT); ++v) {
     uint32_t q = v / P.nvo.d, s = std::min((v % P.nvo.d) * (uint32_t)vec, P.ro - (uint32_t)vec), l = 0;
     for (int j = 0; j < P.nro; ++j) { l += q % P.t_out[j].d * P.ls_out[j]; q /= P.t_out[j].d; }
     for (int j = 0; j < P.nrun; ++j) { l += s % P.t_run[j].d * P.ls_run[j]; s /= P.t_run[j].d; }
@@ -931,9 +932,9 @@ bool plan_runs(int es, const Fused &f, int cus, int vec, int max_ept, Planned &p
   const int words = std::max(1, es / 4);
   std::vector<uint32_t> cands = {4, 8, 16, 32, 64, 128, 256, P.ri};
   uint32_t best = 0;
-  int bestc = conflict_cost(slots, words, 0);
+  int bestc = choose_pad ? conflict_cost(slots, words, 0) : 0;
   for (uint32_t c : cands) {
-    if (c < 4 || c >= tv) continue;
+    if (!choose_pad || c < 4 || c >= tv) continue;
     const int cc = conflict_cost(slots, words, c);
     if (cc < bestc) { bestc = cc; best = c; }
   }
@@ -1007,7 +1008,7 @@ int plan(int es, int rank, const int *dims, const int *o2n, Planned &pl, int cus
                      tile_vec(f, tp, es) * es == 16 && (long)tp.in_run * es % kLine == 0 &&
                      (long)tp.out_run * es % kLine == 0;
   if (!tiled) {
-    pl.path = plan_runs(es, f, cus, 16 / es, kMaxEPT, pl) ? 3 : 2;
+    pl.path = plan_runs(es, f, cus, 16 / es, kMaxEPT, pl, choose_pad) ? 3 : 2;
     return 0;
   }
   pl.path = 1;
@@ -1263,7 +1264,7 @@ Planned planned(int es, int rank, const int *dims, const int *o2n, const void *i
   if (add) {
     pl.f = fuse_dims(rank, dims, o2n);
     // (half the vectors per thread: the accumulating form holds D's as well)
-    if (pl.f.rank < 2 || pl.f.rank > kMaxGridDims || !plan_runs(es, pl.f, compute_units(), 16 / es, kMaxEPT / 2, pl))
+    if (pl.f.rank < 2 || pl.f.rank > kMaxGridDims || !plan_runs(es, pl.f, compute_units(), 16 / es, kMaxEPT / 2, pl, true))
       pl.path = 2;
   } else {
     plan(es, rank, dims, o2n, pl, compute_units(), align);
