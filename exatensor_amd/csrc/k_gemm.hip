@@ -447,6 +447,104 @@ __global__ __launch_bounds__(256) void k_realify(const T *__restrict__ x, int64_
   }
 }
 
+// Element offset of index i of a group of at most kSmallDims dimensions.
+__device__ __forceinline__ int64_t group_at(const DevGroup<kSmallDims> &g, int i)
+{
+  uint32_t r = (uint32_t)i;
+  int64_t o = 0;
+#pragma unroll
+  for (int j = 0; j < kSmallDims; ++j) {
+    if (j + 1 < kSmallDims && j + 1 < g.nd) {
+      const uint32_t q = (__umulhi(r, g.div[j].m) + r) >> g.div[j].s;
+      o += (int64_t)(r - q * g.div[j].d) * g.str[j];
+      r = q;
+    } else if (j + 1 == g.nd) {
+      o += (int64_t)r * g.str[j];
+    }
+  }
+  return o;
+}
+
+// Split pass straight from a tensor read in place (rows and k given as index
+// groups): a workgroup takes 64 rows x 64 k-values, decodes their offsets once,
+// reads them with lanes along the tensor's contiguous side into LDS, and each
+// wave splits two blocks out of LDS. Replaces a transpose of the operand (a
+// read and a write of it) and the re-read by k_split3.
+template <bool ROWS>
+__global__ __launch_bounds__(256) void k_split3_gather(const float *__restrict__ x, const DevGroup<kSmallDims> grow,
+                                                       const DevGroup<kSmallDims> gk, int rows, int k,
+                                                       unsigned short *__restrict__ planes, int rows_pad, int k_pad,
+                                                       int64_t blk, int64_t plane)
+{
+  typedef B3Layout<16, 32> Lay;
+  constexpr int TS = 64;
+  __shared__ float t[TS][TS + 1];         // [k][row]
+  __shared__ int64_t off[2][TS];          // rows, k
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int nkt = (k_pad + TS - 1) / TS, ntiles = rows_pad / TS * nkt;
+  const int rr = lane / Lay::kChunks, c = Lay::pos(rr, lane % Lay::kChunks);
+  for (int ti = blockIdx.x; ti < ntiles; ti += gridDim.x) {
+    const int rt = ti / nkt, r0 = rt * TS, k0 = (ti - rt * nkt) * TS;
+    if (tid < TS) off[0][tid] = group_at(grow, min(r0 + tid, rows - 1));
+    else if (tid < 2 * TS) off[1][tid - TS] = group_at(gk, min(k0 + tid - TS, k - 1));
+    __syncthreads();
+    float v[TS / 4];
+#pragma unroll
+    for (int u = 0; u < TS / 4; ++u) {
+      const int i = ROWS ? lane : wave + 4 * u, j = ROWS ? wave + 4 * u : lane;  // row, k
+      v[u] = x[off[0][i] + off[1][j]];
+    }
+#pragma unroll
+    for (int u = 0; u < TS / 4; ++u) {
+      const int i = ROWS ? lane : wave + 4 * u, j = ROWS ? wave + 4 * u : lane;
+      t[j][i] = (r0 + i < rows && k0 + j < k) ? v[u] : 0.f;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      if (k0 + u * 32 >= k_pad) break;
+      us8 h0, h1, h2;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        unsigned short e0, e1, e2;
+        split3(t[u * 32 + c * 8 + e][wave * 16 + rr], e0, e1, e2);
+        h0[e] = e0; h1[e] = e1; h2[e] = e2;
+      }
+      const int64_t o = (int64_t)(rt * 4 + wave) * blk + (int64_t)(k0 / 32 + u) * 512 + lane * 8;
+      *reinterpret_cast<us8 *>(planes + o) = h0;
+      *reinterpret_cast<us8 *>(planes + plane + o) = h1;
+      *reinterpret_cast<us8 *>(planes + 2 * plane + o) = h2;
+    }
+    __syncthreads();
+  }
+}
+
+// k_splitk_reduce into a tensor written in place: D element (r, c) sits at the
+// offsets of its row and column groups. A wave takes 64 rows (which hold D's
+// contiguous index) of 16 columns. Replaces the product's own pass, D's
+// transpose back and, accumulating, its transpose in.
+__global__ __launch_bounds__(256) void k_splitk_reduce_gather(const float *__restrict__ part, int nz, int m, int n,
+                                                              const DevGroup<kSmallDims> grow,
+                                                              const DevGroup<kSmallDims> gcol, float *__restrict__ d,
+                                                              double alpha, int beta_zero)
+{
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int r = blockIdx.x * 64 + lane;
+  if (r >= m) return;
+  const int64_t ro = group_at(grow, r), mn = (int64_t)m * n;
+#pragma unroll 4
+  for (int u = 0; u < 16; ++u) {
+    const int c = blockIdx.y * 64 + wave * 16 + u;
+    if (c >= n) break;
+    double v = 0.0;
+    for (int z = 0; z < nz; ++z) v += (double)part[(int64_t)z * mn + (int64_t)c * m + r];
+    v *= alpha;
+    float *dst = d + ro + group_at(gcol, c);
+    if (!beta_zero) v += (double)*dst;
+    *dst = (float)v;
+  }
+}
+
 constexpr int kB3Form = 16;               // kernel form of the three-way split
 
 int64_t round_up(int64_t x, int64_t q) { return (x + q - 1) / q * q; }
@@ -470,6 +568,22 @@ B3Geom b3_geom(const GemmArgs &g)
   G.plane_b = G.np / rb * G.blk;
   G.nz = (G.kp + kB3Chunk - 1) / kB3Chunk;
   return G;
+}
+
+// The matrix kernel over split planes a3 and b3, K-chunk partials behind them.
+B3Params b3_product(const GemmArgs &g, const B3Geom &G, unsigned short *a3, unsigned short *b3, hipStream_t s)
+{
+  const bool cx = g.kind == C4;
+  B3Params p{};
+  p.a3 = a3; p.b3 = b3;
+  p.part = reinterpret_cast<float *>(b3 + 3 * G.plane_b);
+  p.m = (cx ? 2 : 1) * (int64_t)g.m; p.n = (int64_t)g.n; p.k_pad = G.kp;
+  p.kchunk = std::min<int64_t>(G.kp, kB3Chunk);
+  p.blk = G.blk; p.plane_a = G.plane_a; p.plane_b = G.plane_b;
+  p.tiles_m = (int)(G.mp / kB3M);
+  p.tiles_n = (int)(G.np / kB3N);
+  hipLaunchKernelGGL(k_gemm_bf16x3<kB3Form>, dim3(p.tiles_m * p.tiles_n, (int)G.nz), dim3(512), 0, s, p);
+  return p;
 }
 
 int launch_bf16x3(const GemmArgs &g, void *ws, hipStream_t s)
@@ -510,15 +624,7 @@ int launch_bf16x3(const GemmArgs &g, void *ws, hipStream_t s)
                        static_cast<const float2 *>(g.b), (int64_t)g.n, (int64_t)g.k, ldb, g.b_kfast ? 1 : 0,
                        g.conj_b ? 1 : 0, b3, G.np, G.kp, G.blk, G.plane_b);
   }
-  B3Params p{};
-  p.a3 = a3; p.b3 = b3;
-  p.part = reinterpret_cast<float *>(b3 + 3 * G.plane_b);
-  p.m = (cx ? 2 : 1) * (int64_t)g.m; p.n = (int64_t)g.n; p.k_pad = G.kp;
-  p.kchunk = std::min<int64_t>(G.kp, kB3Chunk);
-  p.blk = G.blk; p.plane_a = G.plane_a; p.plane_b = G.plane_b;
-  p.tiles_m = (int)(G.mp / kB3M);
-  p.tiles_n = (int)(G.np / kB3N);
-  hipLaunchKernelGGL(k_gemm_bf16x3<kB3Form>, dim3(p.tiles_m * p.tiles_n, (int)G.nz), dim3(512), 0, s, p);
+  const B3Params p = b3_product(g, G, a3, b3, s);
   const int64_t mn = (int64_t)g.m * (int64_t)g.n;
   if (cx) {
     const int rb = (int)std::min<int64_t>((mn + 255) / 256, 8192);
@@ -901,6 +1007,56 @@ int launch_gemm_ws(const GemmArgs &g, void *ws, size_t ws_bytes, hipStream_t s)
                        reinterpret_cast<float *>(b2));
   }
   return launch_matrix(r, 0, nullptr, 0, s);
+}
+
+// Three-way split product of tensors read in place. Groups of at most
+// kSmallDims dimensions and matrix indices below 2^31; rows along each
+// operand's contiguous side need not be known (a_kfast, b_kfast say which).
+bool split3_gather_ok(const GatherMaps &mp, size_t m, size_t n, size_t k)
+{
+  for (const GatherGroup *x : {&mp.a_row, &mp.a_k, &mp.b_row, &mp.b_k, &mp.c_row, &mp.c_col})
+    if (x->nd > kSmallDims) return false;
+  // runs of four elements on every side: with shorter ones the gathers and the
+  // scatter move single elements (2574 x 2560 x 3072, L's and D's runs shortened:
+  // 16 elements 267 us against 339 with transposes, 4 302 against 338, 2 357
+  // against 334)
+  auto run = [](const GatherGroup &x) { return x.nd > 0 && x.str[0] == 1 && x.ext[0] >= 4; };
+  return (run(mp.a_row) || run(mp.a_k)) && (run(mp.b_row) || run(mp.b_k)) && run(mp.c_row) &&
+         std::max({m, n, k}) < (size_t)1 << 24 && n <= (size_t)65535 * 64;
+}
+
+int launch_split3_gather(const GemmArgs &g, const GatherMaps &mp, void *ws, size_t ws_bytes, hipStream_t s)
+{
+  if (g.kind != R4 || !gemm_uses_split3(g) || !split3_gather_ok(mp, g.m, g.n, g.k)) return TALSH_INVALID_ARGS;
+  if (!ws || ws_bytes < gemm_workspace_bytes(g)) return TALSH_INVALID_ARGS;
+  const B3Geom G = b3_geom(g);
+  unsigned short *a3 = static_cast<unsigned short *>(ws), *b3 = a3 + 3 * G.plane_a;
+  auto shrink = [](const GatherGroup &x) {
+    const FullGroup f = dev_group(x);
+    DevGroup<kSmallDims> d{};
+    d.nd = f.nd;
+    for (int j = 0; j < kSmallDims; ++j) d.str[j] = f.str[j];
+    for (int j = 0; j + 1 < kSmallDims; ++j) d.div[j] = f.div[j];
+    return d;
+  };
+  auto split = [&](const void *x, const GatherGroup &row, const GatherGroup &kg, size_t rows, bool kfast,
+                   unsigned short *out, int64_t rows_pad, int64_t plane) {
+    const int64_t tiles = rows_pad / 64 * ((G.kp + 63) / 64);
+    const dim3 grid((unsigned)std::min<int64_t>(tiles, 1 << 16));
+    if (kfast)
+      hipLaunchKernelGGL(k_split3_gather<false>, grid, dim3(256), 0, s, static_cast<const float *>(x), shrink(row),
+                         shrink(kg), (int)rows, (int)g.k, out, (int)rows_pad, (int)G.kp, G.blk, plane);
+    else
+      hipLaunchKernelGGL(k_split3_gather<true>, grid, dim3(256), 0, s, static_cast<const float *>(x), shrink(row),
+                         shrink(kg), (int)rows, (int)g.k, out, (int)rows_pad, (int)G.kp, G.blk, plane);
+  };
+  split(g.a, mp.a_row, mp.a_k, g.m, g.a_kfast, a3, G.mp, G.plane_a);
+  split(g.b, mp.b_row, mp.b_k, g.n, g.b_kfast, b3, G.np, G.plane_b);
+  const B3Params p = b3_product(g, G, a3, b3, s);
+  hipLaunchKernelGGL(k_splitk_reduce_gather, dim3((unsigned)((g.m + 63) / 64), (unsigned)((g.n + 63) / 64)), dim3(256), 0,
+                     s, p.part, (int)G.nz, (int)g.m, (int)g.n, shrink(mp.c_row), shrink(mp.c_col),
+                     static_cast<float *>(g.c), g.alpha_re, g.beta_zero ? 1 : 0);
+  return XT_HIP_OK(hipGetLastError()) ? 0 : TALSH_FAILURE;
 }
 
 int launch_gemm_gather(const GemmArgs &args, const GatherMaps &mp, void *ws, size_t ws_bytes, hipStream_t s)

@@ -110,6 +110,10 @@ size_t gemm_gather_workspace_bytes(const GemmArgs &g);
 // ws: partials of split K (gemm_split_bytes; may be null). Groups of more than
 // one dimension need fewer than 2^31 indices (TALSH_LIMIT_EXCEEDED otherwise).
 int launch_gemm_gather(const GemmArgs &g, const GatherMaps &maps, void *ws, size_t ws_bytes, hipStream_t s);
+// The three-way split (R4) with operands and result in place; same workspace
+// as the matricized form (gemm_workspace_bytes).
+bool split3_gather_ok(const GatherMaps &maps, size_t m, size_t n, size_t k);
+int launch_split3_gather(const GemmArgs &g, const GatherMaps &maps, void *ws, size_t ws_bytes, hipStream_t s);
 // Fixed per-GPU scratch of the allocation-free product entry point: a
 // file-scope device array in k_gemm.hip (64 MiB, held by every GPU the
 // library runs on until the process ends). gemm_noalloc_scratch returns its
