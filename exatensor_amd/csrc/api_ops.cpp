@@ -1652,7 +1652,7 @@ static int svd_op(const char *cptrn, talsh_tens_t *dtens, talsh_tens_t *ltens, t
     int64_t lu, ru, nv;
     std::vector<int> dd, d_o2n, ln, l_n2o, rn, r_n2o;
     bool dperm, lperm, rperm;
-    void *z = nullptr, *lm = nullptr, *rm = nullptr, *work = nullptr;
+    void *z = nullptr, *lm = nullptr, *rm = nullptr, *work = nullptr, *spare = nullptr;
     int allocate(Temps &t)
     {
       const size_t es = (size_t)kind_size(kind);
@@ -1661,6 +1661,8 @@ static int svd_op(const char *cptrn, talsh_tens_t *dtens, talsh_tens_t *ltens, t
       if (!e && lperm) e = t.alloc(es * (size_t)(lu * nv), &lm);
       if (!e && rperm) e = t.alloc(es * (size_t)(nv * ru), &rm);
       if (!e) e = t.alloc(svd_workspace_bytes(kind, lu, ru), &work);
+      const size_t sp = svd_spare_bytes(kind, lu, ru);
+      if (!e && sp && t.alloc(sp, &spare)) spare = nullptr;  // slower without
       return e;
     }
     int enqueue(Task *k, Device *)
@@ -1676,6 +1678,7 @@ static int svd_op(const char *cptrn, talsh_tens_t *dtens, talsh_tens_t *ltens, t
       g.rmat = rperm ? rm : R->exec;
       g.svals = S->exec;
       g.work = work;
+      g.spare = spare;
       g.absorb = mode;
       g.max_sweeps = 80;
       e = launch_svd(g, k->stream);

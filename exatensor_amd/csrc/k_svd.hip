@@ -132,6 +132,196 @@ __global__ __launch_bounds__(kSvdThreads) void k_jacobi_round(typename Z<CPLX>::
   apply(V + (int64_t)p * n, V + (int64_t)q * n, n);
 }
 
+// Several rounds of a sweep in one launch, on columns held in LDS, with the
+// same arithmetic as k_jacobi_round to the last bit (singular vectors are
+// unique up to a sign or phase only, and which one comes out depends on the
+// rounding of every rotation on the way).
+//
+// Pair k of round r holds columns r + k and r - k (mod ne - 1); in the next
+// round the first belongs to pair k - 1, the second to pair k + 1 (with the
+// ends k = 0 and ne / 2 - 1 as walls). So what pairs [a, b) hold after `rounds`
+// rounds depends on pairs [a - rounds + 1, b + rounds - 1) at the start only:
+// a workgroup owns W pairs, loads the columns (of B and of V) of that wider
+// window, repeats its neighbours' rotations where it needs them, and writes
+// the columns that its own pairs hold at the end, to a second pair of
+// matrices. What is left per round is a rotation's own serial chain (three
+// dot products, the rotation's square roots and quotients, the update), one
+// wave per pair: about 2.1 us, and 8 us for each launch with its loads and
+// stores, against 3.6 us for a launch per round.
+//
+// Windows have as many pairs as the workgroup has waves (all of what LDS holds
+// and the waves in turn: R8 186 x 150 11.7 ms, 96 x 95 11.3; 24 pairs 11.3 and
+// 6.9; 16 pairs 10.3 and 6.4; a launch per round 11.8 and 8.0), and at least
+// kSvdWindowMin, or all: with fewer a launch covers too few rounds (R8 500 x
+// 400, 10 pairs: 51.5 ms against 50.4; C8 1000 x 100, 4 pairs: 15.5 against
+// 11.7; with 12, C8 300 x 97: 7.9 against 9.6). One wave must not take too long
+// over a column either: all pairs in one window gain at R8 2000 x 8 (0.58
+// against 0.71) and C8 400 x 20 (1.25 against 1.67) and lose at C8 1000 x 16
+// (1.37 against 1.31).
+constexpr int kSvdWaves = 16;
+constexpr size_t kSvdLds = 150 * 1024;
+constexpr int kSvdWindow = kSvdWaves, kSvdWindowMin = 12;  // pairs in a window
+
+// Lane 0: the sum of a wave's share of 256 partial sums (lane l holds numbers
+// l, l + 64, l + 128, l + 192), halved as k_jacobi_round's tree does: 128 and
+// 64 within the lane, 32 and 16 across rows of 16 lanes, the rest inside the
+// first row by row shifts.
+template <int SHIFT>
+__device__ __forceinline__ double row_shift_add(double t)
+{
+  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(t), 0x100 | SHIFT, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(t), 0x100 | SHIFT, 0xf, 0xf, true);
+  return t + __hiloint2double(hi, lo);
+}
+__device__ __forceinline__ double svd_tree(const double (&v)[4])
+{
+  double t = (v[0] + v[2]) + (v[1] + v[3]);
+  t += __shfl_xor(t, 32);
+  t += __shfl_xor(t, 16);
+  t = row_shift_add<8>(t);
+  t = row_shift_add<4>(t);
+  t = row_shift_add<2>(t);
+  return row_shift_add<1>(t);
+}
+
+template <bool CPLX>
+__global__ __launch_bounds__(64 * kSvdWaves) void k_jacobi_rounds(
+    const typename Z<CPLX>::T *__restrict__ B, const typename Z<CPLX>::T *__restrict__ V,
+    typename Z<CPLX>::T *__restrict__ Bo, typename Z<CPLX>::T *__restrict__ Vo, int m, int n, int ne, int r0, int rounds,
+    int own, double tol, double *__restrict__ off)
+{
+  typedef typename Z<CPLX>::T T;
+  extern __shared__ __align__(16) unsigned char svd_lds[];
+  T *cols = reinterpret_cast<T *>(svd_lds);
+  __shared__ double dots[kSvdWindow][4], rot[kSvdWindow][4];  // of pair lo0 + index
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int n1 = ne - 1, np = ne / 2, len = m + n;
+  const int a0 = blockIdx.x * own, b0 = min(a0 + own, np);
+  const int lo0 = max(0, a0 - (rounds - 1)), hi0 = min(np, b0 + (rounds - 1));
+  // column in slot s at round r0: first (side 0) or second column of pair lo0 + s / 2
+  auto column = [&](int r, int k, int side) {
+    int p, q;
+    pair_of(ne, r, k, p, q);
+    return side ? q : p;
+  };
+  auto slot_of = [&](int c) {
+    int k = 0, side = 0;
+    if (c != n1) {
+      int d = c - r0;
+      if (d < 0) d += n1;
+      if (d == 0) side = 1;
+      else if (d < np) k = d;
+      else { k = n1 - d; side = 1; }
+    }
+    return 2 * (k - lo0) + side;
+  };
+  for (int s = wave; s < 2 * (hi0 - lo0); s += kSvdWaves) {
+    const int c = column(r0, lo0 + s / 2, s & 1);
+    if (c >= n) continue;  // a bye
+    T *dst = cols + (size_t)s * len;
+    for (int i = lane; i < m; i += 64) dst[i] = B[(int64_t)c * m + i];
+    for (int i = lane; i < n; i += 64) dst[m + i] = V[(int64_t)c * n + i];
+  }
+  __syncthreads();
+  for (int h = 0; h < rounds; ++h) {
+    const int reach = rounds - 1 - h, lo = max(0, a0 - reach), hi = min(np, b0 + reach);
+    // dot products, one wave per pair
+    for (int k = lo + wave; k < hi; k += kSvdWaves) {
+      int p, q;
+      pair_of(ne, r0 + h, k, p, q);
+      if (p >= n || q >= n) continue;  // a bye
+      if (p > q) { const int t = p; p = q; q = t; }
+      const T *bp = cols + (size_t)slot_of(p) * len, *bq = cols + (size_t)slot_of(q) * len;
+      // partial sums and their tree as 256 threads form them
+      double a[4] = {0.0, 0.0, 0.0, 0.0}, b[4] = {0.0, 0.0, 0.0, 0.0}, gr[4] = {0.0, 0.0, 0.0, 0.0},
+             gi[4] = {0.0, 0.0, 0.0, 0.0};
+      for (int base = 0; base < m; base += kSvdThreads) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const int i = base + lane + 64 * j;
+          if (i < m) {
+            const T x = bp[i], y = bq[i];
+            a[j] += Z<CPLX>::nrm2(x);
+            b[j] += Z<CPLX>::nrm2(y);
+            if constexpr (CPLX) {
+              const T g = Z<CPLX>::cdot(x, y);
+              gr[j] += g.x;
+              gi[j] += g.y;
+            } else {
+              gr[j] += x * y;
+            }
+          }
+        }
+      }
+      const double sa = svd_tree(a), sb = svd_tree(b), sr = svd_tree(gr), si = CPLX ? svd_tree(gi) : 0.0;
+      if (lane == 0) {
+        dots[k - lo0][0] = sa;
+        dots[k - lo0][1] = sb;
+        dots[k - lo0][2] = sr;
+        dots[k - lo0][3] = si;
+      }
+    }
+    __syncthreads();
+    // the rotations, one lane per pair (a wave per pair would issue the same
+    // chain of quotients and square roots for all its lanes)
+    if (wave == 0 && lo + lane < hi) {
+      const int k = lo + lane;
+      int p, q;
+      pair_of(ne, r0 + h, k, p, q);
+      double c = 1.0, s = 0.0, cp = 1.0, sp = 0.0;
+      if (p < n && q < n) {
+        const double sa = dots[k - lo0][0], sb = dots[k - lo0][1], sr = dots[k - lo0][2], si = dots[k - lo0][3];
+        // a real column pair's modulus is |sr| to the bit where its square neither overflows nor underflows
+        double ag = fabs(sr);
+        if (CPLX || !(ag > 1e-150 && ag < 1e150)) ag = sqrt(sr * sr + si * si);
+        const double scale = sqrt(sa * sb);
+        if (scale > 0.0 && ag > tol * scale) {
+          const double zeta = (sb - sa) / (2.0 * ag);
+          const double t = (zeta >= 0.0 ? 1.0 : -1.0) / (fabs(zeta) + sqrt(1.0 + zeta * zeta));
+          c = 1.0 / sqrt(1.0 + t * t);
+          s = c * t;
+          cp = sr / ag;
+          sp = si / ag;
+          if (k >= a0 && k < b0) off[k] = fmax(off[k], ag / scale);
+        }
+      }
+      rot[k - lo0][0] = c;
+      rot[k - lo0][1] = s;
+      rot[k - lo0][2] = cp;
+      rot[k - lo0][3] = sp;
+    }
+    __syncthreads();
+    for (int k = lo + wave; k < hi; k += kSvdWaves) {
+      const double c = rot[k - lo0][0], s = rot[k - lo0][1], cp = rot[k - lo0][2], sp = rot[k - lo0][3];
+      if (s == 0.0) continue;
+      int p, q;
+      pair_of(ne, r0 + h, k, p, q);
+      if (p > q) { const int t = p; p = q; q = t; }
+      T *bp = cols + (size_t)slot_of(p) * len, *bq = cols + (size_t)slot_of(q) * len;
+      for (int i = lane; i < len; i += 64) {
+        const T x = bp[i], y = bq[i];
+        if constexpr (CPLX) {
+          const double2 yt = make_double2(cp * y.x + sp * y.y, cp * y.y - sp * y.x);
+          bp[i] = make_double2(c * x.x - s * yt.x, c * x.y - s * yt.y);
+          bq[i] = make_double2(s * x.x + c * yt.x, s * x.y + c * yt.y);
+        } else {
+          const double yt = cp * y;
+          bp[i] = c * x - s * yt;
+          bq[i] = s * x + c * yt;
+        }
+      }
+    }
+    __syncthreads();
+  }
+  for (int s = wave; s < 2 * (b0 - a0); s += kSvdWaves) {
+    const int c = column(r0 + rounds - 1, a0 + s / 2, s & 1);
+    if (c >= n) continue;
+    const T *src = cols + (size_t)slot_of(c) * len;
+    for (int i = lane; i < m; i += 64) Bo[(int64_t)c * m + i] = src[i];
+    for (int i = lane; i < n; i += 64) Vo[(int64_t)c * n + i] = src[m + i];
+  }
+}
+
 template <bool CPLX>
 __global__ __launch_bounds__(kSvdThreads) void k_colnorm(const typename Z<CPLX>::T *__restrict__ B, int64_t m,
                                                           double *__restrict__ sigma)
@@ -258,6 +448,15 @@ __global__ void k_zero(double *__restrict__ p, int64_t n)
 
 int grid_for(int64_t n) { return (int)std::min<int64_t>((n + 255) / 256, 4096); }
 
+// Pairs in a window of k_jacobi_rounds; 0: a launch per round.
+int svd_window(size_t word, int64_t m, int64_t n)
+{
+  const int64_t np = (n + 1) / 2, fit = (int64_t)(kSvdLds / (word * (size_t)(m + n))) / 2;
+  const int64_t w = std::min({np, fit, (int64_t)kSvdWindow});
+  const bool all = w == np && m <= (word == 16 ? 512 : 2048);
+  return all || w >= kSvdWindowMin ? (int)w : 0;
+}
+
 template <typename T, bool CPLX>
 int svd_t(const SvdArgs &g, hipStream_t s)
 {
@@ -278,11 +477,36 @@ int svd_t(const SvdArgs &g, hipStream_t s)
                      words);
   const double tol = 1e-15;
   std::vector<double> offh(ne / 2);
+  // rounds per launch: what a window of columns in LDS allows (all of a sweep
+  // when it holds every pair)
+  W *B2 = static_cast<W *>(g.spare), *V2 = B2 ? B2 + m * n : nullptr;
+  const int np = ne / 2, window = svd_window(sizeof(W), m, n);
+  int own = np, per_launch = ne - 1;
+  if (window < np) {
+    own = std::max(1, window / 8);
+    per_launch = (window - own) / 2 + 1;
+  }
+  const bool many =
+      B2 && window > 0 &&
+      hipFuncSetAttribute(reinterpret_cast<const void *>(&k_jacobi_rounds<CPLX>),
+                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)kSvdLds) == hipSuccess;
+  const size_t lds = sizeof(W) * (size_t)(m + n) * 2 * (size_t)window;
   int sweep = 0;
   for (; sweep < g.max_sweeps && n > 1; ++sweep) {
     hipLaunchKernelGGL(k_zero, dim3(1), dim3(256), 0, s, off, (int64_t)(ne / 2));
-    for (int r = 0; r < ne - 1; ++r)
-      hipLaunchKernelGGL((k_jacobi_round<CPLX>), dim3(ne / 2), dim3(kSvdThreads), 0, s, B, V, m, n, ne, r, tol, off);
+    for (int r = 0; r < ne - 1;) {
+      if (!many) {
+        hipLaunchKernelGGL((k_jacobi_round<CPLX>), dim3(ne / 2), dim3(kSvdThreads), 0, s, B, V, m, n, ne, r, tol, off);
+        ++r;
+        continue;
+      }
+      const int rounds = std::min(per_launch, ne - 1 - r);
+      hipLaunchKernelGGL((k_jacobi_rounds<CPLX>), dim3((np + own - 1) / own), dim3(64 * kSvdWaves), lds, s, B, V, B2, V2,
+                         (int)m, n, ne, r, rounds, own, tol, off);
+      std::swap(B, B2);
+      std::swap(V, V2);
+      r += rounds;
+    }
     if (!XT_HIP_OK(hipMemcpyAsync(offh.data(), off, sizeof(double) * (ne / 2), hipMemcpyDeviceToHost, s)) ||
         !XT_HIP_OK(hipStreamSynchronize(s)))
       return TALSH_FAILURE;
@@ -317,6 +541,12 @@ size_t svd_workspace_bytes(int kind, int64_t lu, int64_t ru)
   const int64_t m = std::max(lu, ru), n = std::min(lu, ru), ne = n + (n & 1);
   const int64_t w = kind_complex(kind) ? 16 : 8;
   return (size_t)(w * (m * n + n * n) + 8 * (ne / 2 + n) + 4 * n + 64);
+}
+
+size_t svd_spare_bytes(int kind, int64_t lu, int64_t ru)
+{
+  const int64_t m = std::max(lu, ru), n = std::min(lu, ru), w = kind_complex(kind) ? 16 : 8;
+  return svd_window((size_t)w, m, n) > 0 ? (size_t)(w * (m * n + n * n)) : 0;
 }
 
 int launch_svd(const SvdArgs &g, hipStream_t s)

@@ -143,11 +143,13 @@ struct SvdArgs {
   const void *a;
   void *lmat, *rmat, *svals;
   void *work;          // svd_workspace_bytes(kind, lu, ru)
+  void *spare;         // svd_spare_bytes(kind, lu, ru) if any, or null: a launch per round then
   int absorb;
   int max_sweeps;
   double *sigma_out;   // optional host copy of the min(lu, ru) singular values
 };
 int launch_svd(const SvdArgs &g, hipStream_t s);
 size_t svd_workspace_bytes(int kind, int64_t lu, int64_t ru);
+size_t svd_spare_bytes(int kind, int64_t lu, int64_t ru);
 
 }  // namespace xt
