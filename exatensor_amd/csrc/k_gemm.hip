@@ -723,6 +723,19 @@ SplitGeom split_geom(const GemmArgs &g, const TileShape &ts, int cus, size_t bud
   return G;
 }
 
+bool gemm_vec_loads(int es, bool kfast, size_t rows, size_t k)
+{
+  return kfast ? k * (size_t)es % 16 == 0 : k % 8 == 0 && rows % 2 == 0;
+}
+
+bool gather_vec_loads(int es, bool kfast, const GatherGroup &row, const GatherGroup &kg, size_t k)
+{
+  const GatherGroup &x = kfast ? kg : row;
+  return x.nd > 0 && x.str[0] == 1 && x.ext[0] % (kfast ? std::max(16 / es, 1) : 2) == 0 && (kfast || k % 8 == 0);
+}
+
+bool gather_uniform_k(int kind, const GatherGroup &kg) { return kg.nd <= 1 || kg.ext[0] % tile_shape(kind, 0).bk == 0; }
+
 // Large complex products in native precision run realified through the real
 // 128x128 kernels (which re-read operands from L2 half as often as the 64x64
 // complex kernel), when the real product has enough 128x128 tiles to fill the
@@ -843,6 +856,7 @@ void gemm_tile_shape(int kind, R4Mode r4mode, int tile, int *bm, int *bn, int *o
   const TileShape ts = tile_shape(kind, tile);
   *bm = ts.bm;
   *bn = ts.bn;
+  if (ts.groups > 1) *occupancy = 1;
 }
 
 namespace {
@@ -951,9 +965,8 @@ int launch_matrix(GemmArgs g, int tile, void *ws, size_t ws_bytes, hipStream_t s
   const int es = kind_size(g.kind);
   const int64_t lim = (1ll << 31) - 1, bytes = std::max(p.m, p.n) * p.k * es;
   const bool off32 = p.m <= lim && p.n <= lim && p.k <= lim && bytes < (1ll << 32);
-  const int64_t vw = 16 / es;
-  auto vec = [&](bool kfast, int64_t rows) { return kfast ? p.k % vw == 0 : p.k % 8 == 0 && rows % 2 == 0; };
-  q.mode = !off32 ? kWide : vec(g.a_kfast, p.m) && vec(g.b_kfast, p.n) ? kVec : kUni;
+  q.mode = !off32 ? kWide
+           : gemm_vec_loads(es, g.a_kfast, g.m, g.k) && gemm_vec_loads(es, g.b_kfast, g.n, g.k) ? kVec : kUni;
   exchange(q, g);
   return launch_product(q, g, tile, ws, ws_bytes, s);
 }
@@ -1089,15 +1102,6 @@ int launch_gemm_gather(const GemmArgs &args, const GatherMaps &mp, void *ws, siz
   p.b_k = dev_group(mp.b_k);
   p.c_row = dev_group(mp.c_row);
   p.c_col = dev_group(mp.c_col);
-  // a k-tile starts at one offset for all lanes when it cannot cross a digit
-  // of the first contracted dimension; operands of real kinds then load
-  // vectors if their runs hold whole ones
-  const int bk = tile_shape(g.kind, 0).bk, vw = 16 / es;
-  auto uniform = [&](const GatherGroup &x) { return x.nd <= 1 || x.ext[0] % bk == 0; };
-  auto vec = [&](bool kfast, const GatherGroup &row, const GatherGroup &k) {
-    const GatherGroup &x = kfast ? k : row;
-    return x.nd > 0 && x.str[0] == 1 && x.ext[0] % (kfast ? vw : 2) == 0 && (kfast || g.k % 8 == 0);
-  };
   const size_t lim = INT32_MAX;
   const bool off32 = g.m <= lim && g.n <= lim && g.k <= lim && (last[0] + last[1] + 1) * es < (1ll << 32) &&
                      (last[2] + last[3] + 1) * es < (1ll << 32);
@@ -1105,8 +1109,9 @@ int launch_gemm_gather(const GemmArgs &args, const GatherMaps &mp, void *ws, siz
   for (int t = 0; t < 6; ++t) small = small && grp[t]->nd <= kSmallDims;
   q.mode = kGen;
   if (!off32 || !small) q.mode = kWide;
-  else if (uniform(mp.a_k) && uniform(mp.b_k))
-    q.mode = vec(g.a_kfast, mp.a_row, mp.a_k) && vec(g.b_kfast, mp.b_row, mp.b_k) ? kVec : kUni;
+  else if (gather_uniform_k(g.kind, mp.a_k) && gather_uniform_k(g.kind, mp.b_k))
+    q.mode = gather_vec_loads(es, g.a_kfast, mp.a_row, mp.a_k, g.k) && gather_vec_loads(es, g.b_kfast, mp.b_row, mp.b_k, g.k)
+                 ? kVec : kUni;
   const int tile = resolved_tile(g);
   // write along the columns: they should hold C's stride-1 index
   if (mp.c_row.nd > 0 && mp.c_row.str[0] == 1 && !(mp.c_col.nd > 0 && mp.c_col.str[0] == 1)) exchange(q, g);

@@ -114,6 +114,13 @@ int launch_gemm_gather(const GemmArgs &g, const GatherMaps &maps, void *ws, size
 // as the matricized form (gemm_workspace_bytes).
 bool split3_gather_ok(const GatherMaps &maps, size_t m, size_t n, size_t k);
 int launch_split3_gather(const GemmArgs &g, const GatherMaps &maps, void *ws, size_t ws_bytes, hipStream_t s);
+// What the native kernels' loads need of an operand (real kinds, element size
+// es): whole 16-byte vectors along k, or row pairs with the k-values in
+// eights; for a gathered operand also, that a k-tile starts at one offset for
+// all lanes (it does not cross a digit of the first contracted dimension).
+bool gemm_vec_loads(int es, bool kfast, size_t rows, size_t k);
+bool gather_vec_loads(int es, bool kfast, const GatherGroup &row, const GatherGroup &kg, size_t k);
+bool gather_uniform_k(int kind, const GatherGroup &kg);
 // Fixed per-GPU scratch of the allocation-free product entry point: a
 // file-scope device array in k_gemm.hip (64 MiB, held by every GPU the
 // library runs on until the process ends). gemm_noalloc_scratch returns its

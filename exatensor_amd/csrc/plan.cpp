@@ -8,7 +8,7 @@
 // heuristics elsewhere (TALSH/tensor_algebra_gpu_nvidia.cu:1188-1272,
 // TALSH/talshc.cpp:366-488). Here the GEMM reads either operand k-fast or
 // m/n-fast and may compute D^T, and a fused-gather plan reads the tensors
-// where they lie through offset tables, so several candidates exist; the
+// where they lie through groups of extents and strides, so several candidates exist; the
 // byte-count heuristic ranks the transposing ones and an optional learned
 // model (a small MLP predicting the log of kernel time from the features
 // below) chooses among all candidates and GEMM tile shapes.
@@ -356,11 +356,10 @@ int plan_candidates(const std::vector<int> &dig, int dr, int lr, int rr, const s
       f[33] = lg2(tm * bm * tn * bn / (gm * gn));
       f[34] = (float)std::log2(tm * tn / (double)(num_cus > 0 ? num_cus : 256));
       f[35] = (float)occ;
-      // 16-byte vector loads of the GEMM operands (k-fast rows of 16-byte multiples;
-      // a_kfast / b_kfast already describe the GEMM's A and B after a swap)
-      const bool kal = ((size_t)gk * es) % 16 == 0;
-      f[36] = c.a_kfast && kal && !cplx;
-      f[37] = c.b_kfast && kal && !cplx;
+      // vector loads of the GEMM operands (a_kfast / b_kfast already describe
+      // the GEMM's A and B after a swap)
+      f[36] = !cplx && gemm_vec_loads(es, c.a_kfast, (size_t)gm, (size_t)gk);
+      f[37] = !cplx && gemm_vec_loads(es, c.b_kfast, (size_t)gn, (size_t)gk);
       // transpose kernel plans: vector width and the scatter fallback
       f[53] = lg2(gemm_splitk_count(kind, r4mode, (size_t)gm, (size_t)gn, (size_t)gk, t, num_cus > 0 ? num_cus : 256));
       put_plan(f + 38, kind, ld, c.l_o2n);
@@ -377,7 +376,6 @@ int plan_candidates(const std::vector<int> &dig, int dr, int lr, int rr, const s
     const double gm = (double)(c.swap ? c.n : c.m), gn = (double)(c.swap ? c.m : c.n), gk = (double)c.k;
     const GatherGroup &sa = c.a_kfast ? c.maps.a_k : c.maps.a_row, &sb = c.b_kfast ? c.maps.b_k : c.maps.b_row;
     auto unit_run = [](const GatherGroup &g) { return (g.nd > 0 && g.str[0] == 1) ? (double)g.ext[0] : 1.0; };
-    auto first_ext = [](const GatherGroup &g) { return g.nd > 0 ? g.ext[0] : 1; };
     for (int t = 0; t < ntiles; ++t) {
       PlanCandidate pc;
       pc.variant = kFusedVariantBase + v;
@@ -396,12 +394,12 @@ int plan_candidates(const std::vector<int> &dig, int dr, int lr, int rr, const s
       f[33] = lg2(tm * bm * tn * bn / (gm * gn));
       f[34] = (float)std::log2(tm * tn / (double)(num_cus > 0 ? num_cus : 256));
       f[35] = (float)occ;
-      // 16-byte groups along each operand's staging direction
-      f[36] = !cplx && unit_run(sa) * es >= 16 && ((int)unit_run(sa) * es) % 16 == 0;
-      f[37] = !cplx && unit_run(sb) * es >= 16 && ((int)unit_run(sb) * es) % 16 == 0;
+      // vector loads along each operand's staging direction, and whether a
+      // k-tile starts at one offset for all lanes
+      f[36] = !cplx && gather_vec_loads(es, c.a_kfast, c.maps.a_row, c.maps.a_k, (size_t)gk);
+      f[37] = !cplx && gather_vec_loads(es, c.b_kfast, c.maps.b_row, c.maps.b_k, (size_t)gk);
       f[44] = 1.f;  // fused gather
-      const int run = bm / 16;  // elements one thread stages along its direction
-      f[45] = first_ext(sa) % run == 0 && first_ext(sb) % run == 0;
+      f[45] = gather_uniform_k(kind, c.maps.a_k) && gather_uniform_k(kind, c.maps.b_k);
       f[46] = c.maps.c_row.nd > 0 && c.maps.c_row.str[0] == 1;  // result rows along D's stride-1 index
       // contiguous run along each operand's staging direction, and the
       // stride between its staged elements when that is not 1
