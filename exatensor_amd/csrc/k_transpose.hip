@@ -44,6 +44,11 @@ constexpr int kMaxEPT = 8;         // tile vectors per thread (more cost occupan
 constexpr int kTiledPerCU = 2;     // persistent workgroups per CU (16 waves)
 constexpr int kTileMaxBytes = 65536;  // LDS tile (before padding)
 constexpr long kTileMinVol = 8192;    // tiles are grown to at least this many elements
+// Tiles of the run form: at most four vectors per thread (eight hold 76
+// registers per thread in R4 and keep a workgroup's loads and stores apart for
+// longer: R4 37x29x41x23x31 88 us with 64 KB tiles, 60 with these, 67 with 26
+// KB; 4001 x 4003 transposed 53, 33 and 34), grown to 16 KB.
+constexpr long kRunTileMaxBytes = 34 << 10, kRunTileMinBytes = 16 << 10;
 constexpr int kLine = 128;            // cache line bytes
 
 struct DevDiv { uint32_t d, m, s; };
@@ -816,9 +821,9 @@ bool plan_runs(int es, const Fused &f, int cus, int vec, int max_ept, Planned &p
   for (int i = 0; i < r; ++i) n2o[f.o2n[i]] = i;
   uint64_t vol = 1;
   for (int e : f.ext) vol *= (uint64_t)e;
-  const long max_vol = std::min<long>((long)kTNT * max_ept * vec, kTileMaxBytes / es);
+  const long max_vol = std::min<long>((long)kTNT * max_ept * vec, kRunTileMaxBytes / es);
   const long min_vol =
-      std::min<long>({max_vol, kTileMinVol, std::max<long>(1024, (long)(vol / (4 * (uint64_t)std::max(cus, 1))))});
+      std::min<long>({max_vol, kRunTileMinBytes / es, std::max<long>(1024, (long)(vol / (4 * (uint64_t)std::max(cus, 1))))});
   std::vector<int> t(r);
   auto volume = [&] {
     long v = 1;
