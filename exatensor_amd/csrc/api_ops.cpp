@@ -478,10 +478,10 @@ bool autotune_choose(const char *cptrn, talsh_tens_t *dtens, talsh_tens_t *ltens
   int bv = -1, bt = -1;
   // Above the selector's flop domain, fused-gather candidates are left out
   // when their operands are not both staged along a contiguous run (each
-  // staged element is then a separate access: 2.5-7 times the matricized
-  // product's time on the 96/128 contraction) and for complex kinds (a large
-  // complex product runs faster realified than in the complex kernel the
-  // gather uses: 61 against 57 TFLOP/s in FP64 there).
+  // staged element is then a separate access: several times the matricized
+  // product's time on the 96/128 contraction) and for complex kinds (with the
+  // realified product they ran slower there; the complex kernel has since come
+  // level with it, 64 TFLOP/s in FP64, so this only spares tuning time).
   double lflops = 1.0;  // log2 of the real flop count, as the selector's domain is defined
   for (int i = 0; i < lr; ++i) lflops += std::log2((double)ld[i]);
   for (int j = 0; j < rr; ++j)

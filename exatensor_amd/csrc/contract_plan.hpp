@@ -24,7 +24,7 @@ struct ContractPlan {
   size_t m = 1, n = 1, k = 1;
   double bytes_moved = 0;
   // fused index gather: no transposes, the product reads L and R and updates
-  // D in place through offset tables (maps in the launched orientation)
+  // D in place by its index groups (maps in the launched orientation)
   bool fused = false;
   GatherMaps maps;
 };

@@ -11,7 +11,7 @@
 //  2. k_grouped_gemm is persistent: each workgroup pulls work items (a
 //     128x128 tile of one D block plus the chain of (L, R) pairs that
 //     accumulate into it) from per-XCD device queues until all are empty.
-//     The inner loop is the dense engine GEMM's: double-buffered k-fast LDS
+//     The inner loop is one pipeline over a chain: double-buffered k-fast LDS
 //     tiles feeding 16x16x4 MFMAs (FP64 for R8, FP32 for R4). The epilogue
 //     scatters the tile into the D block through its index maps. Every D
 //     element is written by one workgroup in chain order: results are

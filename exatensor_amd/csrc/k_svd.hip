@@ -14,7 +14,9 @@
 // convergence B = A V has orthogonal columns: A = U diag(sigma) V^H with
 // sigma_j = |b_j| and u_j = b_j / sigma_j. A sweep visits every pair once in
 // n_e - 1 rounds of n_e / 2 disjoint pairs (round-robin tournament, n_e = n
-// rounded up to even; the extra index is a bye); one workgroup per pair.
+// rounded up to even; the extra index is a bye): several rounds per launch on
+// columns in LDS (k_jacobi_rounds), or one workgroup per pair and a launch per
+// round where columns are too long for that (k_jacobi_round).
 #include <algorithm>
 #include <vector>
 

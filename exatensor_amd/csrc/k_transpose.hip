@@ -20,8 +20,8 @@
 //    the per-tile work is one base-offset decode per workgroup plus one
 //    coalesced load and one coalesced store per vector.
 // The run form against the lane-masked single-element tiles it replaces, kernel
-// time: R4 37,29,41,23,31 -> 2,4,1,0,3 132 to 89 us; R8 119,70,65,34 reversed
-// 113 to 71; C8 14,23,104,3,35 43 to 32; 26 instead of 34 us in the geometric
+// time: R4 37,29,41,23,31 -> 2,4,1,0,3 132 to 60 us; R8 119,70,65,34 reversed
+// 113 to 69; C8 14,23,104,3,35 43 to 32; 25 instead of 34 us in the geometric
 // mean of 34 random shapes. A permuted addition in one pass: rank-6 extent-24
 // R8 1567 to 890 us.
 #include <algorithm>

@@ -29,10 +29,11 @@ int talshAmdProfileQuery(int kernel_class, double *total_ms, long long *launches
  * variant >= 0 selects the variant-th candidate matricization (ranked by the
  * built-in byte-count heuristic; 0 is the heuristic's choice), variant
  * TALSH_AMD_FUSED_VARIANT + i the i-th fused-gather candidate (no transposes:
- * the matrix product reads L and R and updates D through index offset
- * tables; native precision, so R4/C4 under fast math keep the heuristic's
- * matricization), -1 restores the heuristic; tile selects the GEMM tile
- * shape (-1 default). */
+ * the matrix product reads L and R and updates D by their index groups;
+ * native precision, so R4/C4 under fast math take the heuristic's
+ * matricization instead), -1 restores the engine's choice (which for R4 under
+ * fast math reads the tensors in place where their runs are long enough);
+ * tile selects the GEMM tile shape (-1 default). */
 #define TALSH_AMD_FUSED_VARIANT 1000
 int talshAmdSetPlanVariant(int variant, int tile);
 /* Number of distinct matricization candidates of a contraction and the bytes
