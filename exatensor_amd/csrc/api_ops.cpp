@@ -1123,6 +1123,7 @@ static int contract_impl(const char *cptrn, talsh_tens_t *dtens, talsh_tens_t *l
     double are, aim; int tile;
     void *lt = nullptr, *rt = nullptr, *dt = nullptr, *scr = nullptr, *tt = nullptr, *ws = nullptr;
     size_t wsb = 0;
+    bool ws_fixed = false;  // the partials go to the GPU's fixed scratch array
     // The matrix product as it is launched (operands exchanged when the plan
     // swaps them). The workspace is sized from the same arguments: the
     // three-way split pads rows of A and B to different multiples, so the
@@ -1183,14 +1184,29 @@ static int contract_impl(const char *cptrn, talsh_tens_t *dtens, talsh_tens_t *l
       return e;
     }
     // The product's workspace: `need` bytes or the call is deferred (callers
-    // rely on a full arena giving TRY_LATER), `want` bytes if there is room,
-    // so that K can be split further.
+    // rely on a full arena giving TRY_LATER). The `want` bytes of a native
+    // product's K pieces follow from its shape alone, and so must the pieces:
+    // a sum cut otherwise rounds otherwise. In an arena without room for them
+    // they go to the GPU's fixed scratch array, one product after the other.
     int workspace(Temps &t, size_t need, size_t want)
     {
-      wsb = want;
-      if (want > need && t.alloc(want, &ws) == 0) return 0;
-      wsb = need;
+      static_assert(kSplitBytesMax <= kGemmNoAllocScratchBytes, "K pieces fit the fixed scratch array");
+      wsb = want ? want : need;
+      if (need >= want) return need ? t.alloc(need, &ws) : 0;
+      const int e = t.alloc(want, &ws);
+      if (!e || !t.d->noalloc_scratch) return e;
+      ws_fixed = true;
       return need ? t.alloc(need, &ws) : 0;
+    }
+    int product(const GemmArgs &g, Device *dev, hipStream_t s)
+    {
+      auto launch = [&](void *w) {
+        if (!P.fused) return launch_gemm_ws(g, w, wsb, s);
+        return gemm_uses_split3(g) ? launch_split3_gather(g, P.maps, w, wsb, s) : launch_gemm_gather(g, P.maps, w, wsb, s);
+      };
+      if (!ws_fixed) return launch(ws);
+      ScratchUse use(dev, s);
+      return launch(dev->noalloc_scratch);
     }
     int enqueue(Task *k, Device *dev)
     {
@@ -1234,8 +1250,7 @@ static int contract_impl(const char *cptrn, talsh_tens_t *dtens, talsh_tens_t *l
         g.c = D->exec;
         if (k->timed) (void)hipEventRecord(k->ev_mm0, s);
         prof_begin(s, kKGemm, pr);
-        const int e = gemm_uses_split3(g) ? launch_split3_gather(g, P.maps, ws, wsb, s)
-                                          : launch_gemm_gather(g, P.maps, ws, wsb, s);
+        const int e = product(g, dev, s);
         prof_end(s, kKGemm, pr);
         if (k->timed) (void)hipEventRecord(k->ev_mm1, s);
         k->has_mm = k->timed;
@@ -1267,7 +1282,7 @@ static int contract_impl(const char *cptrn, talsh_tens_t *dtens, talsh_tens_t *l
       g.c = dc;
       if (k->timed) (void)hipEventRecord(k->ev_mm0, s);
       prof_begin(s, kKGemm, pr);
-      int e = launch_gemm_ws(g, ws, wsb, s);
+      int e = product(g, dev, s);
       prof_end(s, kKGemm, pr);
       if (k->timed) (void)hipEventRecord(k->ev_mm1, s);
       k->has_mm = k->timed;
@@ -1933,7 +1948,11 @@ int talshAmdGemmNoAlloc(int data_kind, int fast_math, size_t m, size_t n, size_t
   }
   (void)hipSetDevice(d->ordinal);
   hipStream_t s = d->streams[0];
-  const int e = launch_gemm_ws(g, d->noalloc_scratch, need, s);
+  int e;
+  {
+    ScratchUse use(d, s);
+    e = launch_gemm_ws(g, d->noalloc_scratch, need, s);
+  }
   if (e) return e;
   return XT_HIP_OK(hipStreamSynchronize(s)) ? 0 : TALSH_FAILURE;
 }

@@ -433,8 +433,11 @@ int talshInit(size_t *host_buf_size, int *host_arg_max, int ngpus, int gpu_list[
     for (int k = 0; k < kStreamsPerDevice; ++k)
       if (!XT_HIP_OK(hipStreamCreateWithFlags(&d->streams[k], hipStreamNonBlocking))) { delete d; return TALSH_FAILURE; }
     // this GPU's address of the allocation-free product's scratch array (device current)
-    if (gemm_noalloc_scratch(&d->noalloc_scratch))
+    if (gemm_noalloc_scratch(&d->noalloc_scratch) ||
+        !XT_HIP_OK(hipEventCreateWithFlags(&d->scratch_ev, hipEventDisableTiming))) {
+      d->noalloc_scratch = nullptr;
       log_error("GPU %d: scratch of talshAmdGemmNoAlloc not found; that entry point will fail", d->ordinal);
+    }
     E.gpus.push_back(d);
   }
   if (!E.gpus.empty()) (void)hipSetDevice(E.gpus[0]->ordinal);
@@ -485,6 +488,7 @@ int talshShutdown()
   for (Device *d : E.gpus) {
     for (auto &s : d->streams)
       if (s) (void)hipStreamDestroy(s);
+    if (d->scratch_ev) (void)hipEventDestroy(d->scratch_ev);
     if (d->arena.live_blocks() > 0) err = err ? err : NOT_CLEAN;
     if (d->arena_mem) (void)hipFree(d->arena_mem);
     delete d;

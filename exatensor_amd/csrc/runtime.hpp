@@ -32,7 +32,24 @@ struct Device {
   std::atomic<unsigned> next_stream{0};
   DeviceStats stats;
   R4Mode r4mode = R4Mode::kNativeF32;
-  void *noalloc_scratch = nullptr;   // this GPU's copy of the allocation-free product's scratch array
+  // this GPU's fixed scratch array (gemm_noalloc_scratch), used through
+  // ScratchUse: under the lock, each use after the one before (scratch_ev)
+  void *noalloc_scratch = nullptr;
+  std::mutex scratch_mu;
+  hipEvent_t scratch_ev = nullptr;
+};
+
+// One use of a GPU's fixed scratch array by the work that its owner enqueues
+// on stream s: that work starts when the last use, on whichever stream, ends.
+class ScratchUse {
+ public:
+  ScratchUse(Device *d, hipStream_t s) : d_(d), s_(s), g_(d->scratch_mu) { (void)hipStreamWaitEvent(s, d->scratch_ev, 0); }
+  ~ScratchUse() { (void)hipEventRecord(d_->scratch_ev, s_); }
+
+ private:
+  Device *d_;
+  hipStream_t s_;
+  std::lock_guard<std::mutex> g_;
 };
 
 struct Engine {
