@@ -43,8 +43,8 @@
 // slice is one contiguous LDS read (summation order over k is immaterial).
 //
 // Pipeline: at k-tile t the registers holding tile t+1 go to the other LDS
-// buffer first (their loads were issued PD tiles earlier), the loads of tile
-// t+1+PD follow into the same registers, then tile t is multiplied.
+// buffer first, the loads of tile t+2 follow into the same registers, then
+// tile t is multiplied.
 #pragma once
 
 #include <algorithm>
@@ -478,7 +478,7 @@ struct PartLayout {
   }
 };
 
-template <typename T, bool CPLX, bool AK, bool BKF, int BM, int BN, int BK, int KG, int PD, int OCC, GemmMode MODE>
+template <typename T, bool CPLX, bool AK, bool BKF, int BM, int BN, int BK, int KG, int OCC, GemmMode MODE>
 __global__ __launch_bounds__(256 * KG, OCC) void k_gemm_mfma(const GemmParams<group_dims(MODE)>)
 {
   ArgParams<group_dims(MODE)> &p = gemm_args_of_kernel<group_dims(MODE)>();
@@ -539,11 +539,10 @@ __global__ __launch_bounds__(256 * KG, OCC) void k_gemm_mfma(const GemmParams<gr
       sa.clamp_k(left_l);
       sb.clamp_k(left_l);
     }
-    T ra[PD][SA::NE * NP], rb[PD][SB::NE * NP];
-    auto load = [&](auto S) {  // the next k-tile into register set S
-      constexpr int s = decltype(S)::value;
-      sa.load(A, p.a_k, left_l, ra[s]);
-      sb.load(B, p.b_k, left_l, rb[s]);
+    T ra[SA::NE * NP], rb[SB::NE * NP];
+    auto load = [&]() {  // the next k-tile
+      sa.load(A, p.a_k, left_l, ra);
+      sb.load(B, p.b_k, left_l, rb);
       if (!SA::UNI || left_l > BK * KG) {
         left_l -= BK * KG;
         sa.walk.advance(p.a_k);
@@ -554,14 +553,13 @@ __global__ __launch_bounds__(256 * KG, OCC) void k_gemm_mfma(const GemmParams<gr
         }
       }
     };
-    auto store = [&](auto S, int buf) {  // register set S into LDS buffer buf
-      constexpr int s = decltype(S)::value;
+    auto store = [&](int buf) {  // the loaded k-tile into LDS buffer buf
       if (left_s < BK) {  // the last, partial k-tile, or none left for this group
-        sa.zero_past(ra[s], left_s);
-        sb.zero_past(rb[s], left_s);
+        sa.zero_past(ra, left_s);
+        sb.zero_past(rb, left_s);
       }
-      sa.to_lds(la + buf * NP * BM, ra[s], ca);
-      sb.to_lds(lb + buf * NP * BN, rb[s], cb);
+      sa.to_lds(la + buf * NP * BM, ra, ca);
+      sb.to_lds(lb + buf * NP * BN, rb, cb);
       left_s -= BK * KG;
     };
     auto compute = [&](int buf) {
@@ -598,30 +596,17 @@ __global__ __launch_bounds__(256 * KG, OCC) void k_gemm_mfma(const GemmParams<gr
               }
         }
     };
-    const std::integral_constant<int, 0> c0;
-    const std::integral_constant<int, PD - 1> c1;  // register set of odd tiles
-    static_assert(PD == 1 || PD == 2, "register sets");
-    load(c0);
-    if constexpr (PD == 2) load(c1);
-    store(c0, 0);
-    load(c0);
+    load();
+    store(0);
+    load();
     __syncthreads();
     // (past the last k-tile, stores and loads go on harmlessly: into the
     // buffer that is not read any more, from addresses in range)
-    int buf = 0;
-    auto step = [&](auto S) {
-      store(S, buf ^ 1);
-      load(S);
+    for (int t = 0, buf = 0; t < nt; ++t, buf ^= 1) {
+      store(buf ^ 1);
+      load();
       compute(buf);
       __syncthreads();
-      buf ^= 1;
-    };
-    for (int t = 0; t < nt; ++t) {
-      step(c1);
-      if constexpr (PD == 2) {
-        if (++t >= nt) break;
-        step(c0);
-      }
     }
   }
 
@@ -760,14 +745,14 @@ GemmParams<N> shortened(const GemmParams<kGatherMaxDims> &f)
   }
 }
 
-template <typename T, bool CPLX, bool AK, bool BKF, int BM, int BN, int BK, int KG, int PD, int OCC, GemmMode MODE>
+template <typename T, bool CPLX, bool AK, bool BKF, int BM, int BN, int BK, int KG, int OCC, GemmMode MODE>
 int launch_tile(const Product &q, hipStream_t s)
 {
   constexpr int N = group_dims(MODE);
   const GemmParams<N> p = shortened<N>(q.p);
   const int64_t tiles = (int64_t)p.tiles_m * p.tiles_n;
   const int64_t blocks = p.full + (tiles - p.full) * p.parts;
-  hipLaunchKernelGGL((k_gemm_mfma<T, CPLX, AK, BKF, BM, BN, BK, KG, PD, OCC, MODE>), dim3((unsigned)blocks),
+  hipLaunchKernelGGL((k_gemm_mfma<T, CPLX, AK, BKF, BM, BN, BK, KG, OCC, MODE>), dim3((unsigned)blocks),
                      dim3(256 * KG), 0, s, p);
   if (tiles > p.full)
     hipLaunchKernelGGL((k_splitk_sum<T, CPLX, BM, BN, N>), dim3((unsigned)((tiles - p.full) * (BM / 16))), dim3(256), 0, s,
@@ -775,23 +760,23 @@ int launch_tile(const Product &q, hipStream_t s)
   return XT_HIP_OK(hipGetLastError()) ? 0 : TALSH_FAILURE;
 }
 
-template <typename T, bool CPLX, int BM, int BN, int BK, int KG, int PD, int OCC, GemmMode MODE>
+template <typename T, bool CPLX, int BM, int BN, int BK, int KG, int OCC, GemmMode MODE>
 int launch_orient(const Product &q, hipStream_t s)
 {
-  if (q.a_kfast && q.b_kfast) return launch_tile<T, CPLX, true, true, BM, BN, BK, KG, PD, OCC, MODE>(q, s);
-  if (q.a_kfast) return launch_tile<T, CPLX, true, false, BM, BN, BK, KG, PD, OCC, MODE>(q, s);
-  if (q.b_kfast) return launch_tile<T, CPLX, false, true, BM, BN, BK, KG, PD, OCC, MODE>(q, s);
-  return launch_tile<T, CPLX, false, false, BM, BN, BK, KG, PD, OCC, MODE>(q, s);
+  if (q.a_kfast && q.b_kfast) return launch_tile<T, CPLX, true, true, BM, BN, BK, KG, OCC, MODE>(q, s);
+  if (q.a_kfast) return launch_tile<T, CPLX, true, false, BM, BN, BK, KG, OCC, MODE>(q, s);
+  if (q.b_kfast) return launch_tile<T, CPLX, false, true, BM, BN, BK, KG, OCC, MODE>(q, s);
+  return launch_tile<T, CPLX, false, false, BM, BN, BK, KG, OCC, MODE>(q, s);
 }
 
-template <typename T, bool CPLX, int BM, int BN, int BK, int KG, int PD, int OCC>
+template <typename T, bool CPLX, int BM, int BN, int BK, int KG, int OCC>
 int launch_modes(const Product &q, hipStream_t s)
 {
   if constexpr (!CPLX) {
-    if (q.mode == kVec) return launch_orient<T, CPLX, BM, BN, BK, KG, PD, OCC, kVec>(q, s);
+    if (q.mode == kVec) return launch_orient<T, CPLX, BM, BN, BK, KG, OCC, kVec>(q, s);
   }
-  if (q.mode == kGen) return launch_orient<T, CPLX, BM, BN, BK, KG, PD, OCC, kGen>(q, s);
-  return launch_orient<T, CPLX, BM, BN, BK, KG, PD, OCC, kUni>(q, s);
+  if (q.mode == kGen) return launch_orient<T, CPLX, BM, BN, BK, KG, OCC, kGen>(q, s);
+  return launch_orient<T, CPLX, BM, BN, BK, KG, OCC, kUni>(q, s);
 }
 
 }  // namespace
