@@ -5,7 +5,7 @@
 // Every operand is addressed by two index groups (rows and k, GatherMaps): a
 // matricized operand has one dimension per group, a tensor read in place up
 // to kGatherMaxDims. Offsets are digit arithmetic in the kernel, so a product
-// is one launch with no offset tables.
+// is one launch with no tables in memory.
 //
 // Workgroup: KG groups of 256 threads = 2x2 waves; each wave owns a (BM/2) x
 // (BN/2) sub-tile of 16x16 MFMA blocks. Groups take alternate k-tiles of the
@@ -35,7 +35,14 @@
 // offset for all lanes (mode kVec, kUni), the tile's start is a scalar that
 // steps by carries, the lanes' offsets are loop invariant, and one compare per
 // k-tile decides what the last tile needs. 128x128 tiles reach 64 (FP64) and
-// 127 (FP32) TFLOP/s, 82% of the matrix peak, and C8 64x64 tiles 64.
+// 127 (FP32) TFLOP/s, 82% of the matrix peak, and C8 64x64 tiles 64. Everywhere
+// else (mode kTab) one lane per k-value works out its offsets for 64 k-values
+// ahead into LDS, and the loads add what they read there to their row's offset.
+// With a digit walk per lane and k-value instead, kernel times were, in us:
+// R8 ranks 10, extents 4 (groups of five dimensions) 116 against 72, extents 3
+// 106 against 22; ranks 8, extents 4 53 against 21; R4 the same three 107, 98
+// and 62 against 52, 20 and 16; R4 24^4 29.6 against 24.2; R8 1537 x 1581 x
+// 2491 with its transposes 301 against 291.
 //
 // Operand tiles sit in LDS with k fastest ([row][k], padded rows). Inside a
 // 16-deep k slice, lane group g = lane/16 feeds k = 4g+s at MFMA step s, so a
@@ -60,8 +67,9 @@ struct DevDivisor { uint32_t d, m, s; };
 template <int N>
 struct DevGroup {
   int nd;
-  DevDivisor div[N - 1];   // of every dimension but the last, whose digit is the quotient
+  DevDivisor div[N - 1];   // of every dimension but the last, whose digit is the quotient; 1 beyond those
   int64_t str[N];
+  int64_t last;            // stride of the last dimension
 };
 
 // Kernel arguments. Groups of up to kSmallDims dimensions go in the short form
@@ -94,16 +102,16 @@ enum GemmMode {
   kVec,   // a k-tile starts at one offset for all lanes; k-fast operands load 16-byte vectors, row-fast ones
           // row pairs (whole vectors everywhere: even rows and k-values in eights there)
   kUni,   // the same, element loads
-  kGen,   // runs along k of any length: k-fast lanes step by digits of their own
-  kWide   // kGen with 64-bit offsets (4 GB and more) and groups of up to kGatherMaxDims dimensions
+  kTab    // offsets from tables in LDS: runs along k of any length, groups of up to kGatherMaxDims dimensions,
+          // 64-bit offsets (operands of 4 GB and more)
 };
-constexpr int group_dims(GemmMode mode) { return mode == kWide ? kGatherMaxDims : kSmallDims; }
+constexpr int group_dims(GemmMode mode) { return mode == kTab ? kGatherMaxDims : kSmallDims; }
 
 // A product ready to launch.
 struct Product {
   GemmParams<kGatherMaxDims> p{};
   bool a_kfast = false, b_kfast = false;
-  GemmMode mode = kGen;
+  GemmMode mode = kTab;
 };
 
 int launch_native_r8(const Product &q, int tile, hipStream_t s);
@@ -164,39 +172,42 @@ __device__ __forceinline__ ArgParams<N> &gemm_args_of_kernel()
 template <typename D>
 __device__ __forceinline__ uint32_t gg_div(uint32_t x, const D &f) { return (__umulhi(x, f.m) + x) >> f.s; }
 
-// Element offset of index x of a group (any number of dimensions).
+// Element offset of index x of a group. The long form takes three dimensions at
+// a time: a loop over single ones waits for the arguments of each in turn. The
+// short form's groups mostly have two (R8 32^4: 147 us against 150).
 template <int N>
 __device__ __forceinline__ int64_t group_off(ArgGroup<N> &g, int64_t x)
 {
+  constexpr int STEP = N > kSmallDims ? 3 : 1;
   if (g.nd <= 1) return x * g.str[0];
   uint32_t r = (uint32_t)x;
   int64_t o = 0;
-  for (int j = 0; j + 1 < g.nd; ++j) {
-    const uint32_t q = gg_div(r, g.div[j]);
-    o += (int64_t)(r - q * g.div[j].d) * g.str[j];
-    r = q;
+  for (int j = 0; j + 1 < g.nd; j += STEP) {
+#pragma unroll
+    for (int i = j; i < j + STEP; ++i) {
+      const uint32_t q = gg_div(r, g.div[i]);
+      o += (int64_t)(r - q * g.div[i].d) * g.str[i];
+      r = q;
+    }
   }
-  return o + (int64_t)r * g.str[g.nd - 1];
+  return o + (int64_t)r * g.last;
 }
 
-// A position along a k group, advanced STEP k-values at a time by carries (a
-// few additions; no division, and no read of the arguments unless the group
-// has more than three dimensions). Offsets in bytes. Scalar when the position
-// is the same for all lanes.
-template <typename OffT, int STEP, int ES, int N>
+// A position along a k group of up to three dimensions, the same for all lanes,
+// advanced STEP k-values at a time by carries (a few scalar additions; no
+// division, no read of the arguments). Offsets in bytes.
+template <int STEP, int ES, int N>
 struct KWalk {
-  OffT at, step, s0, fix0, fix1;  // offset, its change per STEP and per k, its corrections on carries
-  uint32_t x, c0, c1, b0, b1, d0, d1;
-  bool far;                       // more than three dimensions
+  int64_t at, step, s0, fix0, fix1;  // offset, its change per STEP and per k, its corrections on carries
+  uint32_t c0, c1, b0, b1, d0, d1;
   __device__ __forceinline__ void init(ArgGroup<N> &g, int64_t x0)
   {
-    x = (uint32_t)x0;
-    far = g.nd > 3;
-    s0 = (OffT)g.str[0] * ES;
-    const OffT s1 = (OffT)g.str[1] * ES, s2 = (OffT)g.str[2] * ES;
+    const uint32_t x = (uint32_t)x0;
+    s0 = g.str[0] * ES;
+    const int64_t s1 = g.str[1] * ES, s2 = g.str[2] * ES;
     d0 = d1 = 0x7fffffffu;
     c0 = c1 = b0 = b1 = 0;
-    step = (OffT)STEP * s0;
+    step = STEP * s0;
     if (g.nd > 1) {
       const uint32_t q0 = gg_div(x, g.div[0]);
       d0 = g.div[0].d;
@@ -206,41 +217,26 @@ struct KWalk {
       if (g.nd > 2) d1 = g.div[1].d;
       c1 = g.nd > 2 ? q0 - gg_div(q0, g.div[1]) * d1 : q0;
       b1 = bq % d1;
-      step = (OffT)b0 * s0 + (OffT)b1 * s1 + (OffT)(bq / d1) * s2;
+      step = b0 * s0 + b1 * s1 + (int64_t)(bq / d1) * s2;
     }
-    fix0 = s1 - (OffT)d0 * s0;
-    fix1 = s2 - (OffT)d1 * s1;
-    at = (OffT)(group_off(g, x0) * ES);
-    if (far) d0 = 0;  // every step "carries", into a fresh decomposition
+    fix0 = s1 - d0 * s0;
+    fix1 = s2 - d1 * s1;
+    at = group_off(g, x0) * ES;
   }
-  __device__ __forceinline__ void carry(ArgGroup<N> &g)
+  __device__ __forceinline__ void advance()
   {
-    if (far) {
-      at = (OffT)(group_off(g, x) * ES);
-      return;
-    }
-    const bool k0 = c0 >= d0;
-    c0 -= k0 ? d0 : 0u;
-    at += k0 ? fix0 : OffT(0);
-    c1 += k0 ? 1u : 0u;
-    const bool k1 = c1 >= d1;
-    c1 -= k1 ? d1 : 0u;
-    at += k1 ? fix1 : OffT(0);
-  }
-  __device__ __forceinline__ void advance(ArgGroup<N> &g)
-  {
-    x += STEP;
     at += step;
     c0 += b0;
     c1 += b1;
-    if (c0 >= d0 || c1 >= d1) carry(g);
-  }
-  __device__ __forceinline__ void next(ArgGroup<N> &g)  // one k-value on
-  {
-    x += 1;
-    at += s0;
-    c0 += 1;
-    if (c0 >= d0) carry(g);
+    if (c0 >= d0 || c1 >= d1) {
+      const bool k0 = c0 >= d0;
+      c0 -= k0 ? d0 : 0u;
+      at += k0 ? fix0 : 0;
+      c1 += k0 ? 1u : 0u;
+      const bool k1 = c1 >= d1;
+      c1 -= k1 ? d1 : 0u;
+      at += k1 ? fix1 : 0;
+    }
   }
 };
 
@@ -254,9 +250,9 @@ __device__ __forceinline__ float flip_sign(float x, uint32_t m) { return __uint_
 // group, one k-tile in KG.
 template <typename T, bool CPLX, bool KF, int BX, int BK, int KG, GemmMode MODE>
 struct Staging {
-  typedef typename std::conditional<MODE == kWide, uint64_t, uint32_t>::type OffT;
+  static constexpr bool TAB = MODE == kTab;
+  typedef typename std::conditional<TAB, uint64_t, uint32_t>::type OffT;
   static constexpr int N = group_dims(MODE);
-  static constexpr bool UNI = MODE == kVec || MODE == kUni;
   static constexpr bool VEC = MODE == kVec && !CPLX;
   static constexpr int NP = CPLX ? 2 : 1;
   static constexpr int KP = BK + (sizeof(T) == 4 ? 4 : 2);  // padded k extent of an LDS row
@@ -278,29 +274,45 @@ struct Staging {
   typedef T LdsRow[KP];
   OffT ro[NR];
   int row, kk;
-  // UNI: at the start of a k-tile (scalar); k-fast otherwise: at this lane's
-  // k-value; row-fast otherwise: at this wave's first k-value (scalar)
-  KWalk<typename std::conditional<UNI || !KF, int64_t, OffT>::type, STEP, ES, N> walk;
+  KWalk<STEP, ES, N> walk;  // at the start of a k-tile
 
-  __device__ __forceinline__ void init(ArgGroup<N> &g, ArgGroup<N> &gk, int64_t r0, int64_t rows, int64_t kbeg, int64_t k0,
-                                       int64_t kend, int tid, int wave)
+  __device__ __forceinline__ void place(int tid, int wave)
   {
     if (KF) { kk = (tid % LR) * VW; row = tid / LR; }
     else { kk = (RV == 1 ? wave : tid / LR) * KV; row = tid % LR * RV; }
+  }
+  __device__ __forceinline__ void init(ArgGroup<N> &g, ArgGroup<N> &gk, int64_t r0, int64_t rows, int64_t kbeg, int64_t k0,
+                                       int64_t kend, int tid, int wave)
+  {
+    place(tid, wave);
     const int64_t last = rows - RV;
-    if (UNI) {
-      walk.init(gk, k0 < kend ? k0 : kbeg);
-      // (element-form row-fast loads add their k offset as a scalar)
-      const OffT lane_k = KF || RV > 1 ? (OffT)(kk * walk.s0) : OffT(0);
+    walk.init(gk, k0 < kend ? k0 : kbeg);
+    // (element-form row-fast loads add their k offset as a scalar)
+    const OffT lane_k = KF || RV > 1 ? (OffT)(kk * walk.s0) : OffT(0);
 #pragma unroll
-      for (int i = 0; i < NR; ++i) ro[i] = (OffT)(group_off(g, min(r0 + row + i * RS, last)) * ES) + lane_k;
-    } else {
-      walk.init(gk, k0 + kk);
+    for (int i = 0; i < NR; ++i) ro[i] = (OffT)(group_off(g, min(r0 + row + i * RS, last)) * ES) + lane_k;
+  }
+  // TAB: rows from the tile's table of row offsets (in bytes; rows past the
+  // edge repeat the last)
+  __device__ __forceinline__ void init_tab(const uint64_t *rows, int tid, int wave)
+  {
+    place(tid, wave);
 #pragma unroll
-      for (int i = 0; i < NR; ++i) ro[i] = (OffT)(group_off(g, min(r0 + row + i * RS, last)) * ES);
+    for (int i = 0; i < NR; ++i) ro[i] = rows[row + i * RS];
+  }
+  // Loads the k-tile whose offsets start at kt (in bytes; k-values past the
+  // end repeat the last), elements as load() does.
+  __device__ __forceinline__ void load_tab(const char *base, const uint64_t *kt, T (&r)[NE * NP]) const
+  {
+    constexpr int J = KF ? 1 : KV;
+#pragma unroll
+    for (int j = 0; j < J; ++j) {
+      const char *p = base + kt[kk + j];
+#pragma unroll
+      for (int i = 0; i < NR; ++i) load_one(p + ro[i], &r[(i * J + j) * W * NP]);
     }
   }
-  // UNI: in the last k-tile, `left` k-values deep, lanes past the end read the
+  // In the last k-tile, `left` k-values deep, lanes past the end read the
   // tile's first k-values (a lane's KV k-values lie on one side of the end)
   __device__ __forceinline__ void clamp_k(int left)
   {
@@ -325,30 +337,19 @@ struct Staging {
   // Loads the k-tile the walk stands at; left: k-values from the tile's start
   // to the end. r[e * NP + q]: element e, component q; k-fast e = row * VW +
   // k, row-fast e = (row group * KV + k) * RV + row.
-  __device__ __forceinline__ void load(const char *base, ArgGroup<N> &gk, int left, T (&r)[NE * NP])
+  __device__ __forceinline__ void load(const char *base, int left, T (&r)[NE * NP]) const
   {
     if constexpr (KF) {
-      if constexpr (UNI) {
-        const char *p = base + walk.at;
+      const char *p = base + walk.at;
 #pragma unroll
-        for (int i = 0; i < NR; ++i) load_one(p + ro[i], &r[i * W * NP]);
-      } else {
-        const OffT here = kk < left ? walk.at : OffT(0);
-#pragma unroll
-        for (int i = 0; i < NR; ++i) load_one(base + (OffT)(ro[i] + here), &r[i * W * NP]);
-      }
+      for (int i = 0; i < NR; ++i) load_one(p + ro[i], &r[i * W * NP]);
     } else {
-      auto sub = walk;
 #pragma unroll
       for (int j = 0; j < KV; ++j) {
-        int64_t o;
-        if (UNI && RV > 1) o = walk.at + (j < left ? j : 0) * walk.s0;
-        else if (UNI) o = walk.at + (kk + j < left ? kk + j : 0) * walk.s0;
-        else o = kk + j < left ? sub.at : 0;
-        const char *p = base + o;
+        const int x = RV > 1 ? j : kk + j;
+        const char *p = base + (walk.at + (x < left ? x : 0) * walk.s0);
 #pragma unroll
         for (int i = 0; i < NR; ++i) load_one(p + ro[i], &r[(i * KV + j) * W * NP]);
-        if (!UNI && j + 1 < KV) sub.next(gk);
       }
     }
   }
@@ -396,13 +397,14 @@ struct Staging {
 };
 
 // C = alpha * acc + beta * C (beta 0 or 1) for the FM x FN blocks of a wave;
-// get(i, j, r, q) is component q of the accumulator's element r.
+// get(i, j, r, q) is component q of the accumulator's element r, rows(x) and
+// cols(x) the offsets of row and column x (clamped into C).
 // Per 16-row block the offsets (-1: outside C), then every C load of the
 // block at once (clamped addresses, no lane-masked branches), one wait, then
 // the stores; a load-add-store per element would wait for each load in turn
 // behind the stores already issued.
-template <typename T, bool CPLX, int FM, int FN, int N, typename Get>
-__device__ __forceinline__ void store_c(ArgParams<N> &p, int64_t m0, int64_t n0, int lane, Get get)
+template <typename T, bool CPLX, int FM, int FN, int N, typename Get, typename Rows, typename Cols>
+__device__ __forceinline__ void store_c(ArgParams<N> &p, int64_t m0, int64_t n0, int lane, Get get, Rows rows, Cols cols)
 {
   constexpr int NP = CPLX ? 2 : 1;
   T *C = static_cast<T *>(p.c);
@@ -412,7 +414,7 @@ __device__ __forceinline__ void store_c(ArgParams<N> &p, int64_t m0, int64_t n0,
 #pragma unroll
   for (int j = 0; j < FN; ++j) {
     const int64_t col = n0 + j * 16 + fr;
-    gcol[j] = col < p.n ? group_off(p.c_col, col) : -1;
+    gcol[j] = col < p.n ? cols(col) : -1;
   }
 #pragma unroll
   for (int i = 0; i < FM; ++i) {
@@ -423,7 +425,7 @@ __device__ __forceinline__ void store_c(ArgParams<N> &p, int64_t m0, int64_t n0,
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int64_t row = m0 + i * 16 + (sizeof(T) == 8 ? fk + 4 * r : fk * 4 + r);
-      const int64_t grow = group_off(p.c_row, min(row, p.m - 1));
+      const int64_t grow = rows(min(row, p.m - 1));
 #pragma unroll
       for (int j = 0; j < FN; ++j) off[j][r] = (row < p.m && gcol[j] >= 0) ? grow + gcol[j] : -1;
     }
@@ -492,6 +494,12 @@ __global__ __launch_bounds__(256 * KG, OCC) void k_gemm_mfma(const GemmParams<gr
   typedef T LdsRow[KP];
   __shared__ __align__(16) T As[KG][2][NP * BM][KP];
   __shared__ __align__(16) T Bs[KG][2][NP * BN][KP];
+  // TAB: offsets in bytes of the tile's rows of A and B and of two chunks of
+  // 64 k-values per k-group, in elements of its rows and columns of C.
+  constexpr bool TAB = MODE == kTab;
+  constexpr int TN = TAB ? 64 : 1, TPC = 64 / BK;  // k-tiles per chunk
+  __shared__ uint64_t t_ab[TAB ? BM + BN : 1], t_k[TAB ? KG : 1][2][2][TN];
+  __shared__ int64_t t_c[TAB ? BM + BN : 1];
 
   const int tid = threadIdx.x & 255, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -524,30 +532,65 @@ __global__ __launch_bounds__(256 * KG, OCC) void k_gemm_mfma(const GemmParams<gr
 #pragma unroll
       for (int j = 0; j < FN; ++j) acc[q][i][j] = AccT{0, 0, 0, 0};
 
+  if constexpr (TAB) {
+    for (int x = threadIdx.x; x < 2 * (BM + BN); x += 256 * KG) {
+      const int y = x % (BM + BN);
+      const bool row = y < BM;
+      const int64_t at = row ? min(m0 + y, p.m - 1) : min(n0 + y - BM, p.n - 1);
+      if (x < BM + BN) t_ab[y] = (uint64_t)((row ? group_off(p.a_row, at) : group_off(p.b_row, at)) * SA::ES);
+      else t_c[y] = row ? group_off(p.c_row, at) : group_off(p.c_col, at);
+    }
+    __syncthreads();
+  }
   const int fr = lane & 15, fg = (lane >> 4) * 4;
   const int nt = (int)((kend - kbeg + BK * KG - 1) / (BK * KG));  // steps: k-tiles per group
   if (nt > 0) {
     SA sa;
     SB sb;
     const int64_t k0 = kbeg + grp * BK;
-    sa.init(p.a_row, p.a_k, m0, p.m, kbeg, k0, kend, tid, wave);
-    sb.init(p.b_row, p.b_k, n0, p.n, kbeg, k0, kend, tid, wave);
+    constexpr int ES = SA::ES;
+    auto k_table = [&](int c) {  // chunk c of this k-group: wave 0 for A, wave 1 for B
+      if (wave > 1) return;
+      const int64_t x = min(k0 + (int64_t)(c * TPC + lane / BK) * (BK * KG) + lane % BK, kend - 1);
+      const int64_t o = wave == 0 ? group_off(p.a_k, x) : group_off(p.b_k, x);
+      t_k[TAB ? grp : 0][wave][c & 1][TAB ? lane : 0] = (uint64_t)(o * ES);
+    };
+    if constexpr (TAB) {
+      k_table(0);
+      __syncthreads();
+      sa.init_tab(t_ab, tid, wave);
+      sb.init_tab(t_ab + BM, tid, wave);
+    } else {
+      sa.init(p.a_row, p.a_k, m0, p.m, kbeg, k0, kend, tid, wave);
+      sb.init(p.b_row, p.b_k, n0, p.n, kbeg, k0, kend, tid, wave);
+    }
+    int lt = 0;  // TAB: k-tiles loaded
     // k-values from the next k-tile's start to the end: of the tile to load
-    // (uniform walks stay at the last tile), of the tile to store
-    int left_s = (int)(kend - k0), left_l = SA::UNI && left_s <= 0 ? (int)min(kend - kbeg, (int64_t)BK) : left_s;
-    if (SA::UNI && left_l < BK) {
+    // (walks stay at the last tile), of the tile to store
+    int left_s = (int)(kend - k0), left_l = left_s <= 0 ? (int)min(kend - kbeg, (int64_t)BK) : left_s;
+    if (!TAB && left_l < BK) {
       sa.clamp_k(left_l);
       sb.clamp_k(left_l);
     }
     T ra[SA::NE * NP], rb[SB::NE * NP];
     auto load = [&]() {  // the next k-tile
-      sa.load(A, p.a_k, left_l, ra);
-      sb.load(B, p.b_k, left_l, rb);
-      if (!SA::UNI || left_l > BK * KG) {
+      if constexpr (TAB) {
+        const int c = lt / TPC;
+        // the chunk after this one, over the one before (the last read of
+        // which lies a barrier back)
+        if (lt % TPC == 0) k_table(c + 1);
+        sa.load_tab(A, &t_k[grp][0][c & 1][lt % TPC * BK], ra);
+        sb.load_tab(B, &t_k[grp][1][c & 1][lt % TPC * BK], rb);
+        ++lt;
+        return;
+      }
+      sa.load(A, left_l, ra);
+      sb.load(B, left_l, rb);
+      if (left_l > BK * KG) {
         left_l -= BK * KG;
-        sa.walk.advance(p.a_k);
-        sb.walk.advance(p.b_k);
-        if (SA::UNI && left_l < BK) {
+        sa.walk.advance();
+        sb.walk.advance();
+        if (left_l < BK) {
           sa.clamp_k(left_l);
           sb.clamp_k(left_l);
         }
@@ -649,7 +692,9 @@ __global__ __launch_bounds__(256 * KG, OCC) void k_gemm_mfma(const GemmParams<gr
   }
   const int64_t mw = m0 + wm + oi * 16, nw = n0 + wn + oj * 16;
   if (!split) {
-    store_c<T, CPLX, OM, ON>(p, mw, nw, lane, [&](int i, int j, int r, int q) { return acc[q][i][j][r]; });
+    store_c<T, CPLX, OM, ON>(p, mw, nw, lane, [&](int i, int j, int r, int q) { return acc[q][i][j][r]; },
+                             [&](int64_t x) { return TAB ? t_c[x - m0] : group_off(p.c_row, x); },
+                             [&](int64_t x) { return TAB ? t_c[BM + (x - n0)] : group_off(p.c_col, x); });
     return;
   }
   const PartLayout<BM, BN> pl(p, tile, m0, n0);
@@ -737,6 +782,7 @@ GemmParams<N> shortened(const GemmParams<kGatherMaxDims> &f)
       d.nd = g.nd;
       for (int j = 0; j < N; ++j) d.str[j] = g.str[j];
       for (int j = 0; j + 1 < N; ++j) d.div[j] = g.div[j];
+      d.last = g.last;
     };
     group(p.a_row, f.a_row); group(p.a_k, f.a_k);
     group(p.b_row, f.b_row); group(p.b_k, f.b_k);
@@ -775,7 +821,7 @@ int launch_modes(const Product &q, hipStream_t s)
   if constexpr (!CPLX) {
     if (q.mode == kVec) return launch_orient<T, CPLX, BM, BN, BK, KG, OCC, kVec>(q, s);
   }
-  if (q.mode == kGen) return launch_orient<T, CPLX, BM, BN, BK, KG, OCC, kGen>(q, s);
+  if (q.mode == kTab) return launch_orient<T, CPLX, BM, BN, BK, KG, OCC, kTab>(q, s);
   return launch_orient<T, CPLX, BM, BN, BK, KG, OCC, kUni>(q, s);
 }
 

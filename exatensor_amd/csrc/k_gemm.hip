@@ -734,7 +734,14 @@ bool gather_vec_loads(int es, bool kfast, const GatherGroup &row, const GatherGr
   return x.nd > 0 && x.str[0] == 1 && x.ext[0] % (kfast ? std::max(16 / es, 1) : 2) == 0 && (kfast || k % 8 == 0);
 }
 
-bool gather_uniform_k(int kind, const GatherGroup &kg) { return kg.nd <= 1 || kg.ext[0] % tile_shape(kind, 0).bk == 0; }
+bool gather_uniform_k(int kind, const GatherMaps &mp)
+{
+  for (const GatherGroup *x : {&mp.a_row, &mp.a_k, &mp.b_row, &mp.b_k, &mp.c_row, &mp.c_col})
+    if (x->nd > kSmallDims) return false;
+  for (const GatherGroup *x : {&mp.a_k, &mp.b_k})
+    if (x->nd > 3 || (x->nd > 1 && x->ext[0] % tile_shape(kind, 0).bk != 0)) return false;
+  return true;
+}
 
 // Large complex products in native precision run realified through the real
 // 128x128 kernels (which re-read operands from L2 half as often as the 64x64
@@ -874,6 +881,8 @@ FullGroup dev_group(const GatherGroup &g)
       d.div[j] = DevDivisor{f.d, f.m, f.s};
     }
   }
+  for (int j = std::max(g.nd - 1, 0); j + 1 < kGatherMaxDims; ++j) d.div[j] = DevDivisor{1, 0, 0};
+  if (g.nd > 0) d.last = g.str[g.nd - 1];
   return d;
 }
 
@@ -881,7 +890,7 @@ FullGroup line_group(int64_t stride)
 {
   FullGroup d{};
   d.nd = 1;
-  d.str[0] = stride;
+  d.str[0] = d.last = stride;
   return d;
 }
 
@@ -889,7 +898,6 @@ FullGroup line_group(int64_t stride)
 // tile choice `tile`, cutting K as the workspace allows.
 int launch_product(Product &q, const GemmArgs &g, int tile, void *ws, size_t ws_bytes, hipStream_t s)
 {
-  if (q.mode == kWide) tile = 0;  // 64-bit offsets: one tile shape
   const TileShape ts = tile_shape(g.kind, tile);
   const int64_t tm = ((int64_t)g.m + ts.bm - 1) / ts.bm, tn = ((int64_t)g.n + ts.bn - 1) / ts.bn;
   if (tm >= (1ll << 31) || tn >= (1ll << 31) || tm * tn >= (1ll << 31) - 65536) return TALSH_LIMIT_EXCEEDED;
@@ -965,7 +973,7 @@ int launch_matrix(GemmArgs g, int tile, void *ws, size_t ws_bytes, hipStream_t s
   const int es = kind_size(g.kind);
   const int64_t lim = (1ll << 31) - 1, bytes = std::max(p.m, p.n) * p.k * es;
   const bool off32 = p.m <= lim && p.n <= lim && p.k <= lim && bytes < (1ll << 32);
-  q.mode = !off32 ? kWide
+  q.mode = !off32 ? kTab
            : gemm_vec_loads(es, g.a_kfast, g.m, g.k) && gemm_vec_loads(es, g.b_kfast, g.n, g.k) ? kVec : kUni;
   exchange(q, g);
   return launch_product(q, g, tile, ws, ws_bytes, s);
@@ -1105,11 +1113,7 @@ int launch_gemm_gather(const GemmArgs &args, const GatherMaps &mp, void *ws, siz
   const size_t lim = INT32_MAX;
   const bool off32 = g.m <= lim && g.n <= lim && g.k <= lim && (last[0] + last[1] + 1) * es < (1ll << 32) &&
                      (last[2] + last[3] + 1) * es < (1ll << 32);
-  bool small = true;
-  for (int t = 0; t < 6; ++t) small = small && grp[t]->nd <= kSmallDims;
-  q.mode = kGen;
-  if (!off32 || !small) q.mode = kWide;
-  else if (gather_uniform_k(g.kind, mp.a_k) && gather_uniform_k(g.kind, mp.b_k))
+  if (off32 && gather_uniform_k(g.kind, mp))
     q.mode = gather_vec_loads(es, g.a_kfast, mp.a_row, mp.a_k, g.k) && gather_vec_loads(es, g.b_kfast, mp.b_row, mp.b_k, g.k)
                  ? kVec : kUni;
   const int tile = resolved_tile(g);

@@ -8,11 +8,9 @@ namespace xt {
 int launch_native_cx(const Product &q, int kind, int tile, hipStream_t s)
 {
   if (kind == C8) {
-    if (q.mode == kWide) return launch_orient<double, true, 64, 64, 16, 1, 2, kWide>(q, s);
     if (tile == 1) return launch_modes<double, true, 64, 64, 16, 2, 2>(q, s);
     return launch_modes<double, true, 64, 64, 16, 1, 2>(q, s);
   }
-  if (q.mode == kWide) return launch_orient<float, true, 64, 64, 16, 1, 2, kWide>(q, s);
   if (tile == 1) return launch_modes<float, true, 64, 64, 16, 2, 2>(q, s);
   return launch_modes<float, true, 64, 64, 16, 1, 2>(q, s);
 }

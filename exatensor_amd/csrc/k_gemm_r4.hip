@@ -7,7 +7,6 @@ namespace xt {
 
 int launch_native_r4(const Product &q, int tile, hipStream_t s)
 {
-  if (q.mode == kWide) return launch_orient<float, false, 128, 128, 32, 1, 2, kWide>(q, s);
   if (tile == 2) return launch_modes<float, false, 64, 64, 32, 1, 4>(q, s);
   if (tile == 1) return launch_modes<float, false, 64, 64, 32, 4, 4>(q, s);
   return launch_modes<float, false, 128, 128, 32, 1, 2>(q, s);

@@ -7,7 +7,6 @@ namespace xt {
 
 int launch_native_r8(const Product &q, int tile, hipStream_t s)
 {
-  if (q.mode == kWide) return launch_orient<double, false, 128, 128, 16, 1, 2, kWide>(q, s);
   if (tile == 2) return launch_modes<double, false, 64, 64, 16, 1, 4>(q, s);
   if (tile == 1) return launch_modes<double, false, 64, 64, 16, 4, 4>(q, s);
   return launch_modes<double, false, 128, 128, 16, 1, 2>(q, s);

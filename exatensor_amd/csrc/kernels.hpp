@@ -116,11 +116,12 @@ bool split3_gather_ok(const GatherMaps &maps, size_t m, size_t n, size_t k);
 int launch_split3_gather(const GemmArgs &g, const GatherMaps &maps, void *ws, size_t ws_bytes, hipStream_t s);
 // What the native kernels' loads need of an operand (real kinds, element size
 // es): whole 16-byte vectors along k, or row pairs with the k-values in
-// eights; for a gathered operand also, that a k-tile starts at one offset for
-// all lanes (it does not cross a digit of the first contracted dimension).
+// eights; for a gathered product also, that a k-tile starts at one offset for
+// all lanes (it does not cross a digit of the first contracted dimension, and
+// the groups are short enough for the walk along k), else by tables in LDS.
 bool gemm_vec_loads(int es, bool kfast, size_t rows, size_t k);
 bool gather_vec_loads(int es, bool kfast, const GatherGroup &row, const GatherGroup &kg, size_t k);
-bool gather_uniform_k(int kind, const GatherGroup &kg);
+bool gather_uniform_k(int kind, const GatherMaps &maps);
 // Fixed per-GPU scratch of the allocation-free product entry point: a
 // file-scope device array in k_gemm.hip (64 MiB, held by every GPU the
 // library runs on until the process ends). gemm_noalloc_scratch returns its

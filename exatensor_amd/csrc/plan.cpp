@@ -399,7 +399,7 @@ int plan_candidates(const std::vector<int> &dig, int dr, int lr, int rr, const s
       f[36] = !cplx && gather_vec_loads(es, c.a_kfast, c.maps.a_row, c.maps.a_k, (size_t)gk);
       f[37] = !cplx && gather_vec_loads(es, c.b_kfast, c.maps.b_row, c.maps.b_k, (size_t)gk);
       f[44] = 1.f;  // fused gather
-      f[45] = gather_uniform_k(kind, c.maps.a_k) && gather_uniform_k(kind, c.maps.b_k);
+      f[45] = gather_uniform_k(kind, c.maps);
       f[46] = c.maps.c_row.nd > 0 && c.maps.c_row.str[0] == 1;  // result rows along D's stride-1 index
       // contiguous run along each operand's staging direction, and the
       // stride between its staged elements when that is not 1
