@@ -641,16 +641,18 @@ __global__ __launch_bounds__(256 * KG, OCC) void k_gemm_mfma(const GemmParams<gr
     };
     load();
     store(0);
-    load();
+    if (nt > 1) load();
     __syncthreads();
-    // (past the last k-tile, stores and loads go on harmlessly: into the
-    // buffer that is not read any more, from addresses in range)
-    for (int t = 0, buf = 0; t < nt; ++t, buf ^= 1) {
+    // (the loop's last load, past the last k-tile, is from addresses in range
+    // and is not used)
+    int buf = 0;
+    for (int t = 1; t < nt; ++t, buf ^= 1) {
       store(buf ^ 1);
       load();
       compute(buf);
       __syncthreads();
     }
+    compute(buf);
   }
 
   // blocks that this wave finishes: all of its own with one group, else a
@@ -669,6 +671,7 @@ __global__ __launch_bounds__(256 * KG, OCC) void k_gemm_mfma(const GemmParams<gr
       return h + ((g * 4 + wave) * (NB / 2) + v % (NB / 2)) * 64 + lane;
     };
     auto at = [&](int q, int i, int j, int r) { return ((i * FN + j) * NP + q) * 4 + r; };
+    __syncthreads();  // the last k-tile is multiplied
 #pragma unroll
     for (int q = 0; q < NP; ++q)
 #pragma unroll

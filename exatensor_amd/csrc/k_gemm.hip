@@ -667,6 +667,8 @@ TileShape tile_shape(int kind, int tile)
 
 bool native_real(const GemmArgs &g) { return g.kind == R8 || (g.kind == R4 && g.r4mode == R4Mode::kNativeF32); }
 
+constexpr int64_t kSplitMinK = 256;  // shortest K that is cut
+
 // How a product's tiles are cut along K: tiles [0, full) run whole, the later
 // ones in `parts` pieces of kchunk k-values.
 struct SplitGeom {
@@ -693,7 +695,7 @@ SplitGeom split_geom(const GemmArgs &g, const TileShape &ts, int cus, size_t bud
   const bool cplx = g.kind == C8 || g.kind == C4, dp = g.kind == R8 || g.kind == C8;
   const int64_t round = (ts.groups > 1 ? 1 : 2) * (int64_t)cus;
   const int64_t full = G.tiles / round * round, rem = G.tiles - full;
-  if (rem == 0 || k < 256 || k > kMaxDepth) return G;
+  if (rem == 0 || k < kSplitMinK || k > kMaxDepth) return G;
   // microseconds of one tile on a CU of its own at 80% of its matrix rate
   const double tau = (cplx ? 8.0 : 2.0) * ts.bm * ts.bn * (double)k / (0.8 * (dp ? 78.6e6 : 157.3e6) / 256.0);
   auto cost = [&](int64_t parts) {
@@ -761,13 +763,19 @@ size_t realified_bytes(const GemmArgs &g)
 }
 
 // Tile choice of the kernels: a caller's, or the default; complex kinds have
-// one choice, their two forms are told apart here (two k-groups per workgroup
-// when the tiles do not give every CU two workgroups).
+// one choice, their two forms are told apart here: two k-groups per workgroup
+// when the tiles do not give every CU two workgroups and K is deep enough. Two
+// groups share at least 64 k-values (C8 64x64, two groups and one: k 8 12 and 9
+// us, 48 17 and 14, 64 17 and 17, 128 25 and 26, 512 76 and 81); where a CU
+// would run its two workgroups one after the other they need K deep enough for
+// a cut of the last round besides (C8 1280x960: k 8 24 and 14 us, 160 60 and 52;
+// 512, in pieces, 109 and 141; C4 14 and 11, 33 and 32, 59 and 81).
 int resolved_tile(const GemmArgs &g)
 {
   if (g.kind == C8 || g.kind == C4) {
     const int64_t tiles = (int64_t)((g.m + 63) / 64) * (int64_t)((g.n + 63) / 64);
-    return tiles < 2 * (int64_t)current_cus() ? 1 : 0;
+    const int64_t cus = current_cus();
+    return g.k > 64 && (tiles <= cus || (tiles < 2 * cus && g.k >= kSplitMinK)) ? 1 : 0;
   }
   return g.tile < 0 ? gemm_default_tile(g.kind, g.r4mode, g.m, g.n, g.k) : g.tile;
 }
