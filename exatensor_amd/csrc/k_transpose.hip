@@ -411,17 +411,29 @@ __global__ __launch_bounds__(kTNT) void k_permute_runs(const W *__restrict__ in,
       q = n;
     }
     out_off[k] = oo;
+    uint32_t r[VEC], sl[VEC];
 #pragma unroll
     for (int e = 0; e < VEC; ++e) {
-      uint32_t r = s + e, sl = base;
-      for (int j = 0; j < p.nrun; ++j) {
-        const uint32_t n = fdiv(r, p.t_run[j]);
-        sl += (r - n * p.t_run[j].d) * p.ls_run[j];
-        r = n;
+      r[e] = s + e;
+      sl[e] = base;
+    }
+    // (dimensions outside, elements inside: one wait for the arguments of a
+    // dimension, not one per element)
+    for (int j = 0; j < p.nrun; ++j) {
+      const DevDiv t = p.t_run[j];
+      const uint32_t ls = p.ls_run[j];
+#pragma unroll
+      for (int e = 0; e < VEC; ++e) {
+        const uint32_t n = fdiv(r[e], t);
+        sl[e] += (r[e] - n * t.d) * ls;
+        r[e] = n;
       }
-      sl += fdiv(sl, p.pad);
-      if (e & 1) sslot[k][e / 2] |= sl << 16;
-      else sslot[k][e / 2] = sl;
+    }
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) {
+      const uint32_t x = sl[e] + fdiv(sl[e], p.pad);
+      if (e & 1) sslot[k][e / 2] |= x << 16;
+      else sslot[k][e / 2] = x;
     }
   }
   // Place `at` of the grid-stride order -> tile: each XCD (workgroups go round
