@@ -44,10 +44,12 @@ constexpr int kMaxEPT = 8;         // tile vectors per thread (more cost occupan
 constexpr int kTiledPerCU = 2;     // persistent workgroups per CU (16 waves)
 constexpr int kTileMaxBytes = 65536;  // LDS tile (before padding)
 constexpr long kTileMinVol = 8192;    // tiles are grown to at least this many elements
-// Tiles of the run form: at most four vectors per thread (eight hold 76
-// registers per thread in R4 and keep a workgroup's loads and stores apart for
-// longer: R4 37x29x41x23x31 88 us with 64 KB tiles, 60 with these, 67 with 26
-// KB; 4001 x 4003 transposed 53, 33 and 34), grown to 16 KB.
+// Tiles of the run form: at most kRunEPT vectors per thread, counted with the
+// partial last one of every run (eight hold 76 registers per thread in R4 and
+// keep a workgroup's loads and stores apart for longer: R4 37x29x41x23x31 88 us
+// with 64 KB tiles, 60 with these, 67 with 26 KB; 4001 x 4003 transposed 53, 33
+// and 34), grown to 16 KB.
+constexpr int kRunEPT = 4;
 constexpr long kRunTileMaxBytes = 34 << 10, kRunTileMinBytes = 16 << 10;
 constexpr int kLine = 128;            // cache line bytes
 
@@ -816,24 +818,32 @@ int tile_vec(const Fused &f, const TilePlan &tp, int es)
 }
 
 // Tile of the run form: an input-minor and an output-minor group of
-// dimensions, each walked until it covers `target` elements; a dimension that
+// dimensions, each walked until it covers `target` elements. A dimension that
 // is cut gets tiles of nearly equal extent (the last one overlaps its
-// neighbour by less than the number of tiles).
-int balanced(int ext, long need)
+// neighbour by less than the number of tiles); one of sixteen tiles and more
+// gets whole lines (a step is `run` elements) where they are at most a quarter
+// longer: its last tile repeats a sixteenth at most, and with 65 columns instead
+// of 64 every line between two tiles is read twice and written in parts (C4
+// 2350648 x 16 transposed 136 us with 65, 118 with 64).
+int cut_extent(int ext, long need, long run, int es)
 {
   if (need >= ext) return ext;
+  long step = kLine / es;
+  while (step > 1 && run % 2 == 0) { step /= 2; run /= 2; }
+  const long lines = (need + step - 1) / step * step;
+  if (4 * lines <= 5 * need && ext >= 16 * lines) return (int)lines;
   const int n = std::max<int>(1, (int)(ext / need));  // tiles of at least `need`
   return (ext + n - 1) / n;
 }
 
-bool plan_runs(int es, const Fused &f, int cus, int vec, int max_ept, Planned &pl, bool choose_pad)
+bool plan_runs(int es, const Fused &f, int cus, int vec, Planned &pl, bool choose_pad)
 {
   const int r = f.rank;
   std::vector<int> n2o(r);
   for (int i = 0; i < r; ++i) n2o[f.o2n[i]] = i;
   uint64_t vol = 1;
   for (int e : f.ext) vol *= (uint64_t)e;
-  const long max_vol = std::min<long>((long)kTNT * max_ept * vec, kRunTileMaxBytes / es);
+  const long max_vol = kRunTileMaxBytes / es;
   const long min_vol =
       std::min<long>({max_vol, kRunTileMinBytes / es, std::max<long>(1024, (long)(vol / (4 * (uint64_t)std::max(cus, 1))))});
   std::vector<int> t(r);
@@ -842,11 +852,24 @@ bool plan_runs(int es, const Fused &f, int cus, int vec, int max_ept, Planned &p
     for (int x : t) v *= std::max(x, 1);
     return v;
   };
+  // whether the tile's vectors, those at the runs' ends included, fit the threads
+  auto fits = [&] {
+    for (bool in : {true, false}) {
+      long run = 1;
+      for (int q = 0; q < r; ++q) {
+        const int i = in ? q : n2o[q];
+        run *= std::max(t[i], 1);
+        if (t[i] < f.ext[i]) break;
+      }
+      if ((run + vec - 1) / vec * (volume() / run) > (long)kTNT * kRunEPT) return false;
+    }
+    return volume() <= max_vol;
+  };
   auto walk = [&](long target, bool in) {
     long run = 1;
     for (int q = 0; q < r; ++q) {
       const int i = in ? q : n2o[q];
-      const int want = balanced(f.ext[i], (target + run - 1) / run);
+      const int want = cut_extent(f.ext[i], (target + run - 1) / run, run, es);
       t[i] = std::max(t[i], want);
       run *= t[i];
       if (t[i] < f.ext[i] || run >= target) break;
@@ -856,7 +879,7 @@ bool plan_runs(int es, const Fused &f, int cus, int vec, int max_ept, Planned &p
     std::fill(t.begin(), t.end(), 0);
     walk(target, true);
     walk(target, false);
-    return volume() <= max_vol && std::count_if(t.begin(), t.end(), [](int x) { return x > 0; }) <= kMaxTileDims;
+    return fits() && std::count_if(t.begin(), t.end(), [](int x) { return x > 0; }) <= kMaxTileDims;
   };
   // (tiles of at most a sixth of a CU's share: a 31 MB body in 1.5 tiles per
   // resident workgroup took 48 us, in 6 smaller ones 30)
@@ -867,16 +890,22 @@ bool plan_runs(int es, const Fused &f, int cus, int vec, int max_ept, Planned &p
   // grow towards min_vol, alternating sides
   for (int side = 0, stuck = 0; volume() < min_vol && stuck < 2; side ^= 1) {
     int dim = -1;
+    long run = 1;
     for (int q = 0; q < r && dim < 0; ++q) {
       const int i = side == 0 ? q : n2o[q];
       if (t[i] < f.ext[i]) dim = i;
+      else run *= t[i];
     }
     if (dim < 0) { ++stuck; continue; }
-    const int old = t[dim], want = balanced(f.ext[dim], std::max(2l, 2l * old));
-    if (volume() / std::max(old, 1) * want > std::min(max_vol, share)) { ++stuck; continue; }
-    if (old == 0 && std::count_if(t.begin(), t.end(), [](int x) { return x > 0; }) == kMaxTileDims) { ++stuck; continue; }
+    const int old = t[dim];
+    t[dim] = cut_extent(f.ext[dim], std::max(2l, 2l * old), run, es);
+    if (!fits() || volume() > share ||
+        std::count_if(t.begin(), t.end(), [](int x) { return x > 0; }) > kMaxTileDims) {
+      t[dim] = old;
+      ++stuck;
+      continue;
+    }
     stuck = 0;
-    t[dim] = want;
   }
   RunParams &P = pl.rp;
   std::memset(&P, 0, sizeof(P));
@@ -959,7 +988,7 @@ bool plan_runs(int es, const Fused &f, int cus, int vec, int max_ept, Planned &p
   const uint32_t nv = std::max(P.vecs_i, P.vecs_o);
   int ept = 1;
   while ((uint32_t)ept * kTNT < nv) ept *= 2;
-  if (ept > max_ept) return false;
+  if (ept > kRunEPT) return false;
   pl.ept = ept;
   pl.vec = vec;
   pl.wide = vol >= (1ull << 32);
@@ -1025,7 +1054,7 @@ int plan(int es, int rank, const int *dims, const int *o2n, Planned &pl, int cus
                      tile_vec(f, tp, es) * es == 16 && (long)tp.in_run * es % kLine == 0 &&
                      (long)tp.out_run * es % kLine == 0;
   if (!tiled) {
-    pl.path = plan_runs(es, f, cus, 16 / es, kMaxEPT, pl, choose_pad) ? 3 : 2;
+    pl.path = plan_runs(es, f, cus, 16 / es, pl, choose_pad) ? 3 : 2;
     return 0;
   }
   pl.path = 1;
@@ -1181,13 +1210,6 @@ int launch_runs_o(const Planned &pl, const void *in, void *out, double fr, doubl
                        a, b, pl.rp, fr, fi);                                                                    \
     break;
     XT_CASE(1) XT_CASE(2) XT_CASE(4)
-  case 8:
-    if constexpr (KIND == 0) {
-      hipLaunchKernelGGL((k_permute_runs<W, VEC, 8, CONJ, OffT, 0>), dim3(pl.grid), dim3(kTNT), pl.lds_bytes, s, a, b,
-                         pl.rp, fr, fi);
-      break;
-    }
-    return TALSH_FAILURE;
 #undef XT_CASE
   default: return TALSH_FAILURE;
   }
@@ -1280,9 +1302,7 @@ Planned planned(int es, int rank, const int *dims, const int *o2n, const void *i
   Planned pl;
   if (add) {
     pl.f = fuse_dims(rank, dims, o2n);
-    // (half the vectors per thread: the accumulating form holds D's as well)
-    if (pl.f.rank < 2 || pl.f.rank > kMaxGridDims || !plan_runs(es, pl.f, compute_units(), 16 / es, kMaxEPT / 2, pl, true))
-      pl.path = 2;
+    if (pl.f.rank < 2 || pl.f.rank > kMaxGridDims || !plan_runs(es, pl.f, compute_units(), 16 / es, pl, true)) pl.path = 2;
   } else {
     plan(es, rank, dims, o2n, pl, compute_units(), align);
   }
