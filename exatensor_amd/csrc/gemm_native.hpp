@@ -68,8 +68,7 @@ template <int N>
 struct DevGroup {
   int nd;
   DevDivisor div[N - 1];   // of every dimension but the last, whose digit is the quotient; 1 beyond those
-  int64_t str[N];
-  int64_t last;            // stride of the last dimension
+  int64_t str[N];          // in the long form, str[N - 1] is the last dimension's
 };
 
 // Kernel arguments. Groups of up to kSmallDims dimensions go in the short form
@@ -190,7 +189,7 @@ __device__ __forceinline__ int64_t group_off(ArgGroup<N> &g, int64_t x)
       r = q;
     }
   }
-  return o + (int64_t)r * g.last;
+  return o + (int64_t)r * g.str[N > kSmallDims ? N - 1 : g.nd - 1];
 }
 
 // A position along a k group of up to three dimensions, the same for all lanes,
@@ -785,7 +784,6 @@ GemmParams<N> shortened(const GemmParams<kGatherMaxDims> &f)
       d.nd = g.nd;
       for (int j = 0; j < N; ++j) d.str[j] = g.str[j];
       for (int j = 0; j + 1 < N; ++j) d.div[j] = g.div[j];
-      d.last = g.last;
     };
     group(p.a_row, f.a_row); group(p.a_k, f.a_k);
     group(p.b_row, f.b_row); group(p.b_k, f.b_k);

@@ -890,7 +890,7 @@ FullGroup dev_group(const GatherGroup &g)
     }
   }
   for (int j = std::max(g.nd - 1, 0); j + 1 < kGatherMaxDims; ++j) d.div[j] = DevDivisor{1, 0, 0};
-  if (g.nd > 0) d.last = g.str[g.nd - 1];
+  if (g.nd > 0) d.str[kGatherMaxDims - 1] = g.str[g.nd - 1];
   return d;
 }
 
@@ -898,7 +898,7 @@ FullGroup line_group(int64_t stride)
 {
   FullGroup d{};
   d.nd = 1;
-  d.str[0] = d.last = stride;
+  d.str[0] = stride;
   return d;
 }
 
