@@ -80,6 +80,7 @@ struct GemmParams {
   const void *b;
   void *c;
   int64_t m, n, k;
+  int64_t a_line, b_line;    // row stride of an operand whose rows are one dimension, else 0
   int64_t k0;                // this launch covers k-values [k0, k), at most kMaxDepth
   double alpha_re, alpha_im;
   int beta_zero;
@@ -102,7 +103,7 @@ enum GemmMode {
           // row pairs (whole vectors everywhere: even rows and k-values in eights there)
   kUni,   // the same, element loads
   kTab    // offsets from tables in LDS: runs along k of any length, groups of up to kGatherMaxDims dimensions,
-          // 64-bit offsets (operands of 4 GB and more)
+          // 64-bit offsets
 };
 constexpr int group_dims(GemmMode mode) { return mode == kTab ? kGatherMaxDims : kSmallDims; }
 
@@ -280,16 +281,21 @@ struct Staging {
     if (KF) { kk = (tid % LR) * VW; row = tid / LR; }
     else { kk = (RV == 1 ? wave : tid / LR) * KV; row = tid % LR * RV; }
   }
-  __device__ __forceinline__ void init(ArgGroup<N> &g, ArgGroup<N> &gk, int64_t r0, int64_t rows, int64_t kbeg, int64_t k0,
-                                       int64_t kend, int tid, int wave)
+  __device__ __forceinline__ void init(ArgGroup<N> &g, ArgGroup<N> &gk, int64_t line, int64_t r0, int64_t rows,
+                                       int64_t kbeg, int64_t k0, int64_t kend, int tid, int wave)
   {
     place(tid, wave);
     const int64_t last = rows - RV;
     walk.init(gk, k0 < kend ? k0 : kbeg);
+    // lanes hold offsets from the tile's first row where rows are one
+    // dimension (line: its stride, else 0), so that 32 bits do for operands of
+    // any size
+    const int64_t first = r0 * line;
+    walk.at += first * ES;
     // (element-form row-fast loads add their k offset as a scalar)
     const OffT lane_k = KF || RV > 1 ? (OffT)(kk * walk.s0) : OffT(0);
 #pragma unroll
-    for (int i = 0; i < NR; ++i) ro[i] = (OffT)(group_off(g, min(r0 + row + i * RS, last)) * ES) + lane_k;
+    for (int i = 0; i < NR; ++i) ro[i] = (OffT)((group_off(g, min(r0 + row + i * RS, last)) - first) * ES) + lane_k;
   }
   // TAB: rows from the tile's table of row offsets (in bytes; rows past the
   // edge repeat the last)
@@ -560,8 +566,8 @@ __global__ __launch_bounds__(256 * KG, OCC) void k_gemm_mfma(const GemmParams<gr
       sa.init_tab(t_ab, tid, wave);
       sb.init_tab(t_ab + BM, tid, wave);
     } else {
-      sa.init(p.a_row, p.a_k, m0, p.m, kbeg, k0, kend, tid, wave);
-      sb.init(p.b_row, p.b_k, n0, p.n, kbeg, k0, kend, tid, wave);
+      sa.init(p.a_row, p.a_k, p.a_line, m0, p.m, kbeg, k0, kend, tid, wave);
+      sb.init(p.b_row, p.b_k, p.b_line, n0, p.n, kbeg, k0, kend, tid, wave);
     }
     int lt = 0;  // TAB: k-tiles loaded
     // k-values from the next k-tile's start to the end: of the tile to load
@@ -640,18 +646,16 @@ __global__ __launch_bounds__(256 * KG, OCC) void k_gemm_mfma(const GemmParams<gr
     };
     load();
     store(0);
-    if (nt > 1) load();
+    load();
     __syncthreads();
-    // (the loop's last load, past the last k-tile, is from addresses in range
-    // and is not used)
-    int buf = 0;
-    for (int t = 1; t < nt; ++t, buf ^= 1) {
+    // (past the last k-tile, stores and loads go on harmlessly: into the
+    // buffer that is not read any more, from addresses in range)
+    for (int t = 0, buf = 0; t < nt; ++t, buf ^= 1) {
       store(buf ^ 1);
       load();
       compute(buf);
       __syncthreads();
     }
-    compute(buf);
   }
 
   // blocks that this wave finishes: all of its own with one group, else a
@@ -670,7 +674,6 @@ __global__ __launch_bounds__(256 * KG, OCC) void k_gemm_mfma(const GemmParams<gr
       return h + ((g * 4 + wave) * (NB / 2) + v % (NB / 2)) * 64 + lane;
     };
     auto at = [&](int q, int i, int j, int r) { return ((i * FN + j) * NP + q) * 4 + r; };
-    __syncthreads();  // the last k-tile is multiplied
 #pragma unroll
     for (int q = 0; q < NP; ++q)
 #pragma unroll
@@ -773,6 +776,7 @@ GemmParams<N> shortened(const GemmParams<kGatherMaxDims> &f)
     GemmParams<N> p{};
     p.a = f.a; p.b = f.b; p.c = f.c;
     p.m = f.m; p.n = f.n; p.k = f.k; p.k0 = f.k0;
+    p.a_line = f.a_line; p.b_line = f.b_line;
     p.alpha_re = f.alpha_re; p.alpha_im = f.alpha_im;
     p.beta_zero = f.beta_zero;
     p.conj_a = f.conj_a; p.conj_b = f.conj_b;

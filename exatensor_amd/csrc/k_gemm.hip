@@ -902,6 +902,26 @@ FullGroup line_group(int64_t stride)
   return d;
 }
 
+// Whether the offsets that a lane of the uniform modes holds (of its rows, from
+// the tile's first row where they are one dimension, and of its k-values inside
+// a k-tile) fit 32 bits.
+bool lane_offsets_fit(const FullGroup &row, const FullGroup &kg, int64_t rows, int es)
+{
+  int64_t o = 0;
+  if (row.nd <= 1) {
+    o = 127 * row.str[0];
+  } else {
+    int64_t n = 1;
+    for (int j = 0; j + 1 < row.nd; ++j) {
+      o += (int64_t)(row.div[j].d - 1) * row.str[j];
+      n *= row.div[j].d;
+    }
+    o += (rows / n - 1) * row.str[row.nd - 1];
+  }
+  const int64_t k0 = kg.str[0];
+  return o < (1ll << 32) && k0 < (1ll << 32) && (o + 31 * k0) * es + 16 < (1ll << 32);
+}
+
 // Launches product q of g's shape (g.m, g.n after any exchange of A and B) on
 // tile choice `tile`, cutting K as the workspace allows.
 int launch_product(Product &q, const GemmArgs &g, int tile, void *ws, size_t ws_bytes, hipStream_t s)
@@ -910,6 +930,8 @@ int launch_product(Product &q, const GemmArgs &g, int tile, void *ws, size_t ws_
   const int64_t tm = ((int64_t)g.m + ts.bm - 1) / ts.bm, tn = ((int64_t)g.n + ts.bn - 1) / ts.bn;
   if (tm >= (1ll << 31) || tn >= (1ll << 31) || tm * tn >= (1ll << 31) - 65536) return TALSH_LIMIT_EXCEEDED;
   auto &p = q.p;
+  p.a_line = p.a_row.nd <= 1 ? p.a_row.str[0] : 0;
+  p.b_line = p.b_row.nd <= 1 ? p.b_row.str[0] : 0;
   p.tiles_m = (int)tm;
   p.tiles_n = (int)tn;
   const SplitGeom G = split_geom(g, ts, current_cus(), ws ? ws_bytes : 0);
@@ -979,8 +1001,7 @@ int launch_matrix(GemmArgs g, int tile, void *ws, size_t ws_bytes, hipStream_t s
   p.c_row = line_group(1);
   p.c_col = line_group(p.m);
   const int es = kind_size(g.kind);
-  const int64_t lim = (1ll << 31) - 1, bytes = std::max(p.m, p.n) * p.k * es;
-  const bool off32 = p.m <= lim && p.n <= lim && p.k <= lim && bytes < (1ll << 32);
+  const bool off32 = lane_offsets_fit(p.a_row, p.a_k, p.m, es) && lane_offsets_fit(p.b_row, p.b_k, p.n, es);
   q.mode = !off32 ? kTab
            : gemm_vec_loads(es, g.a_kfast, g.m, g.k) && gemm_vec_loads(es, g.b_kfast, g.n, g.k) ? kVec : kUni;
   exchange(q, g);
@@ -1096,15 +1117,12 @@ int launch_gemm_gather(const GemmArgs &args, const GatherMaps &mp, void *ws, siz
   if (g.k == 0 && !g.beta_zero) return 0;  // empty contraction leaves C unchanged
   const GatherGroup *grp[6] = {&mp.a_row, &mp.a_k, &mp.b_row, &mp.b_k, &mp.c_row, &mp.c_col};
   const size_t want[6] = {g.m, g.k, g.n, g.k, g.m, g.n};
-  int64_t last[6];  // offset of a group's last index
   for (int t = 0; t < 6; ++t) {
     if (grp[t]->nd < 0 || grp[t]->nd > kGatherMaxDims) return TALSH_INVALID_ARGS;
     size_t count = 1;
-    last[t] = 0;
     for (int j = 0; j < grp[t]->nd; ++j) {
       if (grp[t]->ext[j] < 1 || grp[t]->str[j] < 0) return TALSH_INVALID_ARGS;
       count *= (size_t)grp[t]->ext[j];
-      last[t] += (int64_t)(grp[t]->ext[j] - 1) * grp[t]->str[j];
     }
     if (count != want[t]) return TALSH_INVALID_ARGS;
     if (count > INT32_MAX && grp[t]->nd > 1) return TALSH_LIMIT_EXCEEDED;  // digits are taken in 32 bits
@@ -1118,10 +1136,8 @@ int launch_gemm_gather(const GemmArgs &args, const GatherMaps &mp, void *ws, siz
   p.b_k = dev_group(mp.b_k);
   p.c_row = dev_group(mp.c_row);
   p.c_col = dev_group(mp.c_col);
-  const size_t lim = INT32_MAX;
-  const bool off32 = g.m <= lim && g.n <= lim && g.k <= lim && (last[0] + last[1] + 1) * es < (1ll << 32) &&
-                     (last[2] + last[3] + 1) * es < (1ll << 32);
-  if (off32 && gather_uniform_k(g.kind, mp))
+  if (lane_offsets_fit(p.a_row, p.a_k, p.m, es) && lane_offsets_fit(p.b_row, p.b_k, p.n, es) &&
+      gather_uniform_k(g.kind, mp))
     q.mode = gather_vec_loads(es, g.a_kfast, mp.a_row, mp.a_k, g.k) && gather_vec_loads(es, g.b_kfast, mp.b_row, mp.b_k, g.k)
                  ? kVec : kUni;
   const int tile = resolved_tile(g);

@@ -1,4 +1,4 @@
-"""Gathered products by offset tables in LDS: contracted groups of more than
+"""Gathered products by offset tables in LDS, and operands beyond 32-bit offsets: contracted groups of more than
 three dimensions or with runs that are no multiple of a k-tile, several chunks
 of 64 k-values per k-group, as many dimensions as a group can have, sums cut
 along K, and tensors of more than 4 GB read in place. Tolerances of the index
@@ -104,3 +104,30 @@ def test_tensor_beyond_4gb(order):
         L.talshAmdSetPlanVariant(-1, -1)
         for h in ts:
             L.talshTensorDestruct(C.byref(h))
+
+
+@pytest.mark.parametrize("ak", [1, 0])
+@pytest.mark.parametrize("m,n,k", [(70000, 40, 8192), (70001, 41, 8195), (130, 6, 4194320)])
+def test_matrix_beyond_4gb(m, n, k, ak):
+    """A matrix of more than 4 GB on either side of the product, in whole
+    vectors and not, and with k-values so far apart that a tile does not fit 32
+    bits either (130 rows of 34 MB): whole numbers that the sums keep exactly,
+    every tile."""
+    import torch
+    L = engine().lib
+    dev = "cuda"
+    rows = torch.arange(m, dtype=torch.float64, device=dev) % 97
+    ks = torch.arange(k, dtype=torch.float64, device=dev) % 11
+    a = rows[:, None] + 100 * ks[None, :] if ak else rows[None, :] + 100 * ks[:, None]
+    b = (torch.arange(n, dtype=torch.float64, device=dev)[:, None] + (ks[None, :] % 3)).contiguous()
+    bs, bk = b.sum(1), (b * ks[None, :]).sum(1)
+    want = rows[None, :] * bs[:, None] + 100 * bk[:, None]
+    c = torch.empty(m * n, dtype=torch.float64, device=dev)
+    for swap in (False, True):
+        for tile in (0, 1, 2):
+            c.fill_(float("nan"))
+            torch.cuda.synchronize()
+            x, y = ((m, a, ak), (n, b, 1)) if not swap else ((n, b, 1), (m, a, ak))
+            assert L.talshAmdGemm(T.R8, 0, x[0], y[0], k, x[1].data_ptr(), x[2], y[1].data_ptr(), y[2], c.data_ptr(), 1.0,
+                                  0.0, 1, tile, None, 0) == 0
+            assert torch.equal(c.view(n, m) if not swap else c.view(m, n).t(), want), (swap, tile)
