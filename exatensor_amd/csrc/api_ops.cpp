@@ -470,6 +470,18 @@ bool autotune_choose(const char *cptrn, talsh_tens_t *dtens, talsh_tens_t *ltens
   std::vector<PlanCandidate> cands;
   if (plan_candidates(dig, dr, lr, rr, dd, ld, rd, kind, d->r4mode, acc, d->num_cus, cands) || cands.empty())
     return false;
+  if (kind == R4 && d->r4mode == R4Mode::kBF16x3) {  // the three-way split in place, where its runs allow
+    std::vector<ContractPlan> fused;
+    if (plan_fused(dig, dr, lr, rr, dd, ld, rd, fused) == 0)
+      for (size_t i = 0; i < fused.size(); ++i) {
+        const ContractPlan &c = fused[i];
+        if (!split3_gather_ok(c.maps, c.swap ? c.n : c.m, c.swap ? c.m : c.n, c.k)) continue;
+        PlanCandidate pc;
+        pc.variant = kFusedVariantBase + (int)i;
+        pc.f[47] = pc.f[48] = 1.f;  // (its runs)
+        cands.push_back(pc);
+      }
+  }
   talsh_tens_t scratch;
   talshTensorClean(&scratch);
   if (talshTensorConstruct(&scratch, kind, dr, dd.data(), d->flat_id, nullptr, -1, nullptr, 0.0, 0.0)) return false;
@@ -1076,26 +1088,22 @@ static int contract_impl(const char *cptrn, talsh_tens_t *dtens, talsh_tens_t *l
   else if ((lr == 0) != (rr == 0)) P.kase = 1;
   else if (dr == 0) P.kase = 2;
   else {
-    // R4 under the three-way split: planes built straight from the tensors
-    // and the result written in place where their runs are long enough (the
-    // candidate that writes along D's contiguous index). No transposes: the
-    // operands are read once instead of three times, the product is not moved
-    // again (2574 x 2560 x 3072: 340 -> 272 us a call)
-    bool in_place = false;
-    if (plan_variant < 0 && kind == R4 && d->r4mode == R4Mode::kBF16x3 && plan_mode() != 0) {
-      std::vector<ContractPlan> fz;
-      if (plan_fused(dig, dr, lr, rr, dd, ld, rd, fz) == 0)
-        for (const ContractPlan &c : fz)
-          if (!in_place && split3_gather_ok(c.maps, c.swap ? c.n : c.m, c.swap ? c.m : c.n, c.k)) {
-            P = c;
-            in_place = true;
-          }
-    }
-    if (!in_place && plan_variant < 0) {
+    const bool split3 = (kind == R4 || kind == C4) && d->r4mode == R4Mode::kBF16x3;
+    bool planned = false;
+    if (plan_variant < 0) {
       const int mode = plan_mode();
       int v = -1, t = -1;
-      bool chosen = mode == 1 && selector_choose(dig, dr, lr, rr, dd, ld, rd, kind, d->r4mode, acc, d->num_cus, &v, &t);
-      if (!chosen && (mode == 2 || (mode == 1 && selector_installed()))) {
+      // R4 under the three-way split: in place where that is the faster form.
+      // No transposes: the operands are read once instead of three times, the
+      // product is not moved again (2574 x 2560 x 3072: 340 -> 272 us a call)
+      if (mode == 1 && split3 && kind == R4) {
+        std::vector<ContractPlan> fused;
+        const int i = plan_split3(dig, dr, lr, rr, dd, ld, rd, fused);
+        if ((planned = i >= 0)) P = fused[i];
+      }
+      bool chosen = !planned && mode == 1 &&
+                    selector_choose(dig, dr, lr, rr, dd, ld, rd, kind, d->r4mode, acc, d->num_cus, &v, &t);
+      if (!planned && !chosen && (mode == 2 || (mode == 1 && selector_installed()))) {
         const std::string key = plan_key(dig, lr, rr, dd, ld, rd, kind, d->r4mode, acc, d->num_cus);
         chosen = autotune_choose(cptrn, dtens, ltens, rtens, sr, si, d, acc, dig, dr, lr, rr, dd, ld, rd, kind, key,
                                  &v, &t);
@@ -1105,11 +1113,12 @@ static int contract_impl(const char *cptrn, talsh_tens_t *dtens, talsh_tens_t *l
         if (plan_tile < 0) plan_tile = t;
       }
     }
-    int e = in_place ? 0 : plan_contraction(dig, dr, lr, rr, dd, ld, rd, es, acc, plan_variant, P, nullptr);
-    // a forced fused gather is for native precision (the three-way split
-    // chooses its own above), and it takes its index digits in 32 bits
+    int e = planned ? 0 : plan_contraction(dig, dr, lr, rr, dd, ld, rd, es, acc, plan_variant, P, nullptr);
+    // a fused gather takes its index digits in 32 bits; the three-way split
+    // has one for R4 only, on runs that are long enough
     const bool wide = P.m > INT32_MAX || P.n > INT32_MAX || P.k > INT32_MAX;
-    if (!e && P.fused && !in_place && (wide || ((kind == R4 || kind == C4) && d->r4mode == R4Mode::kBF16x3)))
+    if (!e && P.fused && !planned &&
+        (wide || (split3 && (kind == C4 || !split3_gather_ok(P.maps, P.swap ? P.n : P.m, P.swap ? P.m : P.n, P.k)))))
       e = plan_contraction(dig, dr, lr, rr, dd, ld, rd, es, acc, -1, P, nullptr);
     if (e) return e;
   }

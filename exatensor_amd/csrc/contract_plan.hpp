@@ -40,6 +40,16 @@ constexpr int kFusedVariantBase = 1000;
 int plan_fused(const std::vector<int> &dig, int dr, int lr, int rr, const std::vector<int> &dd,
                const std::vector<int> &ld, const std::vector<int> &rd, std::vector<ContractPlan> &out);
 
+// R4 under the three-way split: the fused-gather candidate that runs with
+// operands and result in place (split planes straight from the tensors, the
+// result summed into D), -1 if there is none worth running: runs too short
+// (split3_gather_ok), or tensors that are matrices as they lie.
+int plan_split3(const std::vector<int> &dig, int dr, int lr, int rr, const std::vector<int> &dd,
+                const std::vector<int> &ld, const std::vector<int> &rd, std::vector<ContractPlan> &fused);
+// Whether a contraction's tensors are matrices whatever their extents: a
+// matricization without transposes exists.
+bool matrices_as_they_lie(const std::vector<int> &dig, int lr, int rr);
+
 std::vector<int> reorder(const std::vector<int> &from, const std::vector<int> &to);
 bool is_identity(const std::vector<int> &p);
 
@@ -63,7 +73,7 @@ struct PlanCandidate {
 
 // Every candidate of a GEMM-shaped contraction with its features.
 // The matricization candidates, then the fused-gather candidates (native
-// precision only: not for R4/C4 under the three-way split).
+// precision only: the model was not trained on the three-way split's).
 int plan_candidates(const std::vector<int> &dig, int dr, int lr, int rr, const std::vector<int> &dd,
                     const std::vector<int> &ld, const std::vector<int> &rd, int kind, R4Mode r4mode, bool acc,
                     int num_cus, std::vector<PlanCandidate> &out);

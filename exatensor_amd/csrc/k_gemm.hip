@@ -765,11 +765,11 @@ size_t realified_bytes(const GemmArgs &g)
 // Tile choice of the kernels: a caller's, or the default; complex kinds have
 // one choice, their two forms are told apart here: two k-groups per workgroup
 // when the tiles do not give every CU two workgroups and K is deep enough. Two
-// groups share at least 64 k-values (C8 64x64, two groups and one: k 8 12 and 9
-// us, 48 17 and 14, 64 17 and 17, 128 25 and 26, 512 76 and 81); where a CU
+// groups share more than 64 k-values (C8 64x64, two groups and one: k 8 13 and
+// 11 us, 48 18 and 15, 64 18 and 18, 128 26 and 27, 512 77 and 82); where a CU
 // would run its two workgroups one after the other they need K deep enough for
-// a cut of the last round besides (C8 1280x960: k 8 24 and 14 us, 160 60 and 52;
-// 512, in pieces, 109 and 141; C4 14 and 11, 33 and 32, 59 and 81).
+// a cut of the last round besides (C8 1280x960: k 8 25 and 16 us, 160 62 and 53;
+// 512, in pieces, 111 and 141; C4 16 and 12, 35 and 33, 60 and 81).
 int resolved_tile(const GemmArgs &g)
 {
   if (g.kind == C8 || g.kind == C4) {

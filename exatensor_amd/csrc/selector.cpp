@@ -383,6 +383,15 @@ int talshAmdSelectorChoice(const char *cptrn, int drank, const int *ddims, int l
   Engine &E = engine();
   const int cus = (E.on && !E.gpus.empty()) ? E.gpus[0]->num_cus : 256;
   const R4Mode mode = fast_math ? R4Mode::kBF16x3 : R4Mode::kNativeF32;
+  if (fast_math && data_kind == R4 && talshAmdGetPlanMode() == 1) {
+    std::vector<ContractPlan> fused;
+    const int v = plan_split3(dig, dr, lr, rr, dd, ld, rd, fused);
+    if (v >= 0) {
+      *variant = kFusedVariantBase + v;
+      *tile = 0;
+      return 0;
+    }
+  }
   if (!selector_choose(dig, dr, lr, rr, dd, ld, rd, data_kind, mode, accumulative != NOPE, cus, variant, tile)) {
     // the heuristic: fewest transpose bytes, default tile for the GEMM shape
     ContractPlan P;

@@ -29,10 +29,9 @@ int talshAmdProfileQuery(int kernel_class, double *total_ms, long long *launches
  * variant >= 0 selects the variant-th candidate matricization (ranked by the
  * built-in byte-count heuristic; 0 is the heuristic's choice), variant
  * TALSH_AMD_FUSED_VARIANT + i the i-th fused-gather candidate (no transposes:
- * the matrix product reads L and R and updates D by their index groups;
- * native precision, so R4/C4 under fast math take the heuristic's
- * matricization instead), -1 restores the engine's choice (which for R4 under
- * fast math reads the tensors in place where their runs are long enough);
+ * the matrix product reads L and R and updates D by their index groups; under
+ * fast math for R4 where L, R and D have runs of four elements and more, else
+ * the heuristic's matricization runs instead), -1 restores the engine's choice;
  * tile selects the GEMM tile shape (-1 default). */
 #define TALSH_AMD_FUSED_VARIANT 1000
 int talshAmdSetPlanVariant(int variant, int tile);
@@ -143,8 +142,10 @@ int talshAmdPlanFeatures(const char *cptrn, int drank, const int *ddims, int lra
  * libtalsh.so when present; TALSH_PLAN_MODEL set to an empty string disables
  * the selector. */
 int talshAmdSelectorInstall(void *mlp);
-/* The candidate talshTensorContract would run: the installed selector's
- * choice, or the heuristic's (variant 0 with its default GEMM tile). */
+/* The candidate talshTensorContract would run in plan mode 1 inside the
+ * model's domain: R4 under fast math the fused-gather candidate that it runs in
+ * place, where it does; else the installed selector's choice, or the
+ * heuristic's (variant 0 with its default GEMM tile). */
 int talshAmdSelectorChoice(const char *cptrn, int drank, const int *ddims, int lrank, const int *ldims, int rrank,
                            const int *rdims, int data_kind, int accumulative, int fast_math, int *variant, int *tile);
 
@@ -153,7 +154,8 @@ int talshAmdSelectorChoice(const char *cptrn, int drank, const int *ddims, int l
  *   0 heuristic: fewest transpose bytes, default tile;
  *   1 learned (default): the installed selector inside its training domain,
  *     the exhaustive autotuner outside it; with no model installed, the
- *     heuristic;
+ *     heuristic. R4 under fast math: in place, without transposes, where L, R
+ *     and D have runs of four elements and more and would be transposed;
  *   2 autotune: the exhaustive autotuner for every shape.
  * The autotuner runs every candidate on the caller's L and R (resident on the
  * executing GPU; otherwise the heuristic plans that call) into a scratch D,
