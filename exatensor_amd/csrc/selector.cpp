@@ -220,6 +220,7 @@ int talshAmdMlpTrain(void *mlp, const float *x, const float *y, long long n, int
   MlpModel *m = static_cast<MlpModel *>(mlp);
   GpuScope g;
   if (!g.ok) return TALSH_NOT_INITIALIZED;
+  m->format = kPlanModelFormat;  // whatever it was before: the caller has the present features
   const int nin = m->s.nin;
   // normalization from the training set
   for (int i = 0; i < nin; ++i) {
@@ -297,7 +298,7 @@ int talshAmdMlpSave(void *mlp, const char *path)
   const MlpModel *m = static_cast<MlpModel *>(mlp);
   FILE *f = std::fopen(path, "w");
   if (!f) return TALSH_FAILURE;
-  std::fprintf(f, "talsh_plan_mlp 1\n%d %d %d\n%.9g %.9g\n", m->s.nin, m->s.hidden, m->s.width, m->ymean, m->ystd);
+  std::fprintf(f, "talsh_plan_mlp %d\n%d %d %d\n%.9g %.9g\n", m->format, m->s.nin, m->s.hidden, m->s.width, m->ymean, m->ystd);
   for (float v : m->mean) std::fprintf(f, "%.9g ", v);
   std::fprintf(f, "\n");
   for (float v : m->stdv) std::fprintf(f, "%.9g ", v);
@@ -316,11 +317,12 @@ int talshAmdMlpLoad(const char *path, void **mlp)
   int ver = 0, nin = 0, hid = 0, wid = 0;
   float ym = 0, ys = 1;
   bool ok = std::fscanf(f, "%31s %d %d %d %d %f %f", tag, &ver, &nin, &hid, &wid, &ym, &ys) == 7 &&
-            std::strcmp(tag, "talsh_plan_mlp") == 0 && ver == 1;
+            std::strcmp(tag, "talsh_plan_mlp") == 0 && ver >= 1 && ver <= kPlanModelFormat;
   void *h = nullptr;
   if (ok) ok = talshAmdMlpCreate(nin, hid, wid, 0, &h) == 0;
   MlpModel *m = static_cast<MlpModel *>(h);
   if (ok) {
+    m->format = ver;
     m->ymean = ym;
     m->ystd = ys;
     for (int i = 0; ok && i < nin; ++i) ok = std::fscanf(f, "%f", &m->mean[i]) == 1;
@@ -368,6 +370,9 @@ int talshAmdSelectorInstall(void *mlp)
 {
   const MlpModel *m = static_cast<const MlpModel *>(mlp);
   if (m && m->s.nin != kPlanFeatures) return TALSH_INVALID_ARGS;
+  if (m && m->format < kPlanModelFormat)
+    log_error("the plan model (format %d) was trained on features of former kernels; its choices may be poor, train "
+              "it anew", m->format);
   selector_install(m);
   return 0;
 }

@@ -8,7 +8,13 @@
 
 namespace xt {
 
+// What the features of a plan model describe: 2, the present kernels; 1, the
+// ones before (tile choice 1, the vector loads and starts along k, the pieces
+// of K and the transposes' vectors were others).
+constexpr int kPlanModelFormat = 2;
+
 struct MlpModel {
+  int format = kPlanModelFormat;  // of the file it was loaded from
   MlpShape s;
   std::vector<float> params;      // layout of mlp_layer_offsets
   std::vector<float> mean, stdv;  // input normalization: (x - mean) / stdv

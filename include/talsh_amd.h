@@ -140,7 +140,9 @@ int talshAmdPlanFeatures(const char *cptrn, int drank, const int *ddims, int lra
  * autotuner, see talshAmdSetPlanMode). talshInit loads the model file named by the
  * environment variable TALSH_PLAN_MODEL, or else plan_model.txt next to
  * libtalsh.so when present; TALSH_PLAN_MODEL set to an empty string disables
- * the selector. */
+ * the selector. A model file names the format of its features; one of an
+ * earlier format is installed with a message on stderr, since it predicts from
+ * what its features meant for former kernels. */
 int talshAmdSelectorInstall(void *mlp);
 /* The candidate talshTensorContract would run in plan mode 1 inside the
  * model's domain: R4 under fast math the fused-gather candidate that it runs in
