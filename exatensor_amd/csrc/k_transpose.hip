@@ -1391,13 +1391,18 @@ int launch_permute_add(const void *in, void *out, int kind, int rank, const int 
   if (in == out || !permute_add_planned(kind, rank, dims_in, o2n)) return TALSH_INVALID_ARGS;
   const Planned pl = planned(kind_size(kind), rank, dims_in, o2n, in, out, true);
   const double f = real_factor(re, im);
+  hipEvent_t pr[2];
+  prof_begin(s, kKTranspose, pr);
+  int e = TALSH_INVALID_ARGS;
   switch (kind) {
-  case R4: return launch_runs<uint32_t, false, R4>(pl, in, out, f, 0.0, s);
-  case R8: return launch_runs<uint2, false, R8>(pl, in, out, f, 0.0, s);
-  case C4: return conj ? launch_runs<uint2, true, C4>(pl, in, out, re, im, s) : launch_runs<uint2, false, C4>(pl, in, out, re, im, s);
-  case C8: return conj ? launch_runs<uint4, true, C8>(pl, in, out, re, im, s) : launch_runs<uint4, false, C8>(pl, in, out, re, im, s);
-  default: return TALSH_INVALID_ARGS;
+  case R4: e = launch_runs<uint32_t, false, R4>(pl, in, out, f, 0.0, s); break;
+  case R8: e = launch_runs<uint2, false, R8>(pl, in, out, f, 0.0, s); break;
+  case C4: e = conj ? launch_runs<uint2, true, C4>(pl, in, out, re, im, s) : launch_runs<uint2, false, C4>(pl, in, out, re, im, s); break;
+  case C8: e = conj ? launch_runs<uint4, true, C8>(pl, in, out, re, im, s) : launch_runs<uint4, false, C8>(pl, in, out, re, im, s); break;
+  default: break;
   }
+  prof_end(s, kKTranspose, pr);
+  return e;
 }
 
 }  // namespace xt

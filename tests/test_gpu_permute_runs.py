@@ -116,3 +116,26 @@ def test_add_of_a_tensor_to_itself():
     assert np.array_equal(b.cpu().numpy().reshape(n, n, order="F"), m + m.T * 0.5)
     for t in (t1, t2):
         L.talshTensorDestruct(C.byref(t))
+
+
+def test_permuted_addition_is_profiled():
+    """An addition that permutes is a launch of the transpose class, in one pass
+    or (over overlapping bodies) with a permuted copy."""
+    import torch
+    L, gpu = engine().lib, engine().gpu(0)
+    n = 33
+    b = torch.zeros(3 * n * n, dtype=torch.float64, device="cuda")
+    torch.cuda.synchronize()
+    ms, count = C.c_double(), C.c_longlong()
+    L.talshAmdProfile(1)
+    try:
+        for at in (0, n, 2 * n * n):  # the same body, overlapping, apart
+            t1, t2 = _wrap(L, b.data_ptr(), T.R8, (n, n)), _wrap(L, b.data_ptr() + 8 * at, T.R8, (n, n))
+            L.talshAmdProfileQuery(T.KERNEL_TRANSPOSE, C.byref(ms), C.byref(count))
+            assert L.talshTensorAdd(b"D(b,a)+=L(a,b)", C.byref(t1), C.byref(t2), 0.5, 0.0, gpu, T.DEV_NULL, T.COPY_MT, None) == 0
+            L.talshAmdProfileQuery(T.KERNEL_TRANSPOSE, C.byref(ms), C.byref(count))
+            assert count.value == 1 and ms.value > 0, at
+            for t in (t1, t2):
+                L.talshTensorDestruct(C.byref(t))
+    finally:
+        L.talshAmdProfile(0)
