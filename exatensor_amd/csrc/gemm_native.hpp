@@ -1,6 +1,6 @@
 // Native-precision matrix products (FP64 / FP32 16x16x4 MFMAs, real and
-// complex): kernels, and the launchers that the per-kind translation units
-// instantiate (k_gemm_r8.hip, k_gemm_r4.hip, k_gemm_cx.hip).
+// complex): kernels, and the launchers that the translation units of each kind
+// and tile choice instantiate (k_gemm_native.hip).
 //
 // Every operand is addressed by two index groups (rows and k, GatherMaps): a
 // matricized operand has one dimension per group, a tensor read in place up
@@ -114,9 +114,20 @@ struct Product {
   GemmMode mode = kTab;
 };
 
-int launch_native_r8(const Product &q, int tile, hipStream_t s);
-int launch_native_r4(const Product &q, int tile, hipStream_t s);
-int launch_native_cx(const Product &q, int kind, int tile, hipStream_t s);
+// Output tiles of the native-precision kernels: rows x columns, the k-depth of
+// one LDS stage (128 bytes of a row; complex kinds hold two planes) and the
+// k-groups of a workgroup.
+struct TileShape { int bm, bn, bk, groups; };
+constexpr TileShape tile_shape(int kind, int tile)
+{
+  const int bk = kind == R4 ? 32 : 16;
+  if (kind == C8 || kind == C4) return {64, 64, bk, tile == 1 ? 2 : 1};
+  return tile == 2 ? TileShape{64, 64, bk, 1} : tile == 1 ? TileShape{64, 64, bk, 4} : TileShape{128, 128, bk, 1};
+}
+
+// One translation unit (k_gemm_native.hip) for each kind and tile choice.
+template <int KIND, int TILE>
+int launch_native(const Product &q, hipStream_t s);
 
 // The output-tile order: first gather the workgroups that the dispatcher
 // places on one XCD (round-robin over 8) into a contiguous range, then walk

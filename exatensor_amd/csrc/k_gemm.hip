@@ -655,16 +655,6 @@ int current_cus()
   return cus;
 }
 
-// Output tiles of the native-precision kernels: rows x columns and the k-depth
-// of one LDS stage (128 bytes of a row; complex kinds hold two planes).
-struct TileShape { int bm, bn, bk, groups; };
-TileShape tile_shape(int kind, int tile)
-{
-  const int bk = kind == R4 ? 32 : 16;
-  if (kind == C8 || kind == C4) return {64, 64, bk, tile == 1 ? 2 : 1};
-  return tile == 2 ? TileShape{64, 64, bk, 1} : tile == 1 ? TileShape{64, 64, bk, 4} : TileShape{128, 128, bk, 1};
-}
-
 bool native_real(const GemmArgs &g) { return g.kind == R8 || (g.kind == R4 && g.r4mode == R4Mode::kNativeF32); }
 
 constexpr int64_t kSplitMinK = 256;  // shortest K that is cut
@@ -948,10 +938,14 @@ int launch_product(Product &q, const GemmArgs &g, int tile, void *ws, size_t ws_
     if (k0 > 0) p.beta_zero = 0;
     int e;
     switch (g.kind) {
-    case R8: e = launch_native_r8(q, tile, s); break;
-    case R4: e = launch_native_r4(q, tile, s); break;
-    case C8:
-    case C4: e = launch_native_cx(q, g.kind, tile, s); break;
+    case R8:
+      e = tile == 2 ? launch_native<R8, 2>(q, s) : tile == 1 ? launch_native<R8, 1>(q, s) : launch_native<R8, 0>(q, s);
+      break;
+    case R4:
+      e = tile == 2 ? launch_native<R4, 2>(q, s) : tile == 1 ? launch_native<R4, 1>(q, s) : launch_native<R4, 0>(q, s);
+      break;
+    case C8: e = tile == 1 ? launch_native<C8, 1>(q, s) : launch_native<C8, 0>(q, s); break;
+    case C4: e = tile == 1 ? launch_native<C4, 1>(q, s) : launch_native<C4, 0>(q, s); break;
     default: return TALSH_INVALID_ARGS;
     }
     if (e) return e;
