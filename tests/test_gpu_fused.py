@@ -1,8 +1,8 @@
-"""Fused index gather on the GPU: contractions whose matrix product reads L
-and R and updates D through index offset tables, with no transposes. Every
-fused candidate and GEMM tile of each case is checked against long-double
-direct evaluation (relative Frobenius 1e-12 for R8/C8, 1e-5 for R4/C4), and
-the kernel profile shows that no transpose ran."""
+"""Fused index gather on the GPU: contractions whose matrix product reads L and
+R and updates D by their index groups, with no transposes. Every fused
+candidate and GEMM tile of each case is checked against long-double direct
+evaluation (relative Frobenius 1e-12 for R8/C8, 1e-5 for R4/C4), and the kernel
+profile shows that no transpose ran."""
 import ctypes as C
 
 import numpy as np

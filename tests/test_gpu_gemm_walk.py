@@ -1,8 +1,9 @@
 """Index walks of the native-precision matrix kernels: contracted groups of one
-to five dimensions with odd extents (carries, the fresh decomposition beyond
-three dimensions, the long argument form beyond four), k-tails on both sides of
-a k-tile and of a workgroup's share of them, row and column edges, and operands
-of more than 4 GB (64-bit offsets), against float64 / complex128 products."""
+to five dimensions with odd extents (carries, the offset tables beyond three
+dimensions and for runs that are no multiple of a k-tile, the long argument
+form), k-tails on both sides of a k-tile and of a workgroup's share of them,
+row and column edges, and operands of more than 4 GB, against float64 /
+complex128 products."""
 import ctypes as C
 
 import numpy as np
@@ -71,8 +72,8 @@ def test_contracted_groups(kind, ks, lk, rk, lf, rf):
 @pytest.mark.parametrize("k", [1, 2, 8, 15, 16, 17, 24, 31, 33, 63, 64, 65, 72, 127, 130, 264])
 def test_k_tails(kind, k):
     """Products of 66 x 62 (edges of 64-wide tiles, even: pair loads where k
-    allows) and 65 x 129, every orientation and tile choice, without and with
-    room for pieces of K."""
+    allows) and 65 x 129, every orientation and tile choice, K uncut (pieces of
+    K: test_gpu_k_pieces.py)."""
     import torch
     L = engine().lib
     cx = kind == T.C8
@@ -81,7 +82,6 @@ def test_k_tails(kind, k):
         gen = torch.Generator(device="cuda").manual_seed(k * 1000 + m)
         a, b = (torch.rand(x * k * (2 if cx else 1), dtype=torch.float64, device="cuda", generator=gen) - 0.5 for x in (m, n))
         a, b = ((torch.view_as_complex(x.view(-1, 2)) if cx else x).to(dt) for x in (a, b))
-        ws = torch.empty(1 << 20, dtype=torch.uint8, device="cuda")
         for ak in (0, 1):
             for bk in (0, 1):
                 A = a.view(m, k) if ak else a.view(k, m).t()
@@ -89,13 +89,12 @@ def test_k_tails(kind, k):
                 wide = torch.complex128 if cx else torch.float64
                 want = (A.to(wide).cpu() @ B.to(wide).cpu().t()).t().contiguous().view(-1).numpy()
                 for tile in ((0,) if cx else (0, 1, 2)):
-                    for wsb in (0, 1 << 20):
-                        c = torch.full((m * n,), 7.0, dtype=dt, device="cuda")
-                        torch.cuda.synchronize()
-                        e = L.talshAmdGemm(kind, 0, m, n, k, a.data_ptr(), ak, b.data_ptr(), bk, c.data_ptr(), 1.0, 0.0,
-                                           1, tile, ws.data_ptr(), wsb)
-                        assert e == 0
-                        assert rel_err(c.cpu().numpy(), want) <= TOL[kind], (m, n, ak, bk, tile, wsb)
+                    c = torch.full((m * n,), 7.0, dtype=dt, device="cuda")
+                    torch.cuda.synchronize()
+                    e = L.talshAmdGemm(kind, 0, m, n, k, a.data_ptr(), ak, b.data_ptr(), bk, c.data_ptr(), 1.0, 0.0, 1,
+                                       tile, None, 0)
+                    assert e == 0
+                    assert rel_err(c.cpu().numpy(), want) <= TOL[kind], (m, n, ak, bk, tile)
 
 
 @pytest.mark.parametrize("ak", [1, 0])
