@@ -42,7 +42,9 @@
 // R8 ranks 10, extents 4 (groups of five dimensions) 116 against 72, extents 3
 // 106 against 22; ranks 8, extents 4 53 against 21; R4 the same three 107, 98
 // and 62 against 52, 20 and 16; R4 24^4 29.6 against 24.2; R8 1537 x 1581 x
-// 2491 with its transposes 301 against 291.
+// 2491 (a call) 300 against 290; C4 with runs of a few elements and a deep K 55
+// against 60. (32-bit offsets in the tables, and reading them ahead of the
+// stores to LDS, changed nothing beyond 1%.)
 //
 // Operand tiles sit in LDS with k fastest ([row][k], padded rows). Inside a
 // 16-deep k slice, lane group g = lane/16 feeds k = 4g+s at MFMA step s, so a
