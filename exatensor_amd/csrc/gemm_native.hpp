@@ -36,13 +36,14 @@
 // steps by carries, the lanes' offsets are loop invariant, and one compare per
 // k-tile decides what the last tile needs. 128x128 tiles reach 64 (FP64) and
 // 127 (FP32) TFLOP/s, 82% of the matrix peak, and C8 64x64 tiles 64. Everywhere
-// else (mode kTab) one lane per k-value works out its offsets for 64 k-values
-// ahead into LDS, and the loads add what they read there to their row's offset.
+// else (modes kTab, kTabLong) one lane per k-value works out its offsets for 64
+// k-values ahead into LDS, and the loads add what they read there to their
+// row's offset.
 // With a digit walk per lane and k-value instead, kernel times were, in us:
 // R8 ranks 10, extents 4 (groups of five dimensions) 116 against 72, extents 3
 // 106 against 22; ranks 8, extents 4 53 against 21; R4 the same three 107, 98
-// and 62 against 52, 20 and 16; R4 24^4 29.6 against 24.2; R8 1537 x 1581 x
-// 2491 (a call) 300 against 290; C4 with runs of a few elements and a deep K 55
+// and 62 against 52, 20 and 16; R4 24^4 29.6 against 23; R8 1537 x 1581 x
+// 2491 (a call) 300 against 286; C4 with runs of a few elements and a deep K 55
 // against 60. (32-bit offsets in the tables, and reading them ahead of the
 // stores to LDS, changed nothing beyond 1%.)
 //
@@ -74,7 +75,9 @@ struct DevGroup {
 };
 
 // Kernel arguments. Groups of up to kSmallDims dimensions go in the short form
-// (0.6 KB in all): with 2 KB of arguments every launch took about 1 us longer.
+// (0.6 KB in all): with 2 KB of arguments every launch took about 1 us longer
+// (calls by offset tables: R8 8^4 40.4 against 38.3 us, R8 1537 x 1581 x 2491
+// 291 against 286).
 constexpr int kSmallDims = 4;
 template <int N>
 struct GemmParams {
@@ -104,10 +107,11 @@ enum GemmMode {
   kVec,   // a k-tile starts at one offset for all lanes; k-fast operands load 16-byte vectors, row-fast ones
           // row pairs (whole vectors everywhere: even rows and k-values in eights there)
   kUni,   // the same, element loads
-  kTab    // offsets from tables in LDS: runs along k of any length, groups of up to kGatherMaxDims dimensions,
-          // 64-bit offsets
+  kTab,   // offsets from tables in LDS: runs along k of any length, 64-bit offsets
+  kTabLong  // the same with arguments in the long form, for groups of up to kGatherMaxDims dimensions
 };
-constexpr int group_dims(GemmMode mode) { return mode == kTab ? kGatherMaxDims : kSmallDims; }
+constexpr int group_dims(GemmMode mode) { return mode == kTabLong ? kGatherMaxDims : kSmallDims; }
+constexpr bool tabled(GemmMode mode) { return mode == kTab || mode == kTabLong; }
 
 // A product ready to launch.
 struct Product {
@@ -263,7 +267,7 @@ __device__ __forceinline__ float flip_sign(float x, uint32_t m) { return __uint_
 // group, one k-tile in KG.
 template <typename T, bool CPLX, bool KF, int BX, int BK, int KG, GemmMode MODE>
 struct Staging {
-  static constexpr bool TAB = MODE == kTab;
+  static constexpr bool TAB = tabled(MODE);
   typedef typename std::conditional<TAB, uint64_t, uint32_t>::type OffT;
   static constexpr int N = group_dims(MODE);
   static constexpr bool VEC = MODE == kVec && !CPLX;
@@ -514,7 +518,7 @@ __global__ __launch_bounds__(256 * KG, OCC) void k_gemm_mfma(const GemmParams<gr
   __shared__ __align__(16) T Bs[KG][2][NP * BN][KP];
   // TAB: offsets in bytes of the tile's rows of A and B and of two chunks of
   // 64 k-values per k-group, in elements of its rows and columns of C.
-  constexpr bool TAB = MODE == kTab;
+  constexpr bool TAB = tabled(MODE);
   constexpr int TN = TAB ? 64 : 1, TPC = 64 / BK;  // k-tiles per chunk
   __shared__ uint64_t t_ab[TAB ? BM + BN : 1], t_k[TAB ? KG : 1][2][2][TN];
   __shared__ int64_t t_c[TAB ? BM + BN : 1];
@@ -840,6 +844,7 @@ int launch_modes(const Product &q, hipStream_t s)
     if (q.mode == kVec) return launch_orient<T, CPLX, BM, BN, BK, KG, OCC, kVec>(q, s);
   }
   if (q.mode == kTab) return launch_orient<T, CPLX, BM, BN, BK, KG, OCC, kTab>(q, s);
+  if (q.mode == kTabLong) return launch_orient<T, CPLX, BM, BN, BK, KG, OCC, kTabLong>(q, s);
   return launch_orient<T, CPLX, BM, BN, BK, KG, OCC, kUni>(q, s);
 }
 

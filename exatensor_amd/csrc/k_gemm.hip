@@ -1130,6 +1130,8 @@ int launch_gemm_gather(const GemmArgs &args, const GatherMaps &mp, void *ws, siz
   p.b_k = dev_group(mp.b_k);
   p.c_row = dev_group(mp.c_row);
   p.c_col = dev_group(mp.c_col);
+  for (const GatherGroup *x : grp)
+    if (x->nd > kSmallDims) q.mode = kTabLong;
   if (lane_offsets_fit(p.a_row, p.a_k, p.m, es) && lane_offsets_fit(p.b_row, p.b_k, p.n, es) &&
       gather_uniform_k(g.kind, mp))
     q.mode = gather_vec_loads(es, g.a_kfast, mp.a_row, mp.a_k, g.k) && gather_vec_loads(es, g.b_kfast, mp.b_row, mp.b_k, g.k)

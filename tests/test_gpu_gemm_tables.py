@@ -22,6 +22,10 @@ GROUPS = [
     ((3, 5, 4, 3), False, False, (3, 3, 3, 3, 3), (2, 5, 2, 3)),
     ((16, 3, 3, 5), True, True, (130,), (5, 7)),
     ((2,) * 16, True, True, (33,), (17,)),
+    # four dimensions in every group, the short form of the arguments at its limit; five in one group
+    ((3, 5, 4, 3), True, False, (3, 2, 5, 4), (2, 5, 2, 3)),
+    ((5, 9), False, True, (3, 3, 3, 2, 2), (6,)),
+    ((5, 9), True, True, (7,), (2, 3, 2, 2, 5)),
 ]
 
 
